@@ -323,7 +323,8 @@ __attribute__((amdgpu_waves_per_eu(CztRowsShape<Q, ZL>::WAVES))) void czt_rows_k
 #pragma unroll
     for (int q = 0; q < HO::R; ++q) u.v[b][q] = cmul(u.v[b][q], a.ax.gf[HO::index(t, b, q)]);
   float2* dst = a.t + (int64_t)f * a.t_cs;
-  auto store = [&](int k, float2 v) {
+  auto store = [&](int k0, float2 v) {
+    const int k = t + k0;
     if (k < lout) dst[czt_tidx(a.rin4, row, k)] = cmul(v, a.ax.post[k]);
   };
   fft_inverse_from_regs<Q, TPF, DST_FN, ZL>(s, t, u, store);
@@ -396,7 +397,8 @@ __attribute__((amdgpu_waves_per_eu(CztColsShape<Q>::WAVES))) void czt_cols_kerne
     __syncthreads();
     fft_forward_to_regs<Q, TPF, SRC_LDS, ZL>(s, t, none, u);
   } else {
-    auto load = [&](int r) -> float2 {
+    auto load = [&](int k0) -> float2 {
+      const int r = t + k0;
       return (colok && r < lin) ? cmul(src[czt_tidx(a.rin4, r, kx)], a.ay.pre[r]) : make_float2(0.f, 0.f);
     };
     // (twiddle bases loaded at each pass: prefetched, they cost the 3 * 2^k
@@ -435,7 +437,8 @@ __attribute__((amdgpu_waves_per_eu(CztColsShape<Q>::WAVES))) void czt_cols_kerne
       }
     }
   } else {
-    auto store = [&](int ky, float2 v) {
+    auto store = [&](int k0, float2 v) {
+      const int ky = t + k0;
       if (colok && ky < lout) {
         v = cmul(v, a.ay.post[ky]);
         if (a.f0tab) v = c_mul(v, a.f0tab[(int64_t)ky * lout_x + kx]);

@@ -264,11 +264,12 @@ __device__ __forceinline__ void fft_lds(float2* s, int t) {
 
 // Block-index remap so that consecutive logical blocks (which share 128-byte
 // lines of the tiled intermediates) land on the same XCD: hardware dispatches
-// block b to XCD b % 8.
+// block b to XCD b % 8, whose blocks take one contiguous logical range (the
+// first nblocks % 8 ranges are one block longer).
 __device__ __forceinline__ int xcd_remap(int b, int nblocks) {
   constexpr int NX = 8;
-  if (nblocks % NX) return b;
-  return (b % NX) * (nblocks / NX) + b / NX;
+  const int x = b % NX, rem = nblocks % NX;
+  return x * (nblocks / NX) + (x < rem ? x : rem) + b / NX;
 }
 
 // --- float64 phase helpers ---------------------------------------------------

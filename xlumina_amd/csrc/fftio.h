@@ -10,10 +10,11 @@
 // chirp spectrum) is applied in registers between the two chains, with no
 // LDS round trip.
 //
-// Functor interfaces:
-//   load(int idx) -> float2        input sample idx in [0, L) (0 where padded)
-//   store(int idx, float2 v)       output sample idx (the functor skips unneeded ones)
-//   mul(int idx, int slot, float2 v) -> float2   frequency-domain product
+// Functor interfaces (thread t of the transform handles the samples t + k, k a
+// multiple of TPF that is a constant after unrolling: a functor adds k to a
+// block-uniform base and keeps one per-thread offset for all its accesses):
+//   load(int k) -> float2          input sample t + k (0 where padded)
+//   store(int k, float2 v)         output sample t + k (the functor skips unneeded ones)
 #pragma once
 #include "fft.h"
 
@@ -40,6 +41,7 @@ __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& sto
   constexpr int BPT = (NB + TPF - 1) / TPF;
   static_assert(!(ZHI && LOW), "a pass is either the first or the last of a chain here");
   static_assert(!ZHI || NS == 1, "zero upper inputs only on the first pass");
+  static_assert(DST != DST_FN || NS == NB, "a functor takes the outputs of the last pass");
   float2 v[BPT][R];
 #pragma unroll
   for (int b = 0; b < BPT; ++b) {
@@ -49,7 +51,7 @@ __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& sto
       for (int r = 0; r < R; ++r) {
         if (ZHI && r >= R / 2) v[b][r] = make_float2(0.f, 0.f);
         else if constexpr (SRC == SRC_LDS) v[b][r] = s[lpad(j + r * NB)];
-        else if constexpr (SRC == SRC_FN) v[b][r] = load(j + r * NB);
+        else if constexpr (SRC == SRC_FN) v[b][r] = load(b * TPF + r * NB);
         else v[b][r] = reg.v[b][r];
       }
       if constexpr (NS > 1) {
@@ -71,7 +73,7 @@ __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& sto
 #pragma unroll
       for (int r = 0; r < (LOW ? R / 2 : R); ++r) {
         if constexpr (DST == DST_LDS) s[lpad(idxD + r * NS)] = v[b][r];
-        else if constexpr (DST == DST_FN) store(idxD + r * NS, v[b][r]);
+        else if constexpr (DST == DST_FN) store(b * TPF + r * NS, v[b][r]);
         else reg.v[b][r] = v[b][r];
       }
     }
@@ -119,9 +121,9 @@ template <int L, int TPF, bool FWD> struct TwSet {
 // need a plan that starts (ZHI) or ends (LOW) with an unstrided radix-16 pass
 // over the L/2 split, i.e. a power-of-two L.
 template <int L, int TPF, bool INV, bool FWD, int I, int SRC, int DST, bool ZHI, bool LOW, bool TWPRE, class Load,
-          class Store, class RegIn, class RegOut>
+          class Store, class RegIn, class RegOut, class Hook>
 __device__ __forceinline__ void chain_pass(float2* s, int t, Load& load, Store& store, RegIn& rin, RegOut& rout,
-                                           TwSet<L, TPF, FWD>& tw) {
+                                           TwSet<L, TPF, FWD>& tw, Hook& hook) {
   using P = FftPlan<L>;
   constexpr int R = P::radix(FWD, I), NS = P::ns(FWD, I);
   constexpr bool first = I == 0, last = I == P::NP - 1;
@@ -136,24 +138,37 @@ __device__ __forceinline__ void chain_pass(float2* s, int t, Load& load, Store& 
   if constexpr (first) {
     pass_io<L, R, NS, TPF, INV, S, D, ZHI, false, TWPRE>(s, t, load, store, rin, wb);
   } else if constexpr (last) {
+    hook();
     pass_io<L, R, NS, TPF, INV, S, D, false, LOW, TWPRE>(s, t, load, store, rout, wb);
   } else {
     pass_io<L, R, NS, TPF, INV, S, D, false, false, TWPRE>(s, t, load, store, rout, wb);
   }
   if constexpr (!last)
-    chain_pass<L, TPF, INV, FWD, I + 1, SRC, DST, ZHI, LOW, TWPRE>(s, t, load, store, rin, rout, tw);
+    chain_pass<L, TPF, INV, FWD, I + 1, SRC, DST, ZHI, LOW, TWPRE>(s, t, load, store, rin, rout, tw, hook);
 }
 
-// The whole chain (I = 0).  TWPRE: the twiddle bases of all passes are loaded
+struct NoHook {
+  __device__ void operator()() const {}
+};
+
+// The whole chain (I = 0).  hook() runs right before the last pass, behind its
+// barrier (loads issued there are in flight during the pass).  TWPRE: the twiddle bases of all passes are loaded
 // first (a few registers per pass: the kernels that cannot spare them keep
 // loading each pass's bases at the pass).
 template <int L, int TPF, bool INV, bool FWD, int I, int SRC, int DST, bool ZHI = false, bool LOW = false,
-          bool TWPRE = true, class Load, class Store, class RegIn, class RegOut>
-__device__ __forceinline__ void chain_io(float2* s, int t, Load& load, Store& store, RegIn& rin, RegOut& rout) {
+          bool TWPRE = true, class Load, class Store, class RegIn, class RegOut, class Hook>
+__device__ __forceinline__ void chain_io(float2* s, int t, Load& load, Store& store, RegIn& rin, RegOut& rout,
+                                         Hook& hook) {
   static_assert(I == 0, "a chain starts at its first pass");
   TwSet<L, TPF, FWD> tw;
   if constexpr (TWPRE) tw.load(t);
-  chain_pass<L, TPF, INV, FWD, 0, SRC, DST, ZHI, LOW, TWPRE>(s, t, load, store, rin, rout, tw);
+  chain_pass<L, TPF, INV, FWD, 0, SRC, DST, ZHI, LOW, TWPRE>(s, t, load, store, rin, rout, tw, hook);
+}
+template <int L, int TPF, bool INV, bool FWD, int I, int SRC, int DST, bool ZHI = false, bool LOW = false,
+          bool TWPRE = true, class Load, class Store, class RegIn, class RegOut>
+__device__ __forceinline__ void chain_io(float2* s, int t, Load& load, Store& store, RegIn& rin, RegOut& rout) {
+  NoHook none;
+  chain_io<L, TPF, INV, FWD, I, SRC, DST, ZHI, LOW, TWPRE>(s, t, load, store, rin, rout, none);
 }
 
 template <int L, int TPF> struct HandOff {
@@ -162,18 +177,25 @@ template <int L, int TPF> struct HandOff {
   static constexpr int NB = P::NBH;
   static constexpr int BPT = (NB + TPF - 1) / TPF;
   using Type = Regs<BPT, R>;
-  // element index held in slot (b, q)
-  __device__ static int index(int t, int b, int q) { return t + b * TPF + q * NB; }
+  // element index held in slot (b, q): t + koff(b, q)
+  __device__ static constexpr int koff(int b, int q) { return b * TPF + q * NB; }
+  __device__ static int index(int t, int b, int q) { return t + koff(b, q); }
   __device__ static bool valid(int t, int b) { return NB % TPF == 0 || t + b * TPF < NB; }
 };
 
 // forward FFT: SRC -> registers (hand-off layout)
+template <int L, int TPF, int SRC, bool ZHI = false, bool TWPRE = true, class Load, class Hook>
+__device__ __forceinline__ void fft_forward_to_regs(float2* s, int t, Load& load,
+                                                    typename HandOff<L, TPF>::Type& out, Hook& hook) {
+  NoIO none;
+  typename HandOff<L, TPF>::Type dummy;
+  chain_io<L, TPF, false, true, 0, SRC, DST_REG, ZHI, false, TWPRE>(s, t, load, none, dummy, out, hook);
+}
 template <int L, int TPF, int SRC, bool ZHI = false, bool TWPRE = true, class Load>
 __device__ __forceinline__ void fft_forward_to_regs(float2* s, int t, Load& load,
                                                     typename HandOff<L, TPF>::Type& out) {
-  NoIO none;
-  typename HandOff<L, TPF>::Type dummy;
-  chain_io<L, TPF, false, true, 0, SRC, DST_REG, ZHI, false, TWPRE>(s, t, load, none, dummy, out);
+  NoHook none;
+  fft_forward_to_regs<L, TPF, SRC, ZHI, TWPRE>(s, t, load, out, none);
 }
 
 // inverse FFT: registers (hand-off layout) -> DST

@@ -161,23 +161,34 @@ struct PixRaw {
   float v[2][2];   // [stage][m0, m1]
 };
 
-template <int U>
+// Element `i` of an array with a block-uniform base: the 32-bit byte offset is
+// one register for every array of that element size (arrays up to 4 GiB).
+template <class T> __device__ __forceinline__ T at32(const T* base, uint32_t i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + i * (uint32_t)sizeof(T));
+}
+
+// pix: pixel indices, 64-bit or (planes of up to 2^29 pixels) 32-bit.
+template <int U, class I>
 __device__ __forceinline__ void pix_load_n(const float2* in, int64_t cs, int nin, const MaskArgs& m,
-                                           const int64_t (&pix)[U], PixRaw (&r)[U]) {
+                                           const I (&pix)[U], PixRaw (&r)[U]) {
+  auto at = [](const auto* base, I i) {
+    if constexpr (sizeof(I) == 4) return at32(base, i);
+    else return base[i];
+  };
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     r[u].e[1] = r[u].e[2] = make_float2(0.f, 0.f);
     r[u].v[0][0] = r[u].v[0][1] = r[u].v[1][0] = r[u].v[1][1] = 0.f;
   }
 #pragma unroll
-  for (int u = 0; u < U; ++u) r[u].e[0] = in[pix[u]];
+  for (int u = 0; u < U; ++u) r[u].e[0] = at(in, pix[u]);
   if (nin > 1) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u].e[1] = in[cs + pix[u]];
+    for (int u = 0; u < U; ++u) r[u].e[1] = at(in + cs, pix[u]);
   }
   if (nin > 2) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u].e[2] = in[2 * cs + pix[u]];
+    for (int u = 0; u < U; ++u) r[u].e[2] = at(in + 2 * cs, pix[u]);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -188,7 +199,7 @@ __device__ __forceinline__ void pix_load_n(const float2* in, int64_t cs, int nin
       const int f = param_form(m.st[i], j);
       if (!(f & PF_F64)) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) r[u].v[i][j] = p[pix[u]];
+        for (int u = 0; u < U; ++u) r[u].v[i][j] = at(p, pix[u]);
       } else if (f & PF_SCALAR) {
         const float v = param_value(reinterpret_cast<const double*>(p)[0], f);
 #pragma unroll
@@ -196,7 +207,7 @@ __device__ __forceinline__ void pix_load_n(const float2* in, int64_t cs, int nin
       } else {
         double d[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) d[u] = reinterpret_cast<const double*>(p)[pix[u]];
+        for (int u = 0; u < U; ++u) d[u] = at(reinterpret_cast<const double*>(p), pix[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u) r[u].v[i][j] = param_value(d[u], f);
       }

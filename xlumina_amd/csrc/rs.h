@@ -12,15 +12,17 @@
 // is even in both axes, so only rows 0..P/2-1 of its row transform are built
 // and the column pass mirrors them.
 //
-// Passes (all intermediates in 4x4-tile layout, 128 B per tile, ordered
-// [column group][row group], so row passes write and column passes read whole
-// 128 B lines):
-//   rs_hrow   : H rows 0..P/2-1 generated in float64 phase -> row FFT -> Hr
-//   rs_urow   : masks + Ez on the input rows -> zero-padded row FFT -> T
-//   rs_hcol   : per column: FFT(Hr col, mirrored) -> Hhat, in place (half spectrum)
+// Passes (intermediates of N x P samples in 4x4 tiles of 128 B, ordered [column
+// group][row group]: a row pass touches 32 B of each line per row, a column
+// pass every line of its columns):
+//   rs_hrow   : H rows 0..N-1 generated in float64 phase -> row FFT -> Hr (tiles)
+//   rs_hcol   : per column kx <= P/2: FFT(Hr col, mirrored) -> Hhat, one contiguous
+//               column of ky <= P/2 (quarter spectrum: the kernel array is even)
+//   rs_urow   : masks + Ez on the input rows -> zero-padded row FFT -> T (tiles)
 //   rs_col    : per (column, component): FFT(T col) * Hhat -> IFFT, keep rows
 //               0..N-1 -> T
 //   rs_final  : row IFFT of T, keep columns 0..N-1 -> output (+ |E|^2)
+// Hr lives where rs_urow puts T afterwards.
 #pragma once
 #include "fft.h"
 #include "fftio.h"
@@ -36,9 +38,8 @@ struct RsArgs {
   int64_t out_cs;
   float* intensity;       // optional N x N, sum_c |out_c|^2
   float2* t;              // tiles, ncomp x NR4*4 x P
-  float2* hr;             // tiles, (P/2) x (P/2 + 1) of a (P/2) x P array: Hr after the row pass,
-                          // Hhat (ky < P/2) after rs_hcol; columns kx > P/2 mirror (Hhat is even in kx)
-  float2* hmid;           // P/2 + 1: Hhat at ky = P/2
+  float2* hr;             // Hr: N rows x (P/2 + 1) columns in tiles (rs_hr_elems)
+  float2* hh;             // Hhat: columns kx <= P/2 of stride rs_hh_stride, ky <= P/2 (even in kx and ky)
   const double* x;
   const double* y;
   double z, k;
@@ -53,17 +54,18 @@ struct RsArgs {
   // between the members' inputs, outputs, intensities, mask parameters, tiles and kernel
   // spectra; with z_dev set, member b reads z_dev[b].
   int batch;
-  int64_t in_bs, out_bs, inten_bs, mask_bs, t_bs, hr_bs;
+  int64_t in_bs, out_bs, inten_bs, mask_bs, t_bs, hh_bs;
   // Gradients by Parseval (one problem).  spec_mode 1: rs_col keeps the input
-  // column spectra in `spec`, unit-major in the hand-off register order
-  // (unit u, slot j, thread t at u P + j TPF + t).  spec_mode 2: rs_col adds
-  // Re(conj(G) dg[i] U) over its column into gpart[i][unit] for each
+  // column spectra in `spec`, in the hand-off register order of its blocks
+  // (block b, slot j, thread tid at (b SLOTS + j) NT + tid).  spec_mode 2: rs_col adds
+  // Re(conj(G) dg[i] U) over its column into gpart[i][comp P + column] for each
   // derivative spectrum dg[i] (Hhat layout) that is set.
   int spec_mode;
   int dg_built;           // spec_mode 2: the derivative spectra were built by the forward call
   int partials_only;      // spec_mode 2: leave the partial sums in gpart (no grad_out reduction)
   float2* spec;
   float2* dg[2];          // spec_mode 1: derivative spectra to build with the kernel spectrum
+  float2* dgr[2];         // their row transforms (Hr layout), while they are built with it
   double* gpart[2];
   double* grad_out;       // spec_mode 2: out[i] = sum of gpart[i]
   double* qf_out;         // optional: quality factor of member b at qf_out[b]
@@ -83,8 +85,8 @@ __device__ __forceinline__ RsArgs rs_member(const RsArgs& a0, int b) {
   a.out += b * a0.out_bs;
   if (a.intensity) a.intensity += b * a0.inten_bs;
   a.t += b * a0.t_bs;
-  a.hr += b * a0.hr_bs;
-  a.hmid += b * a0.hr_bs;
+  a.hr += b * a0.t_bs;
+  a.hh += b * a0.hh_bs;
   if (a.z_dev) a.z_dev += b;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -192,39 +194,98 @@ __device__ __forceinline__ float2 stream_load(const float2* p) {
   return make_float2(__builtin_nontemporal_load(&p->x), __builtin_nontemporal_load(&p->y));
 }
 
-// Hr tile index of (row r, column c): P/8 row groups
-__device__ __forceinline__ int64_t hr_idx(int r, int c, int P) {
-  return ((int64_t)(c >> 2) * (P / 8) + (r >> 2)) * 16 + (r & 3) * 4 + (c & 3);
+// Elements of Hr (n rows, columns kx <= P/2): at most half the n x P tiles of
+// one component of T, where it lives until rs_urow writes T.
+__host__ __device__ constexpr int64_t rs_hr_elems(int n, int P) { return (int64_t)(P / 8 + 1) * ((n + 3) / 4) * 16; }
+// Column stride of Hhat: ky = 0..P/2 and a pad to whole 128 B lines.
+__host__ __device__ constexpr int rs_hh_stride(int P) { return P / 2 + 16; }
+
+// A transform of P points runs on TPF = P/16 threads (one radix-16 butterfly
+// each per pass) in one LDS buffer.  A block takes G rows (or columns) of one
+// 4x4 tile group, lanes spread over the G transforms, so that an access of a
+// wave covers G/4 of each 128 B line it touches instead of a quarter; more
+// than one 35 KB buffer behind common barriers hides less of the transforms'
+// latency, and small grids need all their blocks.  Chosen per kernel (us, one
+// component set of P/2 squared samples, MI355X):
+//                      P = 4096          2048             1024          512
+//                      G = 1     2       1     2     4    1     2       2     4
+//   hrow               26.6  28.2    10.1  10.2  10.2   7.7   7.7     7.2   7.4
+//   hcol               19.2  23.9     7.8   8.0  10.3   4.8   5.3     4.7   5.2
+//   urow (3 comp.)     90.8  97.9    23.7  22.6  25.0  13.6  13.4    10.6  11.6
+//   urow, plain input  78.2  69.5    17.6  17.1  18.8   7.8   6.8     4.4   4.6
+//   col (3 comp.)       133   151    39.2  38.8  51.0  12.6  13.1     6.9   8.2
+//   col (1 comp.)                    15.6  14.8         7.9   7.5
+//   final (3 comp.)    74.5  66.7    17.1  15.0  17.4   6.5   5.8     4.4   4.4
+// Below P = 1024 a block holds at least one wave.
+constexpr int rs_g(int P, int g4096, int g2048, int g1024) {
+  return P >= 4096 ? g4096 : P >= 2048 ? g2048 : P >= 1024 ? g1024 : 1024 / P;
+}
+template <int P, int G_> struct Units {
+  static constexpr int TPF = P / 16;
+  static constexpr int G = G_;
+  static constexpr int NT = G * TPF;   // threads per block
+  static_assert(NT >= 64, "whole waves");
+  // buffer stride: the G buffers start 32 / G bank pairs apart
+  static constexpr int RAW = LdsLen<P>::value;
+  static constexpr int WANT = G == 1 ? 0 : (G >= 8 ? 4 : 32 / G);
+  static constexpr int LS = G == 1 ? RAW : RAW + (WANT - RAW % 32 + 32) % 32;
+  // column pass: neighbouring lanes on the G columns of a row
+  __device__ static int col_g(int tid) { return G == 1 ? 0 : tid % G; }
+  __device__ static int col_t(int tid) { return G == 1 ? tid : tid / G; }
+  // row passes: four neighbouring lanes on four columns, then the G rows
+  __device__ static int row_g(int tid) { return G == 1 ? 0 : (tid / 4) % G; }
+  __device__ static int row_t(int tid) { return G == 1 ? tid : tid / (4 * G) * 4 + tid % 4; }
+};
+template <int P> using UHrow = Units<P, rs_g(P, 1, 1, 1)>;
+template <int P> using UHcol = Units<P, rs_g(P, 1, 1, 1)>;
+template <int P, bool ONE> using UUrow = Units<P, rs_g(P, ONE ? 2 : 1, 2, 2)>;
+template <int P> using UCol = Units<P, rs_g(P, 1, 2, 1)>;
+template <int P> using UFinal = Units<P, rs_g(P, 2, 2, 2)>;
+
+// Element `off` (a per-lane 32-bit offset) from a block-uniform base: one
+// offset register serves all accesses of a thread.
+__device__ __forceinline__ float2 ld_at(const float2* base, uint32_t off) {
+  return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(base) + off * (uint32_t)sizeof(float2));
+}
+__device__ __forceinline__ void st_at(float2* base, uint32_t off, float2 v) {
+  *reinterpret_cast<float2*>(reinterpret_cast<char*>(base) + off * (uint32_t)sizeof(float2)) = v;
 }
 
-// Rows or columns per block for the one-FFT-per-group kernels: an FFT runs on
-// P/16 threads (one radix-16 butterfly each per pass) in one LDS buffer of
-// 35 KB at P = 4096, so four blocks share a CU and their pass barriers
-// interleave; below a wave of threads per FFT a block takes several.
-template <int P> struct Units {
-  static constexpr int TPF = P / 16;
-  static constexpr int CPB = TPF >= 64 ? 1 : 64 / TPF;
+// The tiles of G rows row0..row0+G-1 seen by a row pass's thread (transform g,
+// sample t + k): uniform base of row0, lane offset, and step(k) from k (a
+// multiple of 4).
+struct RowTiles {
+  int nrg;
+  uint32_t lane;
+  __device__ RowTiles(int n, int g, int t) : nrg((n + 3) >> 2) {
+    lane = (uint32_t)((t >> 2) * nrg + (g >> 2)) * 16 + (g & 3) * 4 + (t & 3);
+  }
+  __device__ static int64_t base(int row0) { return (row0 >> 2) * 16 + (row0 & 3) * 4; }
+  __device__ int64_t step(int k) const { return (int64_t)(k >> 2) * nrg * 16; }
 };
 
-// One kernel row per group: H of rows 0..P/2-1 generated in float64 phase
+// G kernel rows per block: H of rows 0..N-1 generated in float64 phase
 // (the array is even in x: columns above P/2 mirror), row FFT, stored as Hr
 // for kx <= P/2 (the transform of an even row is even).  DM != 0: the rows
 // of the derivative kernels in the bit set DM (bit 0 dH/dz, bit 1 dH/dk) are
 // formed from the same geometry, held in registers while H is transformed,
-// then transformed in turn into dg[i] (a forward call that will be
+// then transformed in turn into dgr[i] (a forward call that will be
 // differentiated in z / lambda builds its derivative spectra this way).
 template <int P, int DM = 0>
-__global__ __launch_bounds__(Units<P>::CPB * (P / 16), 4) void rs_hrow_kernel(RsArgs a0) {
+__global__ __launch_bounds__(UHrow<P>::NT, 4) void rs_hrow_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
-  constexpr int TPF = P / 16, LS = LdsLen<P>::value, CPB = Units<P>::CPB;
+  using U = UHrow<P>;
+  constexpr int TPF = U::TPF;
   constexpr int NCOL = (P / 2 + 1 + TPF - 1) / TPF;   // columns kx <= P/2 per thread
-  __shared__ float2 lds[CPB * LS];
-  const int g = threadIdx.x / TPF, t = threadIdx.x % TPF;
-  float2* s = lds + g * LS;
-  const int r = xcd_remap(blockIdx.x, gridDim.x) * CPB + g;      // rows 0..P/2-1
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, r = row0 + g;
+  const RowTiles rt(a.n, g, t);
+  const bool store_ok = r < rt.nrg * 4;
   const double z = a.z_dev ? *a.z_dev : a.z;
   double dy;
-  const bool rowok = lag_of(a.y, r, a.n, P, &dy);
+  const bool rowok = lag_of(a.y, r, a.n, P, &dy) && r < a.n;
   float2 dv[2][NCOL];
 #pragma unroll
   for (int i = 0; i < NCOL; ++i) {
@@ -249,8 +310,9 @@ __global__ __launch_bounds__(Units<P>::CPB * (P / 16), 4) void rs_hrow_kernel(Rs
   NoIO none;
   typename LastPass<P, TPF, true>::Type unused;
   {
-    auto store = [&](int c, float2 v) {
-      if (c <= P / 2) a.hr[hr_idx(r, c, P)] = v;
+    float2* dst = a.hr + RowTiles::base(row0);
+    auto store = [&](int k, float2 v) {
+      if (store_ok && (k < P / 2 || (k == P / 2 && t == 0))) st_at(dst + rt.step(k), rt.lane, v);
     };
     fft_io<P, TPF, false, SRC_LDS, DST_FN>(s, t, none, store, unused);
   }
@@ -267,105 +329,64 @@ __global__ __launch_bounds__(Units<P>::CPB * (P / 16), 4) void rs_hrow_kernel(Rs
       if (c > 0 && c < P / 2) s[lpad(P - c)] = dv[d][i];
     }
     __syncthreads();
-    float2* dst = a.dg[d];
-    auto store = [&](int c, float2 v) {
-      if (c <= P / 2) dst[hr_idx(r, c, P)] = v;
+    float2* dst = a.dgr[d] + RowTiles::base(row0);
+    auto store = [&](int k, float2 v) {
+      if (store_ok && (k < P / 2 || (k == P / 2 && t == 0))) st_at(dst + rt.step(k), rt.lane, v);
     };
     fft_io<P, TPF, false, SRC_LDS, DST_FN>(s, t, none, store, unused);
   }
 }
 
-// One block per input row: the masks / Ez of each pixel are computed once by
-// one thread for all components, component c is transformed by threads
-// [c*TPF, (c+1)*TPF) in LDS buffer c.  Rows 4g..4g+3 run back to back on one
-// XCD, so the four 32 B row slices of each 128 B tile meet in the same L2.
-template <int P>
-__global__ __launch_bounds__(3 * (P / 16)) void rs_urow_kernel(RsArgs a0) {
-  const RsArgs a = rs_member(a0, blockIdx.y);
-  constexpr int TPF = P / 16, LS = LdsLen<P>::value;
-  extern __shared__ float2 lds[];
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int f = tid / TPF, t = tid % TPF;
-  const int nrg = (a.n + 3) >> 2;
-  const int row = xcd_remap(blockIdx.x, gridDim.x);
-  const int nc = a.ncomp;
-  const double z = a.z_dev ? *a.z_dev : a.z;
-  for (int col = tid; col < P / 2; col += nthr) {
-    float2 e0 = make_float2(0.f, 0.f), e1 = e0, e2 = e0;
-    if (row < a.n && col < a.n) {
-      const int64_t pix = (int64_t)row * a.n + col;
-      e0 = a.in[pix];
-      if (a.nin > 1) e1 = a.in[a.in_cs + pix];
-      if (a.nin > 2) e2 = a.in[2 * a.in_cs + pix];
-      apply_mask(a.mask, pix, e0, e1, e2);
-      if (a.ez_mode != EZ_NONE) e2 = build_ez(a.ez_mode, e0, e1, a.x[col], a.y[row], z);
-    }
-    lds[lpad(col)] = e0;
-    lds[lpad(col + P / 2)] = make_float2(0.f, 0.f);
-    if (nc > 1) { lds[LS + lpad(col)] = e1; lds[LS + lpad(col + P / 2)] = make_float2(0.f, 0.f); }
-    if (nc > 2) { lds[2 * LS + lpad(col)] = e2; lds[2 * LS + lpad(col + P / 2)] = make_float2(0.f, 0.f); }
-  }
-  __syncthreads();
-  const int rg = row >> 2, rr = row & 3;
-  float2* dst = a.t + (int64_t)f * nrg * 4 * P + rg * 16 + rr * 4;
-  NoIO none;
-  auto store = [&](int col, float2 v) { dst[(int64_t)(col >> 2) * nrg * 16 + (col & 3)] = v; };
-  typename LastPass<P, TPF, true>::Type unused;
-  fft_io<P, TPF, false, SRC_LDS, DST_FN>(lds + f * LS, t, none, store, unused);
-}
-
-// One input row per block of P/16 threads and one 35 KB buffer, so several
-// blocks share a CU.  Thread t's first-pass inputs are the columns
+// G input rows per block.  Thread t's first-pass inputs are the columns
 // t + r P/16; the nonzero ones (columns < N <= P/2) are r < 8, so each thread
 // computes the masks and Ez of exactly those 8 pixels once, keeps all
 // components in registers, and the components are transformed one after the
 // other from there (no LDS staging pass).
 // ONE (inputs without masks or Ez construction: the adjoint's cotangent): one
-// (row, component) unit per block, the components of a row on consecutive
-// blocks, for grids whose row blocks alone leave resident slots empty.
+// component (blockIdx.z) per block, for grids whose row blocks alone leave
+// resident slots empty.
 template <int P, bool ONE = false>
-__global__ __launch_bounds__(P / 16) void rs_urow1_kernel(RsArgs a0) {
+__global__ __launch_bounds__((UUrow<P, ONE>::NT)) void rs_urow_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
-  constexpr int TPF = P / 16, LS = LdsLen<P>::value;
+  using U = UUrow<P, ONE>;
+  constexpr int TPF = U::TPF;
   constexpr int R0 = FftPlan<P>::radix(true, 0);
   static_assert(R0 == 16 && P / R0 == TPF, "first pass: one radix-16 butterfly per thread");
   constexpr int H = R0 / 2;   // inputs r < H hold the N <= P/2 pixels
-  __shared__ float2 lds[LS];
-  const int t = threadIdx.x;
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
+  const RowTiles rt(a.n, g, t);
+  const bool store_ok = row < rt.nrg * 4, rowok = row < a.n;
+  NoIO none;
+  typename LastPass<P, TPF, true>::Type unused;
   if constexpr (ONE) {
-    const int unit = xcd_remap(blockIdx.x, gridDim.x);
-    const int row = unit / a.ncomp, c = unit - row * a.ncomp;
-    const int nrg = (a.n + 3) >> 2, rg = row >> 2, rr = row & 3;
-    const float2* src = a.in + (int64_t)c * a.in_cs;
+    const int c = blockIdx.z;
+    const float2* src = a.in + (int64_t)c * a.in_cs + (int64_t)row0 * a.n;
     Regs<1, R0> rin;
 #pragma unroll
     for (int r = 0; r < R0; ++r) {
       const int col = t + r * TPF;
-      rin.v[0][r] = (r < H && row < a.n && col < a.n) ? src[(int64_t)row * a.n + col] : make_float2(0.f, 0.f);
+      rin.v[0][r] = (r < H && rowok && col < a.n) ? ld_at(src + r * TPF, g * a.n + t) : make_float2(0.f, 0.f);
     }
-    NoIO none;
-    float2* dst = a.t + (int64_t)c * nrg * 4 * P + rg * 16 + rr * 4;
-    auto store = [&](int col, float2 v) { dst[(int64_t)(col >> 2) * nrg * 16 + (col & 3)] = v; };
-    typename LastPass<P, TPF, true>::Type unused;
-    chain_io<P, TPF, false, true, 0, SRC_REG, DST_FN, true, false>(lds, t, none, store, rin, unused);
+    float2* dst = a.t + (int64_t)c * rt.nrg * 4 * P + RowTiles::base(row0);
+    auto store = [&](int k, float2 v) {
+      if (store_ok) st_at(dst + rt.step(k), rt.lane, v);
+    };
+    chain_io<P, TPF, false, true, 0, SRC_REG, DST_FN, true, false>(s, t, none, store, rin, unused);
     return;
   }
-  const int row = xcd_remap(blockIdx.x, gridDim.x);
-  const int nrg = (a.n + 3) >> 2, rg = row >> 2, rr = row & 3;
   const int nc = a.ncomp;
   const double z = a.z_dev ? *a.z_dev : a.z;
   // all loads of the 8 pixels first (in flight together), then the masks and Ez
-  const bool rowok = row < a.n, ez = a.ez_mode != EZ_NONE;
+  const bool ez = a.ez_mode != EZ_NONE;
+  // (columns beyond N read the row's last pixel and are zeroed below)
   PixRaw raw[H];
-  int64_t pix[H];
-  double xc[H];
+  uint32_t pix[H];
+  const uint32_t row_at = (uint32_t)(rowok ? row : 0) * a.n;
 #pragma unroll
-  for (int r = 0; r < H; ++r) {
-    const int col = t + r * TPF;
-    const bool ok = rowok && col < a.n;
-    pix[r] = ok ? (int64_t)row * a.n + col : 0;
-    xc[r] = ez ? a.x[ok ? col : 0] : 0.0;
-  }
+  for (int r = 0; r < H; ++r) pix[r] = row_at + min(t + r * TPF, a.n - 1);
   pix_load_n<H>(a.in, a.in_cs, a.nin, a.mask, pix, raw);
   const double yr = ez ? a.y[rowok ? row : 0] : 0.0;
   float2 e[3][H];
@@ -375,75 +396,76 @@ __global__ __launch_bounds__(P / 16) void rs_urow1_kernel(RsArgs a0) {
     float2 e0 = make_float2(0.f, 0.f), e1 = e0, e2 = e0;
     if (rowok && col < a.n) {
       pix_masked(a.mask, raw[r], e0, e1, e2);
-      if (ez) e2 = build_ez(a.ez_mode, e0, e1, xc[r], yr, z);
+      if (ez) e2 = build_ez(a.ez_mode, e0, e1, at32(a.x, col), yr, z);
     }
     e[0][r] = e0;
     e[1][r] = e1;
     e[2][r] = e2;
   }
-  NoIO none;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     if (c >= nc) break;
     Regs<1, R0> rin;
 #pragma unroll
     for (int r = 0; r < R0; ++r) rin.v[0][r] = r < H ? e[c][r] : make_float2(0.f, 0.f);
-    float2* dst = a.t + (int64_t)c * nrg * 4 * P + rg * 16 + rr * 4;
-    auto store = [&](int col, float2 v) { dst[(int64_t)(col >> 2) * nrg * 16 + (col & 3)] = v; };
-    typename LastPass<P, TPF, true>::Type unused;
-    chain_io<P, TPF, false, true, 0, SRC_REG, DST_FN, true, false>(lds, t, none, store, rin, unused);
+    float2* dst = a.t + (int64_t)c * rt.nrg * 4 * P + RowTiles::base(row0);
+    auto store = [&](int k, float2 v) {
+      if (store_ok) st_at(dst + rt.step(k), rt.lane, v);
+    };
+    chain_io<P, TPF, false, true, 0, SRC_REG, DST_FN, true, false>(s, t, none, store, rin, unused);
   }
 }
 
-// Kernel spectrum.  Per column kx <= P/2: the Hr column (rows mirrored, row
-// P/2 zero) is transformed along y and the spectrum, times dx dy / P^2
-// (conjugated for the adjoint), replaces the Hr column in place for ky < P/2;
-// ky = P/2 goes to hmid[col].  The array is even in y and in x, so ky > P/2
-// and kx > P/2 are not formed (Hhat(P - ky, kx) = Hhat(ky, P - kx) = Hhat(ky, kx)).
-// Blocks beyond the P/2 + 1 columns (grid padding for the XCD remap) idle.
+// Kernel spectrum.  Per column kx <= P/2: the Hr column (rows mirrored, rows
+// N..P-N zero) is transformed along y and the spectrum, times dx dy / P^2
+// (conjugated for the adjoint), stored contiguously for ky <= P/2.  The array
+// is even in y and in x, so ky > P/2 and kx > P/2 are not formed
+// (Hhat(P - ky, kx) = Hhat(ky, P - kx) = Hhat(ky, kx)).
 template <int P>
-__global__ __launch_bounds__(Units<P>::CPB * (P / 16), 4) void rs_hcol_kernel(RsArgs a0) {
+__global__ __launch_bounds__(UHcol<P>::NT, 4) void rs_hcol_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
-  constexpr int TPF = P / 16, LS = LdsLen<P>::value, CPB = Units<P>::CPB;
+  using U = UHcol<P>;
+  constexpr int TPF = U::TPF;
   using HO = HandOff<P, TPF>;
-  __shared__ float2 lds[CPB * LS];
-  const int g = threadIdx.x / TPF, t = threadIdx.x % TPF;
-  float2* s = lds + g * LS;
-  const int col = xcd_remap(blockIdx.x, gridDim.x) * CPB + g;
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::col_g(threadIdx.x), t = U::col_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int col0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, col = col0 + g;
   const bool act = col <= P / 2;
-  if (CPB == 1 && !act) return;   // whole block
-  const int cg = col >> 2, cc = col & 3;
-  float2* hc = a.hr + (int64_t)cg * (P / 8) * 16 + cc;
-  auto load = [&](int r) -> float2 {
-    const int rr = r <= P / 2 ? r : P - r;
-    return (!act || rr == P / 2) ? make_float2(0.f, 0.f) : hc[(rr >> 2) * 16 + (rr & 3) * 4];
+  const int nrg = (a.n + 3) >> 2;
+  const float2* hc = a.hr + (int64_t)(col0 >> 2) * nrg * 16 + (col0 & 3);
+  const uint32_t lane = (g >> 2) * nrg * 16 + (g & 3);
+  auto load = [&](int k) -> float2 {
+    const int r = t + k, rr = r <= P / 2 ? r : P - r;
+    return (act && rr < a.n) ? ld_at(hc, lane + 4 * rr) : make_float2(0.f, 0.f);
   };
   typename HO::Type u;
   fft_forward_to_regs<P, TPF, SRC_FN>(s, t, load, u);
+  constexpr int HS = rs_hh_stride(P);
+  float2* dst = a.hh + (int64_t)col0 * HS;
 #pragma unroll
   for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
     for (int q = 0; q < HO::R; ++q) {
-      const int ky = HO::index(t, b, q);
+      const int k = HO::koff(b, q);
+      if (k > P / 2) continue;
       float2 h = u.v[b][q] * a.scale;
       if (a.adjoint && !a.hstored) h = conjf2(h);
-      if (!act) continue;
-      if (ky < P / 2) hc[(ky >> 2) * 16 + (ky & 3) * 4] = h;
-      else if (ky == P / 2) a.hmid[col] = h;
+      if (act && (k < P / 2 || t == 0)) st_at(dst + k, g * HS + t, h);
     }
 }
 
-// Sum of v over the TPF threads of each group (groups of TPF < 64 share a
-// wave, aligned to TPF lanes), fixed order; every thread of the block calls
-// it.  `red` holds CPB * (TPF / 64) values when TPF > 64.
-template <int TPF>
-__device__ __forceinline__ double group_sum_f64(double v, double* red, int g, int t) {
-  constexpr int W = TPF < 64 ? TPF : 64;
+// Sum of v over the threads of each of the block's G columns (column g on the
+// lanes tid % G), fixed order; every thread of the block calls it and thread
+// t = 0 of the column holds the sum.  `red` holds G * (waves per block) values.
+template <int P> __device__ __forceinline__ double column_sum_f64(double v, double* red) {
+  using U = UCol<P>;
+  constexpr int NW = U::NT / 64;
 #pragma unroll
-  for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if constexpr (TPF > 64) {
-    constexpr int NW = TPF / 64;
-    if ((t & 63) == 0) red[g * NW + (t >> 6)] = v;
+  for (int o = 32; o >= U::G; o >>= 1) v += __shfl_xor(v, o, 64);
+  if constexpr (NW > 1) {
+    const int g = U::col_g(threadIdx.x), lane = threadIdx.x & 63;
+    if (lane < U::G) red[g * NW + (threadIdx.x >> 6)] = v;
     __syncthreads();
     v = 0.0;
 #pragma unroll
@@ -452,193 +474,146 @@ __device__ __forceinline__ double group_sum_f64(double v, double* red, int g, in
   return v;
 }
 
-// spec_mode 2 of the column pass, after its multiply loop has accumulated
-// acc[i] = sum over the thread's ky of Re(conj(G) dg[i] U) (G the spectrum in
-// registers, the cotangent's; U the kept input spectrum; dg[i] the derivative
-// spectrum, even in kx and ky like Hhat): the unit's sums, fixed order, into
-// gpart[i][unit] for i in the bit set GB.
-template <int TPF, int CPB, int GB>
-__device__ __forceinline__ void rs_col_dot_sums(const RsArgs& a, const double (&acc)[2], int unit, int g, int t) {
-  constexpr int NW = TPF > 64 ? TPF / 64 : 1;
-  __shared__ double red[2][CPB * NW];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    if (!(GB >> i & 1)) continue;
-    const double v = group_sum_f64<TPF>(acc[i], red[i], g, t);
-    if (t == 0) a.gpart[i][unit] = v;
-  }
-}
-
-// Column pass.  One (column, component) unit per thread group: the T column
-// (rows 0..N-1, zero padded) is transformed along y straight from the tiles,
-// multiplied in registers by the kernel spectrum of its column (read from
-// the in-place Hhat, mirrored for ky > P/2), inverse-transformed, and rows
-// 0..N-1 stored back in place.  A block holds one 4096-point FFT (35 KB of
-// LDS), so four blocks share a CU and their pass barriers interleave.  The
-// units of a column and of its tile neighbours run back to back on one XCD,
-// so the Hhat column and the 128 B tile lines are fetched once into its L2.
+// Column pass.  G columns of one component (blockIdx.z) per block: each T
+// column (rows 0..N-1, zero padded) is transformed along y straight from the
+// tiles, multiplied in registers by the kernel spectrum of its column (a
+// contiguous column, mirrored for ky > P/2), inverse-transformed, and rows
+// 0..N-1 stored back in place.  Tile neighbours run back to back on one XCD,
+// so the 128 B tile lines are fetched once into its L2.
+// What bounds it (2048^2, three components): the accesses alone take 112 us
+// (448 MB, 4.0 TB/s), the transforms alone 99 us, together 133 us (141 us with
+// the spectrum in 4x4 tiles and 64-bit addresses per access); more waves, wave
+// priorities or keeping Hhat in registers across the components gain nothing.
 // SPEC 1 also keeps the column's spectrum; SPEC = 2 + GB, GB in 1..3, adds
 // its gradient dots for the derivative spectra in the bit set GB (spec_mode 2
-// of RsArgs).
+// of RsArgs): acc[i] = sum over the column's ky of Re(conj(G) dg[i] U), G the
+// spectrum in registers (the cotangent's), U the kept input spectrum.
 template <int P, int SPEC>
-__global__ __launch_bounds__(Units<P>::CPB * (P / 16), 4) void rs_col_kernel(RsArgs a0) {
+__global__ __launch_bounds__(UCol<P>::NT, 4) void rs_col_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
-  if (a.qf_out && blockIdx.x == 0 && threadIdx.x == 0)
+  if (a.qf_out && blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x == 0)
     a.qf_out[blockIdx.y] = rs_quality_factor(a.z_dev ? *a.z_dev : a.z, a.qf_rmax, a.qf_dr, a.qf_wl);
-  constexpr int TPF = P / 16, LS = LdsLen<P>::value, CPB = Units<P>::CPB;
+  using U = UCol<P>;
+  constexpr int TPF = U::TPF, NT = U::NT, HS = rs_hh_stride(P);
   using HO = HandOff<P, TPF>;
-  __shared__ float2 lds[CPB * LS];
-  const int g = threadIdx.x / TPF, t = threadIdx.x % TPF;
-  float2* s = lds + g * LS;
-  const int unit = xcd_remap(blockIdx.x, gridDim.x) * CPB + g;
-  const int col = unit / a.ncomp, comp = unit - col * a.ncomp;
-  const bool active = col < P;
-  const int nrg = (a.n + 3) >> 2;
-  const int nr = nrg * 4;
-  const int cg = col >> 2, cc = col & 3;
-  const int hcol = col <= P / 2 ? col : P - col;   // Hhat is even in kx
-  const float2* hc = a.hr + (int64_t)(hcol >> 2) * (P / 8) * 16 + (hcol & 3);
-  float2* tc = a.t + (int64_t)comp * nrg * 4 * P + (int64_t)cg * nrg * 16 + cc;
-  auto load = [&](int r) -> float2 {
-    return (active && r < nr) ? tc[(r >> 2) * 16 + (r & 3) * 4] : make_float2(0.f, 0.f);
+  constexpr int SLOTS = HO::BPT * HO::R;
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::col_g(threadIdx.x), t = U::col_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int ub = xcd_remap(blockIdx.x, gridDim.x), comp = blockIdx.z;
+  const int col0 = ub * U::G, col = col0 + g;
+  const int nrg = (a.n + 3) >> 2, nr = nrg * 4;
+  // column element r of a tile group is 4 r elements in
+  float2* tc = a.t + (int64_t)comp * nrg * 4 * P + (int64_t)(col0 >> 2) * nrg * 16 + (col0 & 3);
+  const uint32_t lane = (g >> 2) * nrg * 16 + (g & 3) + 4 * t;
+  auto load = [&](int k) -> float2 { return t + k < nr ? ld_at(tc + 4 * k, lane) : make_float2(0.f, 0.f); };
+  // Hhat is even in kx and ky: ky = t + k at lo + k for k < P/2 (and ky = P/2),
+  // at hi + (P - k) above
+  const uint32_t hcol = (uint32_t)(col <= P / 2 ? col : P - col) * HS;
+  auto hat = [&](const float2* base, int k) -> float2 {
+    return k < P / 2 ? ld_at(base + k, hcol + t) : ld_at(base, hcol + (P - k) - t);
   };
-  typename HO::Type u;
+  typename HO::Type u, h;
   constexpr int GB = SPEC >= 3 ? SPEC - 2 : 0;
+  float2* sp = nullptr;
+  if constexpr (SPEC != 0) sp = a.spec + ((int64_t)comp * gridDim.x + ub) * SLOTS * NT;
   // the gradient dots (SPEC >= 3) read the kept input spectrum U: up to
   // P = 2048 its loads issue before the forward transform and complete behind
-  // it (at 4096 they would not fit beside the transform's registers)
-  constexpr bool UPRE = GB != 0 && P <= 2048;
+  // it (at 4096, or with both derivatives, they would not fit beside the
+  // transform's registers)
+  constexpr bool UPRE = (GB == 1 || GB == 2) && P <= 2048;
   typename HO::Type uk;
   if constexpr (UPRE) {
-    const float2* sp = a.spec + (int64_t)unit * P + t;
 #pragma unroll
     for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
-      for (int q = 0; q < HO::R; ++q) uk.v[b][q] = active ? stream_load(sp + (b * HO::R + q) * TPF) : make_float2(0.f, 0.f);
+      for (int q = 0; q < HO::R; ++q) uk.v[b][q] = stream_load(sp + (b * HO::R + q) * NT + threadIdx.x);
   }
   // rows >= N <= P/2 are zero padding, and the rows kept are < N: the first
   // forward pass skips the upper half of its inputs, the last inverse pass
   // the upper half of its outputs
-  fft_forward_to_regs<P, TPF, SRC_FN, true>(s, t, load, u);
-  if constexpr (SPEC == 1) {
-    if (active) {
-      float2* sp = a.spec + (int64_t)unit * P + t;
+  constexpr bool HPRE = GB == 0;
+  auto hook = [&]() {
+    if constexpr (HPRE) {
 #pragma unroll
       for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
-        for (int q = 0; q < HO::R; ++q) stream_store(sp + (b * HO::R + q) * TPF, u.v[b][q]);
+        for (int q = 0; q < HO::R; ++q) h.v[b][q] = hat(a.hh, HO::koff(b, q));
     }
-  }
-  const float hs = (a.adjoint && a.hstored) ? -1.f : 1.f;   // stored spectrum: conjugate for the adjoint
-  double acc[2] = {0.0, 0.0};
-  if (active) {
-    // dg is read in the same loop as the kernel spectrum, at the same Hhat offsets
+  };
+  fft_forward_to_regs<P, TPF, SRC_FN, true>(s, t, load, u, hook);
+  if constexpr (SPEC == 1) {
 #pragma unroll
     for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
-      for (int q = 0; q < HO::R; ++q) {
-        const int ky = HO::index(t, b, q);
-        const int kk = ky <= P / 2 ? ky : P - ky;
-        const int64_t ho = (int64_t)(hcol >> 2) * (P / 8) * 16 + (hcol & 3) + (kk >> 2) * 16 + (kk & 3) * 4;
-        float2 h = kk == P / 2 ? a.hmid[hcol] : hc[(kk >> 2) * 16 + (kk & 3) * 4];
-        h.y *= hs;
-        if constexpr (GB != 0) {
-          const float2 uv = UPRE ? uk.v[b][q] : stream_load(a.spec + (int64_t)unit * P + t + (b * HO::R + q) * TPF);
-          const float2 gv = u.v[b][q];
-          const int64_t di = kk == P / 2 ? (int64_t)(P / 2) * P + hcol : ho;
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            if (!(GB >> i & 1)) continue;
-            const float2 w = cmul(a.dg[i][di], uv);
-            acc[i] += (double)(gv.x * w.x + gv.y * w.y);
-          }
-        }
-        u.v[b][q] = cmul(u.v[b][q], h);
-      }
+      for (int q = 0; q < HO::R; ++q) stream_store(sp + (b * HO::R + q) * NT + threadIdx.x, u.v[b][q]);
   }
-  auto store = [&](int r, float2 v) {
-    if (active && r < nr) tc[(r >> 2) * 16 + (r & 3) * 4] = v;
+  const float hs = (a.adjoint && a.hstored) ? -1.f : 1.f;   // stored spectrum: conjugate for the adjoint
+  double acc[2] = {0.0, 0.0};
+#pragma unroll
+  for (int b = 0; b < HO::BPT; ++b)
+#pragma unroll
+    for (int q = 0; q < HO::R; ++q) {
+      const int k = HO::koff(b, q);
+      float2 hv = HPRE ? h.v[b][q] : hat(a.hh, k);
+      hv.y *= hs;
+      if constexpr (GB != 0) {
+        const float2 uv = UPRE ? uk.v[b][q] : stream_load(sp + (b * HO::R + q) * NT + threadIdx.x);
+        const float2 gv = u.v[b][q];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (!(GB >> i & 1)) continue;
+          // roundings written out: the float64 gradient shows them
+          const float2 d = hat(a.dg[i], k);
+          const float wx = fmaf(d.x, uv.x, -__fmul_rn(d.y, uv.y)), wy = fmaf(d.x, uv.y, __fmul_rn(d.y, uv.x));
+          acc[i] += (double)fmaf(gv.x, wx, __fmul_rn(gv.y, wy));
+        }
+        // the sums are formed here: sunk behind the inverse transform, their
+        // operands would spill
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (GB >> i & 1) asm volatile("" : "+v"(acc[i]));
+      }
+      u.v[b][q] = cmul(u.v[b][q], hv);
+    }
+  auto store = [&](int k, float2 v) {
+    if (t + k < nr) st_at(tc + 4 * k, lane, v);
   };
   fft_inverse_from_regs<P, TPF, DST_FN, true>(s, t, u, store);
-  if constexpr (GB != 0) rs_col_dot_sums<TPF, CPB, GB>(a, acc, unit, g, t);
-}
-
-// Per block 2 rows (one per thread group): the row halves of
-// each component's tiles are staged into LDS with 64 B loads (the block
-// holding the other two rows of a tile runs next on the same XCD and finds
-// the line in L2), inverse-transformed in LDS, and the first N samples stored;
-// |E|^2 is accumulated over the components.  Two 35 KB buffers per block let
-// two blocks share a CU.
-template <int P>
-__global__ __launch_bounds__(2 * FftThreads<P>::value) void rs_final_kernel(RsArgs a0) {
-  const RsArgs a = rs_member(a0, blockIdx.y);
-  constexpr int TPF = FftThreads<P>::value, LS = LdsLen<P>::value;
-  constexpr int NT = 2 * TPF;
-  constexpr int PPT = (P / 2 + TPF - 1) / TPF;
-  __shared__ float2 lds[2 * LS];
-  const int tid = threadIdx.x, f = tid / TPF, t = tid % TPF;
-  float2* s = lds + f * LS;
-  const int nrg = (a.n + 3) >> 2;
-  const int pair = xcd_remap(blockIdx.x, gridDim.x);
-  const int rg = pair >> 1, r0 = (pair & 1) * 2;
-  const int row = rg * 4 + r0 + f;
-  float inten[PPT];
+  if constexpr (GB != 0) {
+    __shared__ double red[2][U::G * (NT / 64)];
 #pragma unroll
-  for (int i = 0; i < PPT; ++i) inten[i] = 0.f;
-  for (int c = 0; c < a.ncomp; ++c) {
-    const float2* tc = a.t + (int64_t)c * nrg * 4 * P;
-#pragma unroll 4
-    for (int e = tid; e < 2 * P; e += NT) {
-      const int cgp = e >> 3, rr = (e >> 2) & 1, cc = e & 3;
-      lds[rr * LS + lpad(cgp * 4 + cc)] = tc[((int64_t)cgp * nrg + rg) * 16 + (r0 + rr) * 4 + cc];
-    }
-    __syncthreads();
-    fft_lds<P, TPF, true>(s, t);
-    if (row < a.n) {
-      float2* oc = a.out + (int64_t)c * a.out_cs + (int64_t)row * a.n;
-#pragma unroll
-      for (int i = 0; i < PPT; ++i) {
-        const int col = t + i * TPF;
-        if (col < a.n) {
-          const float2 v = s[lpad(col)];
-          oc[col] = v;
-          inten[i] += v.x * v.x + v.y * v.y;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (a.intensity && row < a.n) {
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int col = t + i * TPF;
-      if (col < a.n) a.intensity[(int64_t)row * a.n + col] = inten[i];
+    for (int i = 0; i < 2; ++i) {
+      if (!(GB >> i & 1)) continue;
+      const double v = column_sum_f64<P>(acc[i], red[i]);
+      if (t == 0) a.gpart[i][comp * P + col] = v;
     }
   }
 }
 
-// One output row per block of P/16 threads and one 35 KB buffer, so four
-// blocks share a CU: the components are inverse-transformed one after the
-// other, each read straight from its tiles into the first pass (32 B of each
-// 128 B line; the blocks of the tile's other rows run next on the same XCD),
-// each last pass left in registers, where the first N samples are stored and
-// |E|^2 is accumulated over the components.
-// ONE: one (component, row) unit per block (no |E|^2 to accumulate across
-// components), component-major so a tile's four rows still run back to back:
-// ncomp N blocks divide into the resident slots evenly where N row blocks
-// (2.67 rounds at P = 4096) leave a partly idle last round.
+// G output rows per block: the components are inverse-transformed one after
+// the other, each read straight from its tiles into the first pass (the
+// blocks of a tile's other rows run next on the same XCD), each last pass left
+// in registers, where the first N samples are stored and |E|^2 is accumulated
+// over the components.
+// ONE: one component (blockIdx.z) per block (no |E|^2 to accumulate across
+// components): ncomp N rows divide into the resident slots evenly where N row
+// blocks (2.67 rounds at P = 4096) leave a partly idle last round.
+// Below P = 1024 the passes run in the forward order and form every output
+// (roundings are those of the whole transform).
 template <int P, bool ONE = false>
-__global__ __launch_bounds__(P / 16) void rs_final1_kernel(RsArgs a0) {
+__global__ __launch_bounds__(UFinal<P>::NT) void rs_final_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
-  constexpr int TPF = P / 16, LS = LdsLen<P>::value;
-  using LP = LastPass<P, TPF, false>;
-  __shared__ float2 lds[LS];
-  const int t = threadIdx.x;
-  const int unit = xcd_remap(blockIdx.x, gridDim.x);
-  const int c0 = ONE ? unit / a.n : 0;
-  const int row = ONE ? unit - c0 * a.n : unit;
-  if (row >= a.n || c0 >= a.ncomp) return;   // whole block
-  const int nrg = (a.n + 3) >> 2, rg = row >> 2, rr = row & 3;
+  using U = UFinal<P>;
+  constexpr int TPF = U::TPF;
+  constexpr bool SMALL = P < 1024;
+  using LP = LastPass<P, TPF, SMALL>;
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
+  const RowTiles rt(a.n, g, t);
+  const bool load_ok = row < rt.nrg * 4;
   // output columns < N <= P/2 are slots q < R/2 of the last pass
   constexpr int QH = LP::R / 2;
   float inten[LP::BPT][QH];
@@ -647,22 +622,28 @@ __global__ __launch_bounds__(P / 16) void rs_final1_kernel(RsArgs a0) {
 #pragma unroll
     for (int q = 0; q < QH; ++q) inten[b][q] = 0.f;
   NoIO none;
-  for (int c = c0; c < (ONE ? c0 + 1 : a.ncomp); ++c) {
-    const float2* tc = a.t + (int64_t)c * nrg * 4 * P + rg * 16 + rr * 4;
-    auto load = [&](int col) -> float2 { return tc[(int64_t)(col >> 2) * nrg * 16 + (col & 3)]; };
+  for (int c = ONE ? blockIdx.z : 0; c < (ONE ? blockIdx.z + 1 : a.ncomp); ++c) {
+    const float2* tc = a.t + (int64_t)c * rt.nrg * 4 * P + RowTiles::base(row0);
+    auto load = [&](int k) -> float2 { return load_ok ? ld_at(tc + rt.step(k), rt.lane) : make_float2(0.f, 0.f); };
     typename LP::Type o, unused;
     // the kept columns are < N <= P/2: the last pass forms the lower half only
-    chain_io<P, TPF, true, false, 0, SRC_FN, DST_REG, false, true>(lds, t, load, none, unused, o);
-    float2* oc = a.out + (int64_t)c * a.out_cs + (int64_t)row * a.n;
+    chain_io<P, TPF, true, SMALL, 0, SRC_FN, DST_REG, false, !SMALL>(s, t, load, none, unused, o);
+    if constexpr (SMALL) {
+#pragma unroll
+      for (int b = 0; b < LP::BPT; ++b)
+#pragma unroll
+        for (int q = QH; q < LP::R; ++q) asm volatile("" ::"v"(o.v[b][q].x), "v"(o.v[b][q].y));
+    }
+    float2* oc = a.out + (int64_t)c * a.out_cs + (int64_t)row0 * a.n;
 #pragma unroll
     for (int b = 0; b < LP::BPT; ++b) {
       if (!LP::valid(t, b)) continue;
 #pragma unroll
       for (int q = 0; q < QH; ++q) {
-        const int col = LP::index(t, b, q);
-        if (col < a.n) {
+        const int k = LP::index(0, b, q);
+        if (t + k < a.n && row < a.n) {
           const float2 v = o.v[b][q];
-          oc[col] = v;
+          st_at(oc + k, g * a.n + t, v);
           if constexpr (!ONE) inten[b][q] += v.x * v.x + v.y * v.y;
         }
       }
@@ -674,8 +655,8 @@ __global__ __launch_bounds__(P / 16) void rs_final1_kernel(RsArgs a0) {
       if (!LP::valid(t, b)) continue;
 #pragma unroll
       for (int q = 0; q < QH; ++q) {
-        const int col = LP::index(t, b, q);
-        if (col < a.n) a.intensity[(int64_t)row * a.n + col] = inten[b][q];
+        const int k = LP::index(0, b, q);
+        if (t + k < a.n && row < a.n) a.intensity[(int64_t)row * a.n + t + k] = inten[b][q];
       }
     }
   }
@@ -701,123 +682,101 @@ __global__ __launch_bounds__(1024) void rs_grad_reduce_kernel(const double* p0, 
   }
 }
 
-// Partial sums written by rs_col_kernel<P, 2> for ncomp components (its
-// padded unit count).
-template <int P> inline int rs_col_units(int ncomp) {
-  constexpr int CPB = Units<P>::CPB;
-  return (P * ncomp + CPB - 1) / CPB * CPB;
-}
+inline int rs_rows4(int n) { return ((n + 3) >> 2) * 4; }
+// Grid of `units` rows or columns of nb members and nz components.
+template <class U> inline dim3 rs_grid(int units, int nb, int nz = 1) { return dim3((units + U::G - 1) / U::G, nb, nz); }
 
-// Dynamic-LDS limits of the multi-buffer row kernels (up to three buffers of
-// P points), set once per device by the library's initialisation.
-template <int P> inline hipError_t rs_set_attribute() {
-  return hipFuncSetAttribute((const void*)rs_urow_kernel<P>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             3 * LdsLen<P>::value * (int)sizeof(float2));
-}
-inline hipError_t rs_set_attributes() {
-  hipError_t e = hipSuccess;
-  for (hipError_t r : {rs_set_attribute<64>(), rs_set_attribute<128>(), rs_set_attribute<256>(),
-                       rs_set_attribute<512>()})
-    if (r != hipSuccess) e = r;
-  return e;
+// Launches the kernel-spectrum passes of `a` (H, or the derivative that
+// kernel_dz names) through Hr into a.hh.
+template <int P> inline void rs_spectrum_launch(const RsArgs& a, int nb, hipStream_t st) {
+  hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), rs_grid<UHrow<P>>(rs_rows4(a.n), nb), dim3(UHrow<P>::NT), 0, st, a);
+  hipLaunchKernelGGL(rs_hcol_kernel<P>, rs_grid<UHcol<P>>(P / 2 + 1, nb), dim3(UHcol<P>::NT), 0, st, a);
 }
 
 template <int P>
 inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
-  constexpr int CPB = Units<P>::CPB;
-  const dim3 blk(CPB * (P / 16));
-  const int rows = ((a.n + 3) >> 2) * 4;
+  const int rows = rs_rows4(a.n);
   const int nb = a.batch > 1 ? a.batch : 1;
+  const dim3 ghr = rs_grid<UHrow<P>>(rows, nb), bhr(UHrow<P>::NT), ghc = rs_grid<UHcol<P>>(P / 2 + 1, nb),
+             bhc(UHcol<P>::NT), bcl(UCol<P>::NT), bfn(UFinal<P>::NT);
   // a forward call that keeps its spectra for a gradient builds the derivative
   // spectra with its own kernel rows (one float64 geometry for all of them)
   const int dm = (a.dg[0] ? 1 : 0) | (a.dg[1] ? 2 : 0);
   const bool with_h = a.spec_mode == 1 && dm && !a.hreuse;
-  if (!a.hreuse) {
-    KTimer t(K_RS_HROW, st);
-    if (with_h && dm == 1)
-      hipLaunchKernelGGL((rs_hrow_kernel<P, 1>), dim3(P / 2 / CPB, nb), blk, 0, st, a);
-    else if (with_h && dm == 2)
-      hipLaunchKernelGGL((rs_hrow_kernel<P, 2>), dim3(P / 2 / CPB, nb), blk, 0, st, a);
-    else if (with_h)
-      hipLaunchKernelGGL((rs_hrow_kernel<P, 3>), dim3(P / 2 / CPB, nb), blk, 0, st, a);
-    else
-      hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), dim3(P / 2 / CPB, nb), blk, 0, st, a);
-  }
-  const int ncb = (P / 2 + 1 + CPB - 1) / CPB;   // columns kx <= P/2, grid padded to whole XCD rounds
+  // Hr lives in the tiles that rs_urow fills later, so the spectra come first
   if ((a.spec_mode == 2 && !a.dg_built) || (a.spec_mode == 1 && dm && !with_h)) {
     // derivative spectra (dH/dz, dH/dk) with the spectrum passes, unconjugated
     for (int i = 0; i < 2; ++i) {
       if (!a.dg[i]) continue;
       RsArgs d = a;
-      d.hr = a.dg[i];
-      d.hmid = a.dg[i] + (int64_t)(P / 2) * P;
+      d.hh = a.dg[i];
       d.kernel_dz = i + 1;
       d.adjoint = 0;
       d.hstored = 1;
       KTimer t(K_RS_HROW, st);
-      hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), dim3(P / 2 / CPB, nb), blk, 0, st, d);
-      hipLaunchKernelGGL(rs_hcol_kernel<P>, dim3((ncb + 7) / 8 * 8, nb), blk, 0, st, d);
+      rs_spectrum_launch<P>(d, nb, st);
     }
-  }
-  if constexpr (P >= 1024) {
-    KTimer t(K_RS_UROW, st);
-    bool one = false;
-    if constexpr (P <= 2048) {
-      // plain inputs (no masks, no Ez) over fewer row blocks than resident
-      // slots: one block per (row, component)
-      one = a.ncomp > 1 && a.nin == a.ncomp && a.ez_mode == EZ_NONE && !a.mask.st[0].kind && !a.mask.st[1].kind &&
-            rows * nb < 2048;
-      if (one) hipLaunchKernelGGL((rs_urow1_kernel<P, true>), dim3(rows * a.ncomp, nb), dim3(P / 16), 0, st, a);
-    }
-    if (!one) hipLaunchKernelGGL((rs_urow1_kernel<P, false>), dim3(rows, nb), dim3(P / 16), 0, st, a);
-  } else {
-    KTimer t(K_RS_UROW, st);
-    hipLaunchKernelGGL(rs_urow_kernel<P>, dim3(rows, nb), dim3(a.ncomp * (P / 16)),
-                       (size_t)a.ncomp * LdsLen<P>::value * sizeof(float2), st, a);
   }
   if (!a.hreuse) {
+    {
+      KTimer t(K_RS_HROW, st);
+      if (with_h && dm == 1)
+        hipLaunchKernelGGL((rs_hrow_kernel<P, 1>), ghr, bhr, 0, st, a);
+      else if (with_h && dm == 2)
+        hipLaunchKernelGGL((rs_hrow_kernel<P, 2>), ghr, bhr, 0, st, a);
+      else if (with_h)
+        hipLaunchKernelGGL((rs_hrow_kernel<P, 3>), ghr, bhr, 0, st, a);
+      else
+        hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), ghr, bhr, 0, st, a);
+    }
     KTimer t(K_RS_HCOL, st);
-    hipLaunchKernelGGL(rs_hcol_kernel<P>, dim3((ncb + 7) / 8 * 8, nb), blk, 0, st, a);
+    hipLaunchKernelGGL(rs_hcol_kernel<P>, ghc, bhc, 0, st, a);
     for (int i = 0; with_h && i < 2; ++i) {
       if (!a.dg[i]) continue;
       RsArgs d = a;   // the derivative row transforms, unconjugated
-      d.hr = a.dg[i];
-      d.hmid = a.dg[i] + (int64_t)(P / 2) * P;
+      d.hr = a.dgr[i];
+      d.hh = a.dg[i];
       d.adjoint = 0;
       d.hstored = 1;
-      hipLaunchKernelGGL(rs_hcol_kernel<P>, dim3((ncb + 7) / 8 * 8, nb), blk, 0, st, d);
+      hipLaunchKernelGGL(rs_hcol_kernel<P>, ghc, bhc, 0, st, d);
     }
+  }
+  {
+    KTimer t(K_RS_UROW, st);
+    // plain inputs (no masks, no Ez) over fewer row blocks than resident
+    // slots: one block per (row, component)
+    const bool one = P <= 2048 && a.ncomp > 1 && a.nin == a.ncomp && a.ez_mode == EZ_NONE && !a.mask.st[0].kind &&
+                     !a.mask.st[1].kind && rows * nb < 2048;
+    using U1 = UUrow<P, true>;
+    using U3 = UUrow<P, false>;
+    if (one) hipLaunchKernelGGL((rs_urow_kernel<P, true>), rs_grid<U1>(rows, nb, a.ncomp), dim3(U1::NT), 0, st, a);
+    else hipLaunchKernelGGL((rs_urow_kernel<P, false>), rs_grid<U3>(rows, nb), dim3(U3::NT), 0, st, a);
   }
   {
     KTimer t(K_RS_COL, st);
-    const dim3 grid(rs_col_units<P>(a.ncomp) / CPB, nb);
-    const int gb = (a.dg[0] ? 1 : 0) | (a.dg[1] ? 2 : 0);
+    const dim3 grid = rs_grid<UCol<P>>(P, nb, a.ncomp);
     if (a.spec_mode == 1)
-      hipLaunchKernelGGL((rs_col_kernel<P, 1>), grid, blk, 0, st, a);
-    else if (a.spec_mode == 2 && gb == 1)
-      hipLaunchKernelGGL((rs_col_kernel<P, 3>), grid, blk, 0, st, a);
-    else if (a.spec_mode == 2 && gb == 2)
-      hipLaunchKernelGGL((rs_col_kernel<P, 4>), grid, blk, 0, st, a);
-    else if (a.spec_mode == 2 && gb == 3)
-      hipLaunchKernelGGL((rs_col_kernel<P, 5>), grid, blk, 0, st, a);
+      hipLaunchKernelGGL((rs_col_kernel<P, 1>), grid, bcl, 0, st, a);
+    else if (a.spec_mode == 2 && dm == 1)
+      hipLaunchKernelGGL((rs_col_kernel<P, 3>), grid, bcl, 0, st, a);
+    else if (a.spec_mode == 2 && dm == 2)
+      hipLaunchKernelGGL((rs_col_kernel<P, 4>), grid, bcl, 0, st, a);
+    else if (a.spec_mode == 2 && dm == 3)
+      hipLaunchKernelGGL((rs_col_kernel<P, 5>), grid, bcl, 0, st, a);
     else
-      hipLaunchKernelGGL((rs_col_kernel<P, 0>), grid, blk, 0, st, a);
+      hipLaunchKernelGGL((rs_col_kernel<P, 0>), grid, bcl, 0, st, a);
   }
   if (a.spec_mode == 2 && !a.partials_only) {
     KTimer t(K_LOSS, st);
-    hipLaunchKernelGGL(rs_grad_reduce_kernel, dim3(2), dim3(1024), 0, st, a.gpart[0], a.gpart[1],
-                       rs_col_units<P>(a.ncomp), a.grad_out);
+    hipLaunchKernelGGL(rs_grad_reduce_kernel, dim3(2), dim3(1024), 0, st, a.gpart[0], a.gpart[1], P * a.ncomp,
+                       a.grad_out);
   }
   {
     KTimer t(K_RS_FINAL, st);
-    if constexpr (P >= 1024) {
-      if (a.intensity)
-        hipLaunchKernelGGL((rs_final1_kernel<P, false>), dim3(a.n, nb), dim3(P / 16), 0, st, a);
-      else
-        hipLaunchKernelGGL((rs_final1_kernel<P, true>), dim3(a.n * a.ncomp, nb), dim3(P / 16), 0, st, a);
-    }
+    if (a.intensity)
+      hipLaunchKernelGGL((rs_final_kernel<P, false>), rs_grid<UFinal<P>>(a.n, nb), bfn, 0, st, a);
     else
-      hipLaunchKernelGGL(rs_final_kernel<P>, dim3(rows / 2, nb), dim3(2 * FftThreads<P>::value), 0, st, a);
+      hipLaunchKernelGGL((rs_final_kernel<P, true>), rs_grid<UFinal<P>>(a.n, nb, a.ncomp), bfn, 0, st, a);
   }
   return hipGetLastError();
 }

@@ -65,8 +65,6 @@ int ensure_init() {
   rc = hip_check(hipDeviceSynchronize(), "twiddle init");
   if (rc) return rc;
   // launch attributes are per device: set them here, once, under the lock
-  rc = hip_check(xl::rs_set_attributes(), "RS launch attributes");
-  if (rc) return rc;
   rc = hip_check(xl::czt_set_attributes(), "CZT launch attributes");
   if (rc) return rc;
   rc = hip_check(hipGetSymbolAddress(&g_scratch[dev], HIP_SYMBOL(scratch)), "scratch address");
@@ -142,13 +140,12 @@ size_t rs_ws(int n, int ncomp, int batch = 1) {
 // layout, two arrays of per-unit partial sums; [5] is the total.
 struct RsSpecLayout {
   int64_t off[6];
-  int units;   // padded (column, component) units of the column pass
+  int units;   // (column, component) units of the column pass
 };
 RsSpecLayout rs_spec_layout(int n, int ncomp) {
   const int64_t P = rs_fft_len(n);
-  const int tpf = (int)(P / 16), cpb = tpf >= 64 ? 1 : 64 / tpf;   // Units<P>::CPB
   RsSpecLayout l;
-  l.units = (int)((P * ncomp + cpb - 1) / cpb * cpb);
+  l.units = (int)(P * ncomp);
   auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
   const int64_t hh = ((P / 2) * P + P) * (int64_t)sizeof(float2);
   l.off[0] = 0;
@@ -379,8 +376,8 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
   a.out_cs = p->out_comp_stride;
   a.intensity = p->intensity;
   a.t = (float2*)w;
-  a.hr = p->hhat_mode ? (float2*)p->hhat : a.t + ncomp * nr4 * P;
-  a.hmid = a.hr + (int64_t)(P / 2) * P;
+  a.hr = a.t;   // the row-transformed kernel, until the field's rows take its place
+  a.hh = p->hhat_mode ? (float2*)p->hhat : a.t + ncomp * nr4 * P;
   a.hstored = p->hhat_mode ? 1 : 0;
   a.hreuse = p->hhat_mode == 2 ? 1 : 0;
   a.x = p->x;
@@ -403,10 +400,11 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
   a.inten_bs = batch > 1 ? p->intensity_batch_stride : 0;
   a.mask_bs = batch > 1 ? p->mask_batch_stride : 0;
   a.t_bs = rs_ws_elems(n, ncomp);
-  a.hr_bs = p->hhat_mode ? (int64_t)(P / 2) * P + P : a.t_bs;   // hhat holds one spectrum per member
+  a.hh_bs = p->hhat_mode ? (int64_t)(P / 2) * P + P : a.t_bs;   // hhat holds one spectrum per member
   a.spec_mode = p->spec_mode;
   a.spec = nullptr;
   a.dg[0] = a.dg[1] = nullptr;
+  a.dgr[0] = a.dgr[1] = nullptr;
   a.dg_built = p->spec_mode == 2 && (p->spec_grads & XL_RS_SPEC_PREBUILT) ? 1 : 0;
   a.partials_only = p->spec_mode == 2 && (p->spec_grads & XL_RS_SPEC_PARTIALS) ? 1 : 0;
   a.gpart[0] = a.gpart[1] = nullptr;
@@ -425,6 +423,8 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
       if (p->spec_grads >> i & 1) {
         // a forward call with spec_dg builds nothing: the other call did
         if (!(p->spec_mode == 1 && p->spec_dg)) a.dg[i] = (float2*)(db + l.off[1 + i]);
+        // their row transforms, built with the kernel's: in the spectra's place, which the column pass fills later
+        if (p->spec_mode == 1) a.dgr[i] = a.spec + i * xl::rs_hr_elems(n, P);
         if (p->spec_mode == 2) a.gpart[i] = (double*)(sb + l.off[3 + i]);
       }
   }

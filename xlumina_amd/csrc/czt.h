@@ -330,27 +330,125 @@ __attribute__((amdgpu_waves_per_eu(CztRowsShape<Q, ZL>::WAVES))) void czt_rows_k
   fft_inverse_from_regs<Q, TPF, DST_FN, ZL>(s, t, u, store);
 }
 
-// Per block CPB output columns of the x axis (one per thread group) of one
-// component: the columns of the tiled intermediate feed the first pass, the
-// chirp spectrum is applied in registers, and only the output window is
-// stored with the output-plane factor.  A 128 B tile line holds four columns:
-// the CPB groups of a block (and at CPB = 2 the neighbouring block, kept on
-// the same XCD) share it.  Column-wise, each lane's 8 B access is a line of
-// its own (64 lines per wave for the output rows); staged through LDS, a wave
-// stores CPB-column row segments and loads whole tile lines.  ZL as in the
-// row kernel.
+// The same pass with one buffer per transform: a row per block of Q/16
+// threads, the components transformed one after the other.  Thread t's
+// first-pass inputs are the columns t + r Q/16, so it forms the pre-ops of
+// exactly its own pixels (8 where the upper half is zero, ZL) and keeps all
+// components of them in registers: no staging pass, and a CU holds three or
+// four independent blocks where the three-buffer block of a 4096-point row
+// runs alone.  MULTI: more than one component.  Used for one component (8 x
+// 1024^2 of the 4f systems 95 -> 86 us, 777 -> 301 samples 14.1 -> 12.7 us)
+// and for the 4096-point zero-half rows (2048 -> 512, three components, 121 ->
+// 104 us: accesses and exchanges alone take 65, transforms and pre-ops 82; it
+// needs 168 VGPRs).  At 2048 and below with several components the
+// three-buffer block already shares its CU and stays faster (1024^2, HNA rows:
+// 33 us against 38 us, whose registers spill).
+template <int Q> using CztRows1 = Units<Q, rs_g(Q, 1, 1, 1)>;
+
+template <int Q, int K, bool ZL, bool MULTI>
+__global__ __launch_bounds__(CztRows1<Q>::NT, MULTI ? 3 : 4) void czt_rows1_kernel(CztArgs a0) {
+  const CztArgs a = czt_member(a0, blockIdx.y);
+  using U = CztRows1<Q>;
+  constexpr int TPF = U::TPF, H = ZL ? 8 : 16, NC = MULTI ? 3 : 1;
+  using HO = HandOff<Q, TPF>;
+  static_assert(FftPlan<Q>::radix(true, 0) == 16, "first pass: one radix-16 butterfly per thread");
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
+  const int lin = a.ax.lin, lout = a.ax.lout, nc = a.ncomp;
+  const bool rowok = row < a.rin;
+  // the input-plane grid is read only by the forms that use it
+  const bool ftab = K == PREK_F && a.ftab;
+  const bool grid = K == PREK_HNA || (K == PREK_F && !ftab) || a.ez_mode != EZ_NONE;
+  const uint32_t r0 = rowok ? row : 0, row_at = r0 * lin;
+  const double Y = grid ? a.py[r0] : 0.0;
+  float2 e[NC][H];
+  // PXG pixels at a time: their loads, then their pre-ops (columns beyond lin
+  // read the row's last pixel and are zeroed)
+  constexpr int PXG = 4;
+#pragma unroll
+  for (int r1 = 0; r1 < H; r1 += PXG) {
+    PixRaw raw[PXG];
+    uint32_t pix[PXG], cc[PXG];
+    float2 fr[PXG], pr[PXG];
+    double X[PXG];
+#pragma unroll
+    for (int u = 0; u < PXG; ++u) {
+      cc[u] = min(t + (r1 + u) * TPF, lin - 1);
+      pix[u] = row_at + cc[u];
+      fr[u] = make_float2(1.f, 0.f);
+      X[u] = 0.0;
+    }
+    pix_load_n<PXG>(a.in, a.in_cs, MULTI ? a.nin : 1, a.mask, pix, raw);
+    if (grid) {
+#pragma unroll
+      for (int u = 0; u < PXG; ++u) X[u] = at32(a.px, cc[u]);
+    }
+    if (ftab) {
+#pragma unroll
+      for (int u = 0; u < PXG; ++u) fr[u] = at32(a.ftab, pix[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < PXG; ++u) pr[u] = at32(a.ax.pre, cc[u]);
+#pragma unroll
+    for (int u = 0; u < PXG; ++u) {
+      const int r = r1 + u, col = t + r * TPF;
+      float2 v[3] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+      if (rowok && col < lin) {
+        float2 e0, e1, e2;
+        pix_masked(a.mask, raw[u], e0, e1, e2);
+        float2 fv = make_float2(1.f, 0.f);
+        if constexpr (K == PREK_F) fv = ftab ? fr[u] : czt_f_at(a, X[u], Y);
+        czt_pre_compute<K>(a, e0, e1, e2, X[u], Y, fv, v);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v[c] = c_mul(v[c], pr[u]);
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) e[c][r] = v[c];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // roundings end here (the first pass's sums take the products as they are)
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < H; ++r) asm volatile("" : "+v"(e[c][r].x), "+v"(e[c][r].y));
+  const uint32_t lane = (uint32_t)((t >> 2) * (a.rin4 >> 2) + (g >> 2)) * 16 + (g & 3) * 4 + (t & 3);
+  NoIO none;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    if (c >= nc) break;
+    typename HO::Type in, u;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) in.v[0][r] = r < H ? e[c][r < H ? r : 0] : make_float2(0.f, 0.f);
+    chain_io<Q, TPF, false, true, 0, SRC_REG, DST_REG, ZL, false>(s, t, none, none, in, u);
+#pragma unroll
+    for (int b = 0; b < HO::BPT; ++b)
+#pragma unroll
+      for (int q = 0; q < HO::R; ++q) u.v[b][q] = cmul(u.v[b][q], ld_at(a.ax.gf + HO::koff(b, q), t));
+    float2* dst = a.t + (int64_t)c * a.t_cs + (row0 >> 2) * 16 + (row0 & 3) * 4;
+    auto store = [&](int k, float2 v) {
+      if (rowok && t + k < lout) st_at(dst + (int64_t)(k >> 2) * (a.rin4 >> 2) * 16, lane, cmul(v, ld_at(a.ax.post + k, t)));
+    };
+    fft_inverse_from_regs<Q, TPF, DST_FN, ZL>(s, t, u, store);
+  }
+}
+
+// Column pass of the 3 * 2^k lengths.  Per block CPB output columns of the x
+// axis (one per thread group) of one component: the columns of the tiled
+// intermediate feed the first pass, the chirp spectrum is applied in
+// registers, and only the output window is stored with the output-plane
+// factor.  A 128 B tile line holds four columns: the CPB groups of a block
+// (and at CPB = 2 the neighbouring block, kept on the same XCD) share it.
 template <int Q> struct CztColsShape {
-  static constexpr int CPB = Q >= 3072 ? 2 : 4;   // columns per block (more blocks at 3072 and 4096)
+  static constexpr int CPB = Q >= 3072 ? 2 : 4;   // columns per block (more blocks at 3072)
   // At 3072 three blocks (52 KB of LDS, 6 waves each) fit a CU when a SIMD
   // holds 5 waves, i.e. at most 96 VGPRs; unbounded, the compiler takes 112.
   static constexpr int WAVES = Q == 3072 ? 5 : 1;
-  // Power-of-two lengths stage the tile loads and the output rows through
-  // LDS; the 3 * 2^k lengths read and write columns directly (staged, 3072
-  // no longer fits the 5-wave bound and measured slower).
-  static constexpr bool STAGE = (Q & (Q - 1)) == 0;
 };
 
-template <int Q, bool ZL>
+template <int Q>
 __global__ __launch_bounds__(CztColsShape<Q>::CPB * FftThreads<Q>::value)
 __attribute__((amdgpu_waves_per_eu(CztColsShape<Q>::WAVES))) void czt_cols_kernel(CztArgs a0) {
   const CztArgs a = czt_member(a0, blockIdx.z);
@@ -368,135 +466,144 @@ __attribute__((amdgpu_waves_per_eu(CztColsShape<Q>::WAVES))) void czt_cols_kerne
   const int lin = a.ay.lin, lout = a.ay.lout;
   const float2* src = a.t + (int64_t)c * a.t_cs;
   typename HO::Type u;
-  NoIO none;
-  constexpr int NT = CPB * TPF;
-  const int kx0 = og * CPB;
-  if constexpr (CztColsShape<Q>::STAGE) {
-    // The block's CPB columns lie in one 4-column tile group: they are staged
-    // into LDS with lane-contiguous loads (column fastest) and the first pass
-    // reads them from there.
-    // IT elements per thread, loaded U at a time before their products
-    constexpr int IT = (ZL ? Q / 2 : Q) / TPF, U = IT < 8 ? IT : 8;
-#pragma unroll
-    for (int i0 = 0; i0 < IT; i0 += U) {
-      float2 tv[U], pv[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int e = threadIdx.x + (i0 + u) * NT, r = e / CPB, g = e % CPB;
-        const bool ok = r < lin && kx0 + g < lout_x;
-        tv[u] = src[czt_tidx(a.rin4, ok ? r : 0, ok ? kx0 + g : kx0)];
-        pv[u] = a.ay.pre[ok ? r : 0];
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int e = threadIdx.x + (i0 + u) * NT, r = e / CPB, g = e % CPB;
-        const bool ok = r < lin && kx0 + g < lout_x;
-        lds[g * LS + lpad(r)] = ok ? cmul(tv[u], pv[u]) : make_float2(0.f, 0.f);
-      }
-    }
-    __syncthreads();
-    fft_forward_to_regs<Q, TPF, SRC_LDS, ZL>(s, t, none, u);
-  } else {
-    auto load = [&](int k0) -> float2 {
-      const int r = t + k0;
-      return (colok && r < lin) ? cmul(src[czt_tidx(a.rin4, r, kx)], a.ay.pre[r]) : make_float2(0.f, 0.f);
-    };
-    // (twiddle bases loaded at each pass: prefetched, they cost the 3 * 2^k
-    // forms their 5-wave bound)
-    fft_forward_to_regs<Q, TPF, SRC_FN, ZL, false>(s, t, load, u);
-  }
+  auto load = [&](int k0) -> float2 {
+    const int r = t + k0;
+    return (colok && r < lin) ? cmul(src[czt_tidx(a.rin4, r, kx)], a.ay.pre[r]) : make_float2(0.f, 0.f);
+  };
+  // (twiddle bases loaded at each pass: prefetched, they cost the 5-wave bound)
+  fft_forward_to_regs<Q, TPF, SRC_FN, false, false>(s, t, load, u);
 #pragma unroll
   for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
     for (int q = 0; q < HO::R; ++q) u.v[b][q] = cmul(u.v[b][q], a.ay.gf[HO::index(t, b, q)]);
   float2* oc = a.out + (int64_t)c * a.out_cs;
-  if constexpr (CztColsShape<Q>::STAGE) {
-    // Last pass into registers, the outputs transposed through LDS to
-    // [ky][column] and stored row by row (CPB consecutive columns per row).
-    using LP = LastPass<Q, TPF, false>;
-    typename LP::Type o;
-    chain_io<Q, TPF, true, false, 0, SRC_REG, DST_REG, false, ZL>(s, t, none, none, u, o);
-    __syncthreads();   // the last pass of other waves may still read LDS
-#pragma unroll
-    for (int b = 0; b < LP::BPT; ++b) {
-      if (!LP::valid(t, b)) continue;
-#pragma unroll
-      for (int q = 0; q < (ZL ? LP::R / 2 : LP::R); ++q) {
-        const int ky = LP::index(t, b, q);
-        if (ky < lout) lds[ky * CPB + f] = cmul(o.v[b][q], a.ay.post[ky]);
-      }
+  auto store = [&](int k0, float2 v) {
+    const int ky = t + k0;
+    if (colok && ky < lout) {
+      v = cmul(v, a.ay.post[ky]);
+      if (a.f0tab) v = c_mul(v, a.f0tab[(int64_t)ky * lout_x + kx]);
+      else if (a.post_mode != POST_NONE) v = c_mul(v, czt_post_factor(a, ky, kx));
+      oc[(int64_t)ky * lout_x + kx] = v;
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < lout * CPB; e += NT) {
-      const int ky = e / CPB, kx2 = kx0 + e % CPB;
-      if (kx2 < lout_x) {
-        float2 v = lds[e];
-        if (a.f0tab) v = c_mul(v, a.f0tab[(int64_t)ky * lout_x + kx2]);
-        else if (a.post_mode != POST_NONE) v = c_mul(v, czt_post_factor(a, ky, kx2));
-        oc[(int64_t)ky * lout_x + kx2] = v;
-      }
-    }
-  } else {
-    auto store = [&](int k0, float2 v) {
-      const int ky = t + k0;
-      if (colok && ky < lout) {
-        v = cmul(v, a.ay.post[ky]);
-        if (a.f0tab) v = c_mul(v, a.f0tab[(int64_t)ky * lout_x + kx]);
-        else if (a.post_mode != POST_NONE) v = c_mul(v, czt_post_factor(a, ky, kx));
-        oc[(int64_t)ky * lout_x + kx] = v;
-      }
-    };
-    fft_inverse_from_regs<Q, TPF, DST_FN, ZL, false>(s, t, u, store);
-  }
+  };
+  fft_inverse_from_regs<Q, TPF, DST_FN, false, false>(s, t, u, store);
 }
 
-// Zero-half forms exist for the power-of-two lengths.
-template <int Q> struct CztZl { static constexpr bool value = (Q & (Q - 1)) == 0; };
+// Column pass of the power-of-two lengths: G columns of one component per
+// block, Q/16 threads each, neighbouring lanes on the G columns: a wave reads
+// G/4 of each tile line it touches and stores G-column row segments, straight
+// from and to its registers.  (Staged through LDS by blocks of half the
+// threads per transform, 232 VGPRs at 4096: the adjoint 256^2 -> 2048^2, three
+// components, 109 us, now 78 us of which the accesses alone take 59; zoom
+// 2048 -> 512 columns 31 -> 23 us.  G = 1, 2, 4 at 4096: 83, 78, 88 us; at
+// 2048, 1024^2 -> 400^2: 13.5, 13.3, 16.8 us.)
+template <int Q> using CztCols1 = Units<Q, rs_g(Q, 2, 2, 2)>;
 
 template <int Q, bool ZL>
+__global__ __launch_bounds__(CztCols1<Q>::NT, 4) void czt_cols1_kernel(CztArgs a0) {
+  const CztArgs a = czt_member(a0, blockIdx.z);
+  using U = CztCols1<Q>;
+  constexpr int TPF = U::TPF;
+  using HO = HandOff<Q, TPF>;
+  using LP = LastPass<Q, TPF, false>;
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::col_g(threadIdx.x), t = U::col_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int kx0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, kx = kx0 + g, c = blockIdx.y;
+  const int lout_x = a.ax.lout, lin = a.ay.lin, lout = a.ay.lout;
+  const bool colok = kx < lout_x;
+  const float2* src = a.t + (int64_t)c * a.t_cs + (int64_t)(kx0 >> 2) * (a.rin4 >> 2) * 16 + (kx0 & 3);
+  const uint32_t lane = (g >> 2) * (a.rin4 >> 2) * 16 + (g & 3) + 4 * t;
+  auto load = [&](int k) -> float2 {
+    return (colok && t + k < lin) ? cmul(ld_at(src + 4 * k, lane), ld_at(a.ay.pre + k, t)) : make_float2(0.f, 0.f);
+  };
+  typename HO::Type in, u;
+  NoIO none;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    in.v[0][r] = (ZL && r >= 8) ? make_float2(0.f, 0.f) : load(r * TPF);
+    if (!ZL || r < 8) asm volatile("" : "+v"(in.v[0][r].x), "+v"(in.v[0][r].y));
+  }
+  chain_io<Q, TPF, false, true, 0, SRC_REG, DST_REG, ZL, false>(s, t, none, none, in, u);
+#pragma unroll
+  for (int b = 0; b < HO::BPT; ++b)
+#pragma unroll
+    for (int q = 0; q < HO::R; ++q) u.v[b][q] = cmul(u.v[b][q], ld_at(a.ay.gf + HO::koff(b, q), t));
+  typename LP::Type o;
+  chain_io<Q, TPF, true, false, 0, SRC_REG, DST_REG, false, ZL>(s, t, none, none, u, o);
+  float2* oc = a.out + (int64_t)c * a.out_cs + kx0;
+  const uint32_t olane = (uint32_t)t * lout_x + g;
+#pragma unroll
+  for (int b = 0; b < LP::BPT; ++b)
+#pragma unroll
+    for (int q = 0; q < (ZL ? LP::R / 2 : LP::R); ++q) {
+      const int k = LP::index(0, b, q), ky = t + k;
+      if (!colok || ky >= lout) continue;
+      float2 v = cmul(o.v[b][q], ld_at(a.ay.post + k, t));
+      asm volatile("" : "+v"(v.x), "+v"(v.y));
+      if (a.f0tab) v = c_mul(v, ld_at(a.f0tab + (int64_t)k * lout_x + kx0, olane));
+      else if (a.post_mode != POST_NONE) v = c_mul(v, czt_post_factor(a, ky, kx));
+      st_at(oc + (int64_t)k * lout_x, olane, v);
+    }
+}
+
+// Power-of-two lengths (the 3 * 2^k ones serve the column pass only).
+template <int Q> struct CztPow2 { static constexpr bool value = (Q & (Q - 1)) == 0; };
+
+// The one-buffer form for one component and for the 4096-point zero-half
+// rows, the three-buffer form otherwise (see czt_rows1_kernel).
+template <int Q, int K, bool ZL>
+inline void czt_rows_launch_k(const CztArgs& a, int batch, hipStream_t st) {
+  using U1 = CztRows1<Q>;
+  const dim3 g1((a.rin + U1::G - 1) / U1::G, batch), b1(U1::NT);
+  if constexpr (K != PREK_HNA)
+    if (a.ncomp == 1) {
+      hipLaunchKernelGGL((czt_rows1_kernel<Q, K, ZL, false>), g1, b1, 0, st, a);
+      return;
+    }
+  if constexpr (ZL && Q >= 4096) {
+    hipLaunchKernelGGL((czt_rows1_kernel<Q, K, ZL, true>), g1, b1, 0, st, a);
+  } else {
+    const dim3 g(a.rin, batch), b(a.ncomp * Q / 16);
+    const size_t lds = (size_t)a.ncomp * LdsLen<Q>::value * sizeof(float2);
+    hipLaunchKernelGGL((czt_rows_kernel<Q, K, ZL>), g, b, lds, st, a);
+  }
+}
+template <int Q, bool ZL>
 inline void czt_rows_launch_zl(const CztArgs& a, int batch, hipStream_t st) {
-  const dim3 g(a.rin, batch), b(a.ncomp * Q / 16);
-  const size_t lds = (size_t)a.ncomp * LdsLen<Q>::value * sizeof(float2);
-  if (a.pre_mode == PRE_RS || a.pre_mode == PRE_CONJ_RS)
-    hipLaunchKernelGGL((czt_rows_kernel<Q, PREK_F, ZL>), g, b, lds, st, a);
-  else if (a.pre_mode == PRE_HNA)
-    hipLaunchKernelGGL((czt_rows_kernel<Q, PREK_HNA, ZL>), g, b, lds, st, a);
-  else
-    hipLaunchKernelGGL((czt_rows_kernel<Q, PREK_SIMPLE, ZL>), g, b, lds, st, a);
+  if (a.pre_mode == PRE_RS || a.pre_mode == PRE_CONJ_RS) czt_rows_launch_k<Q, PREK_F, ZL>(a, batch, st);
+  else if (a.pre_mode == PRE_HNA) czt_rows_launch_k<Q, PREK_HNA, ZL>(a, batch, st);
+  else czt_rows_launch_k<Q, PREK_SIMPLE, ZL>(a, batch, st);
 }
 template <int Q>
 inline void czt_rows_launch(const CztArgs& a, int batch, hipStream_t st) {
-  KTimer t(K_CZT_ROWS, st);
-  if constexpr (CztZl<Q>::value)
-    if (a.ax.zl) return czt_rows_launch_zl<Q, true>(a, batch, st);
-  czt_rows_launch_zl<Q, false>(a, batch, st);
+  KTimer t(K_CZT_ROWS, st);   // (the x axis has a power-of-two length)
+  if (a.ax.zl) czt_rows_launch_zl<Q, true>(a, batch, st);
+  else czt_rows_launch_zl<Q, false>(a, batch, st);
 }
-// Dynamic-LDS limit of the row kernel (three Q-point buffers), set once per
-// device by the library's initialisation for every Bluestein length.
+// Dynamic-LDS limit of the three-buffer row kernel, set once per device by
+// the library's initialisation for every length it runs at.
 template <int Q, bool ZL> inline hipError_t czt_set_attribute_zl() {
-  const int mx = 3 * LdsLen<Q>::value * (int)sizeof(float2);
   hipError_t e = hipSuccess;
-  for (const void* f : {(const void*)czt_rows_kernel<Q, PREK_F, ZL>, (const void*)czt_rows_kernel<Q, PREK_HNA, ZL>,
-                        (const void*)czt_rows_kernel<Q, PREK_SIMPLE, ZL>}) {
-    const hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, mx);
-    if (r != hipSuccess) e = r;
+  if constexpr (!(ZL && Q >= 4096)) {
+    const int mx = 3 * LdsLen<Q>::value * (int)sizeof(float2);
+    for (const void* f : {(const void*)czt_rows_kernel<Q, PREK_F, ZL>, (const void*)czt_rows_kernel<Q, PREK_HNA, ZL>,
+                          (const void*)czt_rows_kernel<Q, PREK_SIMPLE, ZL>}) {
+      const hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, mx);
+      if (r != hipSuccess) e = r;
+    }
   }
   return e;
 }
 template <int Q> inline hipError_t czt_set_attribute() {
-  hipError_t e = czt_set_attribute_zl<Q, false>();
-  if constexpr (CztZl<Q>::value) {
-    const hipError_t r = czt_set_attribute_zl<Q, true>();
-    if (r != hipSuccess) e = r;
-  }
-  return e;
+  const hipError_t e = czt_set_attribute_zl<Q, false>(), r = czt_set_attribute_zl<Q, true>();
+  return e != hipSuccess ? e : r;
 }
 inline hipError_t czt_set_attributes() {
   hipError_t e = hipSuccess;
   for (hipError_t r : {czt_set_attribute<64>(), czt_set_attribute<128>(), czt_set_attribute<256>(),
                        czt_set_attribute<512>(), czt_set_attribute<1024>(), czt_set_attribute<2048>(),
-                       czt_set_attribute<4096>(), czt_set_attribute<768>(), czt_set_attribute<1536>(),
-                       czt_set_attribute<3072>()})
+                       czt_set_attribute<4096>()})
     if (r != hipSuccess) e = r;
   return e;
 }
@@ -504,14 +611,16 @@ inline hipError_t czt_set_attributes() {
 template <int Q>
 inline void czt_cols_launch(const CztArgs& a, int batch, hipStream_t st) {
   KTimer t(K_CZT_COLS, st);
-  constexpr int CPB = CztColsShape<Q>::CPB;
-  const dim3 g((a.ax.lout + CPB - 1) / CPB, a.ncomp, batch), b(CPB * FftThreads<Q>::value);
-  if constexpr (CztZl<Q>::value)
-    if (a.ay.zl) {
-      hipLaunchKernelGGL((czt_cols_kernel<Q, true>), g, b, 0, st, a);
-      return;
-    }
-  hipLaunchKernelGGL((czt_cols_kernel<Q, false>), g, b, 0, st, a);
+  if constexpr (CztPow2<Q>::value) {
+    using U = CztCols1<Q>;
+    const dim3 g((a.ax.lout + U::G - 1) / U::G, a.ncomp, batch);
+    if (a.ay.zl) hipLaunchKernelGGL((czt_cols1_kernel<Q, true>), g, dim3(U::NT), 0, st, a);
+    else hipLaunchKernelGGL((czt_cols1_kernel<Q, false>), g, dim3(U::NT), 0, st, a);
+  } else {
+    constexpr int CPB = CztColsShape<Q>::CPB;
+    const dim3 g((a.ax.lout + CPB - 1) / CPB, a.ncomp, batch), b(CPB * FftThreads<Q>::value);
+    hipLaunchKernelGGL(czt_cols_kernel<Q>, g, b, 0, st, a);
+  }
 }
 template <int Q>
 inline void czt_setup_launch(const CztSetupPair& p, int nblocks, hipStream_t st) {

@@ -583,7 +583,7 @@ int xl_czt(const xl_czt_params* p, void* ws, size_t ws_bytes, void* stream) {
   a.rin4 = (cp.rin + 3) / 4 * 4;
   a.t_cs = (int64_t)a.rin4 * ((cp.lout_x + 3) / 4 * 4);
   a.t_bs = (int64_t)cp.ncomp * a.t_cs;
-  if (int rc = dispatch_czt_q(a.ax.q, [&](auto c) { xl::czt_rows_launch<decltype(c)::value>(a, batch, st); }))
+  if (int rc = dispatch_q(a.ax.q, [&](auto c) { xl::czt_rows_launch<decltype(c)::value>(a, batch, st); }))
     return rc;
   if (int rc = dispatch_czt_q(a.ay.q, [&](auto c) { xl::czt_cols_launch<decltype(c)::value>(a, batch, st); }))
     return rc;

@@ -478,7 +478,8 @@ def czt(src: torch.Tensor, geom: ops.CztGeometry, masks: Sequence[MaskSpec] = ()
     mode = geom.mode if mode is None else mode
     if wavelength is not None and abs(float(wavelength.detach().reshape(-1)[0]) - geom.wavelength) > 1e-12 * geom.wavelength:
         raise ValueError("the wavelength tensor must hold the geometry's wavelength")
-    cfg = CZTConfig(geom, ez_mode, nin, mode, _mask_structure(masks), ops.resolve_czt_form(geom, form))
+    ncomp = 3 if ez_mode == N.XL_EZ_VCZT or mode == N.XL_CZT_HNA else nin
+    cfg = CZTConfig(geom, ez_mode, nin, mode, _mask_structure(masks), ops.resolve_czt_form(geom, form, ncomp))
     return _CZTFunction.apply(cfg, src, *_flat_params(masks), z, wavelength)
 
 

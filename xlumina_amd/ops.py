@@ -619,9 +619,18 @@ def _czt_params(g: CztGeometry, dev, ncomp, nin, adjoint, ez_mode, mode=None):
 
 CZT_FORMS = ("auto", "bluestein", "gemm")
 _czt_form = "auto"
-# Output-window size (per axis) below which "auto" picks the split-BF16 MFMA
-# zoom-DFT over the FP32 Bluestein FFT form (measured on MI355X; see bench.py).
+# Where "auto" picks the split-BF16 MFMA zoom-DFT over the FP32 Bluestein FFT
+# form.  RS-mode transforms of several components, measured on MI355X (us,
+# forward + adjoint of three components, Bluestein / GEMM): 2048^2 -> 96^2 240 /
+# 214, 128^2 241 / 231, 160^2 243 / 270; 1500^2 -> 64^2 142 / 150, 128^2 143 /
+# 180; 1024^2 -> 96^2 94 / 116; 256^2 -> 96^2 52 / 85.  One component: 2048^2 ->
+# 96^2 forward 56 / 86.  So the GEMM form is left where an input side exceeds
+# GEMM_MIN_SIDE and the window fits GEMM_RS_WINDOW.  High-NA transforms keep
+# their own line, GEMM_CROSSOVER: the gradients of float64 masks behind them
+# stay what they were to the last bit (1024^2 -> 96^2 88 / 109 us).
 GEMM_CROSSOVER = 160
+GEMM_RS_WINDOW = 128
+GEMM_MIN_SIDE = 1536
 
 
 def set_czt_form(form: str) -> None:
@@ -637,10 +646,15 @@ def get_czt_form() -> str:
     return _czt_form
 
 
-def resolve_czt_form(g: "CztGeometry", form: Optional[str] = None) -> str:
+def resolve_czt_form(g: "CztGeometry", form: Optional[str] = None, ncomp: int = 3) -> str:
+    """The implementation of a transform of geometry g: `form` (default the
+    module setting), with 'auto' resolved by the sizes."""
     form = form or _czt_form
     if form == "auto":
-        small = max(len(g.xout), len(g.yout)) <= GEMM_CROSSOVER
+        window = max(len(g.xout), len(g.yout))
+        if g.mode == N.XL_CZT_HNA:
+            return "gemm" if window <= GEMM_CROSSOVER else "bluestein"
+        small = window <= GEMM_RS_WINDOW and ncomp > 1 and max(len(g.x), len(g.y)) > GEMM_MIN_SIDE
         return "gemm" if small else "bluestein"
     return form
 
@@ -683,7 +697,7 @@ def czt(src: torch.Tensor, g: CztGeometry, masks: Sequence[MaskSpec] = (), ez_mo
     p.out = out.data_ptr()
     p.out_comp_stride = rows_out * cols_out
     keep += fill_masks(p.mask, masks, (rows_in, cols_in), dev, nin)
-    use_gemm = resolve_czt_form(g, form) == "gemm"
+    use_gemm = resolve_czt_form(g, form, ncomp) == "gemm"
     wsfn = lib.xl_czt_gemm_workspace_bytes if use_gemm else lib.xl_czt_workspace_bytes
     runfn = lib.xl_czt_gemm if use_gemm else lib.xl_czt
     need = wsfn(C.byref(p))

@@ -17,7 +17,7 @@ from xlumina_amd.ops import MaskSpec
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
 
-SIZES = [2, 5, 31, 33, 63, 66, 127, 130, 255, 258, 511, 514, 1023, 1026]
+SIZES = [2, 5, 31, 33, 63, 66, 127, 130, 255, 258, 511, 513, 514, 640, 641, 768, 769, 1023, 1026, 1280, 1281, 1536]
 
 
 @pytest.mark.parametrize("n", SIZES)
@@ -44,6 +44,26 @@ def test_block_edges_vs_oracle(cuda_dev, n):
     rhs = torch.sum(hg.to(torch.complex128).conj() * f.to(torch.complex128))
     scale = float(torch.linalg.vector_norm(g) * torch.linalg.vector_norm(af))
     assert abs(complex(lhs - rhs)) <= 1e-5 * scale
+
+
+@pytest.mark.parametrize("n", [513, 700, 1100, 1300])
+def test_plain_and_kept_spectra_agree(cuda_dev, n):
+    """A plain call runs at the shortest length, one that keeps its kernel
+    spectrum at the power of two: the same propagation to rounding (each within
+    1e-6 of float64, so 2e-6 apart at most), with float64 and one-value mask
+    parameters and masks in both stages."""
+    rng = np.random.default_rng(n)
+    x, y = R.space(1.17 * n, n)
+    f = rng.standard_normal((3, n, n)) + 1j * rng.standard_normal((3, n, n))
+    src = torch.tensor(f.astype(np.complex64), device=cuda_dev)
+    p = torch.tensor(rng.uniform(0, 1, (2, n, n)), dtype=torch.float64, device=cuda_dev)
+    v = torch.tensor([0.3], dtype=torch.float64, device=cuda_dev)
+    masks = [MaskSpec(N.XL_MASK_SSLM, p[0], p[1], unit=3), MaskSpec(N.XL_MASK_LCD, v, v)]
+    hh = torch.empty(ops.rs_hhat_bytes(n), dtype=torch.uint8, device=cuda_dev)
+    for kw in (dict(masks=masks, ez_mode=N.XL_EZ_VRS, nin=2), dict(masks=masks, nin=3), dict(nin=3, adjoint=True, masks=())):
+        a = ops.rs_propagate(src, x, y, 4e4, 0.65, **kw)
+        b = ops.rs_propagate(src, x, y, 4e4, 0.65, hhat=hh, hhat_mode=1, **kw)
+        assert rel_l2(a.cpu().numpy(), b.cpu().numpy()) < 2e-6
 
 
 @pytest.mark.parametrize("n", [31, 130, 514])

@@ -351,7 +351,7 @@ __global__ __launch_bounds__(CztRows1<Q>::NT, MULTI ? 3 : 4) void czt_rows1_kern
   using U = CztRows1<Q>;
   constexpr int TPF = U::TPF, H = ZL ? 8 : 16, NC = MULTI ? 3 : 1;
   using HO = HandOff<Q, TPF>;
-  static_assert(FftPlan<Q>::radix(true, 0) == 16, "first pass: one radix-16 butterfly per thread");
+  static_assert(FftPlan<Q, TPF>::radix(true, 0) == 16, "first pass: one radix-16 butterfly per thread");
   __shared__ float2 lds[U::G * U::LS];
   const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
   float2* s = lds + g * U::LS;
@@ -419,7 +419,8 @@ __global__ __launch_bounds__(CztRows1<Q>::NT, MULTI ? 3 : 4) void czt_rows1_kern
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     if (c >= nc) break;
-    typename HO::Type in, u;
+    Regs<1, 16> in;
+    typename HO::Type u;
 #pragma unroll
     for (int r = 0; r < 16; ++r) in.v[0][r] = r < H ? e[c][r < H ? r : 0] : make_float2(0.f, 0.f);
     chain_io<Q, TPF, false, true, 0, SRC_REG, DST_REG, ZL, false>(s, t, none, none, in, u);
@@ -517,7 +518,8 @@ __global__ __launch_bounds__(CztCols1<Q>::NT, 4) void czt_cols1_kernel(CztArgs a
   auto load = [&](int k) -> float2 {
     return (colok && t + k < lin) ? cmul(ld_at(src + 4 * k, lane), ld_at(a.ay.pre + k, t)) : make_float2(0.f, 0.f);
   };
-  typename HO::Type in, u;
+  Regs<1, 16> in;
+  typename HO::Type u;
   NoIO none;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {

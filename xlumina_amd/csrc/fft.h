@@ -19,10 +19,12 @@ namespace xl {
 
 constexpr int TWN = 4096;                 // twiddle table length == max FFT length
 constexpr int TWN3 = 3072;                // table for the lengths 3 * 2^k
+constexpr int TWN5 = 2560;                // table for the lengths 5 * 2^k
 constexpr int MAX_FFT = 4096;
 
 __device__ float2 g_tw[TWN];              // e^{-2 pi i k / TWN}, float64-generated
 __device__ float2 g_tw3[TWN3];            // e^{-2 pi i k / TWN3}, float64-generated
+__device__ float2 g_tw5[TWN5];            // e^{-2 pi i k / TWN5}, float64-generated
 
 __global__ void xl_fft_init_kernel() {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -36,29 +38,46 @@ __global__ void xl_fft_init_kernel() {
     sincospi(-2.0 * (double)k / (double)TWN3, &s, &c);
     g_tw3[k] = make_float2((float)c, (float)s);
   }
+  if (k < TWN5) {
+    double s, c;
+    sincospi(-2.0 * (double)k / (double)TWN5, &s, &c);
+    g_tw5[k] = make_float2((float)c, (float)s);
+  }
 }
 
-// Lengths are 2^k (64..4096) or 3 * 2^k (768..3072); the latter start with one
-// radix-3 pass and take their twiddles from the 3072-entry table.
+// Lengths are 2^k (64..4096), 3 * 2^k (768..3072) and 5 * 2^k (1280, 2560);
+// the latter two take their twiddles from tables of their own.
 template <int L> struct Tw {
-  static constexpr bool TRI = L % 3 == 0;
-  static constexpr int N = TRI ? TWN3 : TWN;
-  __device__ static float2 at(int i) { return TRI ? g_tw3[i] : g_tw[i]; }
+  static constexpr bool TRI = L % 3 == 0, PENT = L % 5 == 0;
+  static constexpr int N = TRI ? TWN3 : PENT ? TWN5 : TWN;
+  __device__ static float2 at(int i) { return TRI ? g_tw3[i] : PENT ? g_tw5[i] : g_tw[i]; }
 };
 
 constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x / 2); }
 
-// Pass sequence of an L-point FFT: forward [3,] 16, ..., 16, REM; the inverse
-// runs the same radices in reverse order, so the last forward pass and the
-// first inverse pass share one register layout.
-template <int L> struct FftPlan {
-  static constexpr bool TRI = L % 3 == 0;
+// Pass sequence of an L-point FFT on TPF threads; the inverse runs the same
+// radices in reverse order, so the last forward pass and the first inverse
+// pass share one register layout.
+//   2^k                               16, ..., 16, REM
+//   3072, 1536 with TPF = L/12        12, 16 or 8, 16
+//   2560, 1280 (TPF = L/10)           10, 16 or 8, 16
+//   3 * 2^k otherwise (TPF = L/16)    3, 16, ..., 16, REM
+// All but the last kind split a zero upper half of the inputs, or a cropped
+// upper half of the outputs, evenly in their first and last passes.  (The odd
+// radix last at 2560 and 3072, on L/16 threads: rs_final of VRS 1200^2 21 -> 35
+// us, the rest equal.)
+template <int L, int TPF> struct FftPlan {
+  static constexpr bool TRI = L % 3 == 0, PENT = L % 5 == 0;
+  static constexpr bool MIXED = PENT || (TRI && TPF * 12 == L);
+  static constexpr bool EVEN = !TRI || MIXED;
+  static constexpr int ODD = TRI ? 12 : 10;
   static constexpr int L2 = TRI ? L / 3 : L;
   static constexpr int LG = ilog2c(L2);
   static constexpr int N16 = LG / 4;
   static constexpr int REM = 1 << (LG % 4);
-  static constexpr int NP = (TRI ? 1 : 0) + N16 + (REM > 1 ? 1 : 0);
+  static constexpr int NP = MIXED ? 3 : (TRI ? 1 : 0) + N16 + (REM > 1 ? 1 : 0);
   static constexpr int fwd_radix(int i) {
+    if (MIXED) return i == 0 ? ODD : i == 2 ? 16 : L / (ODD * 16);
     if (TRI) {
       if (i == 0) return 3;
       i -= 1;
@@ -178,15 +197,121 @@ template <bool INV> struct DFT<3, INV> {
   }
 };
 
+// Radix 5 (Winograd's sums, cos / sin of 72 and 144 degrees).
+template <bool INV> struct DFT<5, INV> {
+  __device__ __forceinline__ static void run(float2* v) {
+    const float c1 = 0.30901699437494742f, c2 = -0.80901699437494742f;
+    const float s1 = 0.95105651629515357f, s2 = 0.58778525229247313f;
+    const float2 a = v[0], t1 = v[1] + v[4], t2 = v[2] + v[3], t3 = v[1] - v[4], t4 = v[2] - v[3];
+    const float2 m1 = a + t1 * c1 + t2 * c2, m2 = a + t1 * c2 + t2 * c1;
+    const float2 n1 = t3 * s1 + t4 * s2, n2 = t3 * s2 - t4 * s1;
+    const float2 j1 = make_float2(-n1.y, n1.x), j2 = make_float2(-n2.y, n2.x);   // i n
+    v[0] = a + t1 + t2;
+    v[1] = INV ? m1 + j1 : m1 - j1;
+    v[4] = INV ? m1 - j1 : m1 + j1;
+    v[2] = INV ? m2 + j2 : m2 - j2;
+    v[3] = INV ? m2 - j2 : m2 + j2;
+  }
+};
+
+// cos / sin of 2 pi q / R for the even radices 6, 10 and 12, q < R / 2.
+template <int R> struct Rot;
+template <> struct Rot<6> {
+  __device__ static constexpr float c(int q) { constexpr float t[3] = {1.f, 0.5f, -0.5f}; return t[q]; }
+  __device__ static constexpr float s(int q) {
+    constexpr float t[3] = {0.f, 0.86602540378443865f, 0.86602540378443865f};
+    return t[q];
+  }
+};
+template <> struct Rot<10> {
+  __device__ static constexpr float c(int q) {
+    constexpr float t[5] = {1.f, 0.80901699437494742f, 0.30901699437494742f, -0.30901699437494742f, -0.80901699437494742f};
+    return t[q];
+  }
+  __device__ static constexpr float s(int q) {
+    constexpr float t[5] = {0.f, 0.58778525229247313f, 0.95105651629515357f, 0.95105651629515357f, 0.58778525229247313f};
+    return t[q];
+  }
+};
+template <> struct Rot<12> {
+  __device__ static constexpr float c(int q) {
+    constexpr float t[6] = {1.f, 0.86602540378443865f, 0.5f, 0.f, -0.5f, -0.86602540378443865f};
+    return t[q];
+  }
+  __device__ static constexpr float s(int q) {
+    constexpr float t[6] = {0.f, 0.5f, 0.86602540378443865f, 1.f, 0.86602540378443865f, 0.5f};
+    return t[q];
+  }
+};
+// v e^{-+ 2 pi i q / R}, q a constant after unrolling
+template <int R, bool INV> __device__ __forceinline__ float2 rot_r(float2 v, int q) {
+  if (q == 0) return v;
+  if (4 * q == R) return INV ? make_float2(-v.y, v.x) : make_float2(v.y, -v.x);
+  const float c = Rot<R>::c(q), s = INV ? Rot<R>::s(q) : -Rot<R>::s(q);
+  return make_float2(v.x * c - v.y * s, v.x * s + v.y * c);
+}
+
+// DFT of R = 2 M points (R = 6, 10, 12) from two of M, even and odd inputs.
+template <int R, bool INV, bool LOW> __device__ __forceinline__ void dft_even(float2* v) {
+  constexpr int M = R / 2;
+  float2 e[M], o[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) { e[i] = v[2 * i]; o[i] = v[2 * i + 1]; }
+  DFT<M, INV>::run(e);
+  DFT<M, INV>::run(o);
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    const float2 t = rot_r<R, INV>(o[k], k);
+    v[k] = e[k] + t;
+    if (!LOW) v[k + M] = e[k] - t;
+  }
+}
+template <bool INV> struct DFT<6, INV> { __device__ __forceinline__ static void run(float2* v) { dft_even<6, INV, false>(v); } };
+template <bool INV> struct DFT<10, INV> { __device__ __forceinline__ static void run(float2* v) { dft_even<10, INV, false>(v); } };
+template <bool INV> struct DFT<12, INV> { __device__ __forceinline__ static void run(float2* v) { dft_even<12, INV, false>(v); } };
+template <bool INV> struct DFTLow<10, INV> { __device__ __forceinline__ static void run(float2* v) { dft_even<10, INV, true>(v); } };
+template <bool INV> struct DFTLow<12, INV> { __device__ __forceinline__ static void run(float2* v) { dft_even<12, INV, true>(v); } };
+// Upper half zero: even outputs are the DFT of the M inputs, odd outputs that
+// of the inputs turned by w^r.
+template <int R, bool INV> __device__ __forceinline__ void dft_half_even(float2* v) {
+  constexpr int M = R / 2;
+  float2 e[M], o[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) { e[i] = v[i]; o[i] = rot_r<R, INV>(v[i], i); }
+  DFT<M, INV>::run(e);
+  DFT<M, INV>::run(o);
+#pragma unroll
+  for (int i = 0; i < M; ++i) { v[2 * i] = e[i]; v[2 * i + 1] = o[i]; }
+}
+template <bool INV> struct DFTHalf<10, INV> { __device__ __forceinline__ static void run(float2* v) { dft_half_even<10, INV>(v); } };
+template <bool INV> struct DFTHalf<12, INV> { __device__ __forceinline__ static void run(float2* v) { dft_half_even<12, INV>(v); } };
+
 // v[r] *= w^r for r < R (w1 = w, e^{-+2 pi i base / TWN}, one table entry);
 // w^2, w^4, w^8 by squaring and the other powers as products formed next to
 // their use, so that only the four bases stay live.  Loads cost more than the
 // products here (each is a scattered L1 access per lane); the squarings add
-// at most a few float32 ulps to w^8.
-template <int R, bool INV> __device__ __forceinline__ void apply_twiddles_w(float2* v, const float2 w1) {
+// at most a few float32 ulps to w^8.  T4 (the mixed-radix plans): w^4 is a table
+// entry too (wt4), which halves the error of the upper powers.
+template <int R, bool INV, bool T4 = false>
+__device__ __forceinline__ void apply_twiddles_w(float2* v, const float2 w1, const float2 wt4 = float2()) {
   if constexpr (R == 3) {
     v[1] = twmul<INV>(v[1], w1);
     v[2] = twmul<INV>(v[2], cmul(w1, w1));
+  } else if constexpr (R == 10 || R == 12) {
+    const float2 w2 = cmul(w1, w1), w3 = cmul(w1, w2), w8 = cmul(wt4, wt4);
+    v[1] = twmul<INV>(v[1], w1);
+    v[2] = twmul<INV>(v[2], w2);
+    v[3] = twmul<INV>(v[3], w3);
+    v[4] = twmul<INV>(v[4], wt4);
+    v[5] = twmul<INV>(v[5], cmul(w1, wt4));
+    v[6] = twmul<INV>(v[6], cmul(w2, wt4));
+    v[7] = twmul<INV>(v[7], cmul(w3, wt4));
+    v[8] = twmul<INV>(v[8], w8);
+    v[9] = twmul<INV>(v[9], cmul(w1, w8));
+    if constexpr (R == 12) {
+      v[10] = twmul<INV>(v[10], cmul(w2, w8));
+      v[11] = twmul<INV>(v[11], cmul(w3, w8));
+    }
   } else if constexpr (R >= 2) {
     v[1] = twmul<INV>(v[1], w1);
     if constexpr (R >= 4) {
@@ -195,7 +320,7 @@ template <int R, bool INV> __device__ __forceinline__ void apply_twiddles_w(floa
       const float2 w3 = cmul(w1, w2);
       v[3] = twmul<INV>(v[3], w3);
       if constexpr (R >= 8) {
-        const float2 w4 = cmul(w2, w2);
+        const float2 w4 = T4 ? wt4 : cmul(w2, w2);
         v[4] = twmul<INV>(v[4], w4);
         v[5] = twmul<INV>(v[5], cmul(w1, w4));
         v[6] = twmul<INV>(v[6], cmul(w2, w4));
@@ -218,6 +343,7 @@ template <int R, bool INV> __device__ __forceinline__ void apply_twiddles_w(floa
 }
 
 template <int R, bool INV, int L> __device__ __forceinline__ void apply_twiddles(float2* v, int base) {
+  static_assert(R != 10 && R != 12, "the mixed-radix plans load their bases ahead (TwSet)");
   apply_twiddles_w<R, INV>(v, Tw<L>::at(base));
 }
 
@@ -255,7 +381,7 @@ __device__ __forceinline__ void stockham_pass(float2* s, int t) {
 
 template <int L, int TPF, bool INV, int I = 0, bool GUARD = false>
 __device__ __forceinline__ void fft_lds(float2* s, int t) {
-  using PL = FftPlan<L>;
+  using PL = FftPlan<L, TPF>;
   if constexpr (I < PL::NP) {
     stockham_pass<L, PL::radix(true, I), PL::ns(true, I), TPF, INV, GUARD>(s, t);
     fft_lds<L, TPF, INV, I + 1, GUARD>(s, t);

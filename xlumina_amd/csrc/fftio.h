@@ -32,10 +32,10 @@ enum { DST_LDS = 0, DST_FN = 1, DST_REG = 2 };
 // half: indices >= L/2); they are neither loaded nor transformed.  LOW: only
 // the outputs r < R/2 are formed and written (a last pass whose indices
 // >= L/2 are cropped away).
-// wb: the pass's twiddle bases, one per butterfly slot b, when PREW (loaded
-// ahead by the caller); otherwise the pass loads them itself (NS > 1).
+// wb: the pass's twiddle bases, PB (w, or w and w^4) per butterfly slot b, when
+// PREW (loaded ahead by the caller); otherwise the pass loads them itself (NS > 1).
 template <int L, int R, int NS, int TPF, bool INV, int SRC, int DST, bool ZHI = false, bool LOW = false,
-          bool PREW = true, class Load, class Store, class RegT>
+          bool PREW = true, int PB = 1, class Load, class Store, class RegT>
 __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& store, RegT& reg, const float2* wb) {
   constexpr int NB = L / R;
   constexpr int BPT = (NB + TPF - 1) / TPF;
@@ -55,7 +55,8 @@ __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& sto
         else v[b][r] = reg.v[b][r];
       }
       if constexpr (NS > 1) {
-        if constexpr (PREW) apply_twiddles_w<R, INV>(v[b], wb[b]);
+        if constexpr (PREW && PB == 2) apply_twiddles_w<R, INV, true>(v[b], wb[2 * b], wb[2 * b + 1]);
+        else if constexpr (PREW) apply_twiddles_w<R, INV>(v[b], wb[b]);
         else apply_twiddles<R, INV, L>(v[b], (j % NS) * (Tw<L>::N / (NS * R)));
       }
       if constexpr (ZHI) DFTHalf<R, INV>::run(v[b]);
@@ -90,11 +91,13 @@ struct NoIO {
 // butterfly slot b of thread t), loaded together when the chain starts: a
 // pass's twiddles then need no memory access behind its barrier.
 template <int L, int TPF, bool FWD> struct TwSet {
-  using P = FftPlan<L>;
+  using P = FftPlan<L, TPF>;
   static constexpr int bpt(int I) { return (L / P::radix(FWD, I) + TPF - 1) / TPF; }
+  // bases per butterfly: w, and w^4 where a mixed-radix pass uses it
+  static constexpr int per(int I) { return P::MIXED && P::radix(FWD, I) >= 8 ? 2 : 1; }
   static constexpr int off(int I) {
     int o = 0;
-    for (int k = 1; k < I; ++k) o += bpt(k);
+    for (int k = 1; k < I; ++k) o += per(k) * bpt(k);
     return o;
   }
   static constexpr int N = off(P::NP) > 0 ? off(P::NP) : 1;
@@ -105,7 +108,10 @@ template <int L, int TPF, bool FWD> struct TwSet {
 #pragma unroll
       for (int b = 0; b < bpt(I); ++b) {
         const int j = t + b * TPF;
-        w[off(I) + b] = (NB % TPF == 0 || j < NB) ? Tw<L>::at((j % NS) * (Tw<L>::N / (NS * R))) : make_float2(1.f, 0.f);
+        const bool ok = NB % TPF == 0 || j < NB;
+        const int base = ok ? (j % NS) * (Tw<L>::N / (NS * R)) : 0;
+        w[off(I) + per(I) * b] = ok ? Tw<L>::at(base) : make_float2(1.f, 0.f);
+        if constexpr (per(I) == 2) w[off(I) + 2 * b + 1] = Tw<L>::at(4 * base);
       }
       load<I + 1>(t);
     }
@@ -124,24 +130,25 @@ template <int L, int TPF, bool INV, bool FWD, int I, int SRC, int DST, bool ZHI,
           class Store, class RegIn, class RegOut, class Hook>
 __device__ __forceinline__ void chain_pass(float2* s, int t, Load& load, Store& store, RegIn& rin, RegOut& rout,
                                            TwSet<L, TPF, FWD>& tw, Hook& hook) {
-  using P = FftPlan<L>;
+  using P = FftPlan<L, TPF>;
   constexpr int R = P::radix(FWD, I), NS = P::ns(FWD, I);
   constexpr bool first = I == 0, last = I == P::NP - 1;
   constexpr int S = first ? SRC : SRC_LDS;
   constexpr int D = last ? DST : DST_LDS;
-  static_assert(!(ZHI || LOW) || (!P::TRI && P::NP >= 2), "zero-half passes need a power-of-two plan");
-  static_assert(!(ZHI && first) || R == 16, "ZHI needs a radix-16 first pass");
-  static_assert(!(LOW && last) || (R == 16 && NS * R == L), "LOW needs an unstrided radix-16 last pass");
+  static_assert(!(ZHI || LOW) || (P::EVEN && P::NP >= 2), "zero-half passes need an even first radix");
+  static_assert(!(ZHI && first) || R >= 10, "ZHI needs a radix-16, -12 or -10 first pass");
+  static_assert(!(LOW && last) || (R >= 10 && NS * R == L), "LOW needs an unstrided last pass of such a radix");
   // TWPRE: the bases were loaded when the chain started; otherwise each pass
   // loads its own
   const float2* wb = tw.template at<I>();
+  constexpr int PB = TwSet<L, TPF, FWD>::per(I);
   if constexpr (first) {
-    pass_io<L, R, NS, TPF, INV, S, D, ZHI, false, TWPRE>(s, t, load, store, rin, wb);
+    pass_io<L, R, NS, TPF, INV, S, D, ZHI, false, TWPRE, PB>(s, t, load, store, rin, wb);
   } else if constexpr (last) {
     hook();
-    pass_io<L, R, NS, TPF, INV, S, D, false, LOW, TWPRE>(s, t, load, store, rout, wb);
+    pass_io<L, R, NS, TPF, INV, S, D, false, LOW, TWPRE, PB>(s, t, load, store, rout, wb);
   } else {
-    pass_io<L, R, NS, TPF, INV, S, D, false, false, TWPRE>(s, t, load, store, rout, wb);
+    pass_io<L, R, NS, TPF, INV, S, D, false, false, TWPRE, PB>(s, t, load, store, rout, wb);
   }
   if constexpr (!last)
     chain_pass<L, TPF, INV, FWD, I + 1, SRC, DST, ZHI, LOW, TWPRE>(s, t, load, store, rin, rout, tw, hook);
@@ -172,7 +179,7 @@ __device__ __forceinline__ void chain_io(float2* s, int t, Load& load, Store& st
 }
 
 template <int L, int TPF> struct HandOff {
-  using P = FftPlan<L>;
+  using P = FftPlan<L, TPF>;
   static constexpr int R = P::RH;
   static constexpr int NB = P::NBH;
   static constexpr int BPT = (NB + TPF - 1) / TPF;
@@ -209,7 +216,7 @@ __device__ __forceinline__ void fft_inverse_from_regs(float2* s, int t, typename
 // Output layout of the last pass of a plan: slot (b, q) holds index j + q*NS,
 // j = t + b*TPF < NB (NS = NB = L / R_last).
 template <int L, int TPF, bool FWD> struct LastPass {
-  using P = FftPlan<L>;
+  using P = FftPlan<L, TPF>;
   static constexpr int R = P::radix(FWD, P::NP - 1);
   static constexpr int NB = L / R;
   static constexpr int BPT = (NB + TPF - 1) / TPF;

@@ -1,6 +1,7 @@
 // Rayleigh-Sommerfeld convolution (scalar RS / vectorial VRS) on a P x P grid,
-// P = next power of two >= 2N-1, with the pre-propagation Jones masks and the
-// Ez construction fused into the first row pass.
+// P >= 2N-1 (the next power of two, or 3 * 2^k / 5 * 2^k below it, rs_fft_len),
+// with the pre-propagation Jones masks and the Ez construction fused into the
+// first row pass.
 //
 // Reference operator (xlumina/wave_optics.py:281-289): zero-pad the N x N field
 // into a (2N-1)^2 grid, multiply fft2(U) by fft2(H) of the sampled RS impulse
@@ -200,8 +201,8 @@ __host__ __device__ constexpr int64_t rs_hr_elems(int n, int P) { return (int64_
 // Column stride of Hhat: ky = 0..P/2 and a pad to whole 128 B lines.
 __host__ __device__ constexpr int rs_hh_stride(int P) { return P / 2 + 16; }
 
-// A transform of P points runs on TPF = P/16 threads (one radix-16 butterfly
-// each per pass) in one LDS buffer.  A block takes G rows (or columns) of one
+// A transform of P points runs on TPF threads (one butterfly each per pass,
+// P/16 for the powers of two) in one LDS buffer.  A block takes G rows (or columns) of one
 // 4x4 tile group, lanes spread over the G transforms, so that an access of a
 // wave covers G/4 of each 128 B line it touches instead of a quarter; more
 // than one 35 KB buffer behind common barriers hides less of the transforms'
@@ -216,12 +217,16 @@ __host__ __device__ constexpr int rs_hh_stride(int P) { return P / 2 + 16; }
 //   col (3 comp.)       133   151    39.2  38.8  51.0  12.6  13.1     6.9   8.2
 //   col (1 comp.)                    15.6  14.8         7.9   7.5
 //   final (3 comp.)    74.5  66.7    17.1  15.0  17.4   6.5   5.8     4.4   4.4
-// Below P = 1024 a block holds at least one wave.
+// The lengths between take the column of the next power of two (VRS 1200^2 at
+// P = 2560, G = 1 / 2 everywhere: 156 / 188 us).  Below P = 1024 a block holds
+// at least one wave.
 constexpr int rs_g(int P, int g4096, int g2048, int g1024) {
-  return P >= 4096 ? g4096 : P >= 2048 ? g2048 : P >= 1024 ? g1024 : 1024 / P;
+  return P > 2048 ? g4096 : P == 2048 ? g2048 : P >= 1024 ? g1024 : 1024 / P;
 }
+// Threads per transform: P over the first radix of its passes.
+constexpr int rs_tpf(int P) { return P % 3 == 0 ? P / 12 : P % 5 == 0 ? P / 10 : P / 16; }
 template <int P, int G_> struct Units {
-  static constexpr int TPF = P / 16;
+  static constexpr int TPF = rs_tpf(P);
   static constexpr int G = G_;
   static constexpr int NT = G * TPF;   // threads per block
   static_assert(NT >= 64, "whole waves");
@@ -338,20 +343,21 @@ __global__ __launch_bounds__(UHrow<P>::NT, 4) void rs_hrow_kernel(RsArgs a0) {
 }
 
 // G input rows per block.  Thread t's first-pass inputs are the columns
-// t + r P/16; the nonzero ones (columns < N <= P/2) are r < 8, so each thread
-// computes the masks and Ez of exactly those 8 pixels once, keeps all
-// components in registers, and the components are transformed one after the
-// other from there (no LDS staging pass).
+// t + r TPF; the nonzero ones (columns < N <= P/2) are the lower half of the
+// first radix (8 at the powers of two), so each thread computes the masks and
+// Ez of exactly those pixels once, keeps all components in registers, and the
+// components are transformed one after the other from there (no LDS staging
+// pass).
 // ONE (inputs without masks or Ez construction: the adjoint's cotangent): one
 // component (blockIdx.z) per block, for grids whose row blocks alone leave
 // resident slots empty.
 template <int P, bool ONE = false>
-__global__ __launch_bounds__((UUrow<P, ONE>::NT)) void rs_urow_kernel(RsArgs a0) {
+__global__ __launch_bounds__((UUrow<P, ONE>::NT), P == 1536 ? 3 : 1) void rs_urow_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
   using U = UUrow<P, ONE>;
   constexpr int TPF = U::TPF;
-  constexpr int R0 = FftPlan<P>::radix(true, 0);
-  static_assert(R0 == 16 && P / R0 == TPF, "first pass: one radix-16 butterfly per thread");
+  constexpr int R0 = FftPlan<P, TPF>::radix(true, 0);
+  static_assert(P / R0 == TPF, "first pass: one butterfly per thread");
   constexpr int H = R0 / 2;   // inputs r < H hold the N <= P/2 pixels
   __shared__ float2 lds[U::G * U::LS];
   const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
@@ -379,7 +385,7 @@ __global__ __launch_bounds__((UUrow<P, ONE>::NT)) void rs_urow_kernel(RsArgs a0)
   }
   const int nc = a.ncomp;
   const double z = a.z_dev ? *a.z_dev : a.z;
-  // all loads of the 8 pixels first (in flight together), then the masks and Ez
+  // all loads of a thread's pixels first (in flight together), then the masks and Ez
   const bool ez = a.ez_mode != EZ_NONE;
   // (columns beyond N read the row's last pixel and are zeroed below)
   PixRaw raw[H];
@@ -448,7 +454,7 @@ __global__ __launch_bounds__(UHcol<P>::NT, 4) void rs_hcol_kernel(RsArgs a0) {
 #pragma unroll
     for (int q = 0; q < HO::R; ++q) {
       const int k = HO::koff(b, q);
-      if (k > P / 2) continue;
+      if (k > P / 2 || !HO::valid(t, b)) continue;
       float2 h = u.v[b][q] * a.scale;
       if (a.adjoint && !a.hstored) h = conjf2(h);
       if (act && (k < P / 2 || t == 0)) st_at(dst + k, g * HS + t, h);
@@ -538,7 +544,8 @@ __global__ __launch_bounds__(UCol<P>::NT, 4) void rs_col_kernel(RsArgs a0) {
 #pragma unroll
       for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
-        for (int q = 0; q < HO::R; ++q) h.v[b][q] = hat(a.hh, HO::koff(b, q));
+        for (int q = 0; q < HO::R; ++q)
+          if (HO::valid(t, b)) h.v[b][q] = hat(a.hh, HO::koff(b, q));
     }
   };
   fft_forward_to_regs<P, TPF, SRC_FN, true>(s, t, load, u, hook);
@@ -550,11 +557,13 @@ __global__ __launch_bounds__(UCol<P>::NT, 4) void rs_col_kernel(RsArgs a0) {
   }
   const float hs = (a.adjoint && a.hstored) ? -1.f : 1.f;   // stored spectrum: conjugate for the adjoint
   double acc[2] = {0.0, 0.0};
+  static_assert(SPEC == 0 || HO::NB % TPF == 0, "spectra are kept at the power-of-two lengths");
 #pragma unroll
   for (int b = 0; b < HO::BPT; ++b)
 #pragma unroll
     for (int q = 0; q < HO::R; ++q) {
       const int k = HO::koff(b, q);
+      if (!HO::valid(t, b)) continue;
       float2 hv = HPRE ? h.v[b][q] : hat(a.hh, k);
       hv.y *= hs;
       if constexpr (GB != 0) {
@@ -693,17 +702,17 @@ template <int P> inline void rs_spectrum_launch(const RsArgs& a, int nb, hipStre
   hipLaunchKernelGGL(rs_hcol_kernel<P>, rs_grid<UHcol<P>>(P / 2 + 1, nb), dim3(UHcol<P>::NT), 0, st, a);
 }
 
+// The kernel-spectrum passes of a call that keeps or reuses spectra: the
+// derivative spectra it asks for, and (unless an earlier call built it) Hhat
+// with the derivatives of a forward call that will be differentiated.
 template <int P>
-inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
-  const int rows = rs_rows4(a.n);
-  const int nb = a.batch > 1 ? a.batch : 1;
-  const dim3 ghr = rs_grid<UHrow<P>>(rows, nb), bhr(UHrow<P>::NT), ghc = rs_grid<UHcol<P>>(P / 2 + 1, nb),
-             bhc(UHcol<P>::NT), bcl(UCol<P>::NT), bfn(UFinal<P>::NT);
+inline void rs_kept_spectra_launch(const RsArgs& a, int nb, hipStream_t st) {
+  const dim3 ghr = rs_grid<UHrow<P>>(rs_rows4(a.n), nb), bhr(UHrow<P>::NT), ghc = rs_grid<UHcol<P>>(P / 2 + 1, nb),
+             bhc(UHcol<P>::NT);
   // a forward call that keeps its spectra for a gradient builds the derivative
   // spectra with its own kernel rows (one float64 geometry for all of them)
   const int dm = (a.dg[0] ? 1 : 0) | (a.dg[1] ? 2 : 0);
   const bool with_h = a.spec_mode == 1 && dm && !a.hreuse;
-  // Hr lives in the tiles that rs_urow fills later, so the spectra come first
   if ((a.spec_mode == 2 && !a.dg_built) || (a.spec_mode == 1 && dm && !with_h)) {
     // derivative spectra (dH/dz, dH/dk) with the spectrum passes, unconjugated
     for (int i = 0; i < 2; ++i) {
@@ -717,36 +726,54 @@ inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
       rs_spectrum_launch<P>(d, nb, st);
     }
   }
-  if (!a.hreuse) {
+  if (a.hreuse) return;
+  {
+    KTimer t(K_RS_HROW, st);
+    if (with_h && dm == 1)
+      hipLaunchKernelGGL((rs_hrow_kernel<P, 1>), ghr, bhr, 0, st, a);
+    else if (with_h && dm == 2)
+      hipLaunchKernelGGL((rs_hrow_kernel<P, 2>), ghr, bhr, 0, st, a);
+    else if (with_h)
+      hipLaunchKernelGGL((rs_hrow_kernel<P, 3>), ghr, bhr, 0, st, a);
+    else
+      hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), ghr, bhr, 0, st, a);
+  }
+  KTimer t(K_RS_HCOL, st);
+  hipLaunchKernelGGL(rs_hcol_kernel<P>, ghc, bhc, 0, st, a);
+  for (int i = 0; with_h && i < 2; ++i) {
+    if (!a.dg[i]) continue;
+    RsArgs d = a;   // the derivative row transforms, unconjugated
+    d.hr = a.dgr[i];
+    d.hh = a.dg[i];
+    d.adjoint = 0;
+    d.hstored = 1;
+    hipLaunchKernelGGL(rs_hcol_kernel<P>, ghc, bhc, 0, st, d);
+  }
+}
+
+// KEEP: calls that keep or reuse spectra (hhat, spec) run at this length.
+template <int P, bool KEEP>
+inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
+  const int rows = rs_rows4(a.n);
+  const int nb = a.batch > 1 ? a.batch : 1;
+  // Hr lives in the tiles that rs_urow fills later, so the spectra come first
+  if (KEEP && (a.hstored || a.spec_mode)) {
+    if constexpr (KEEP) rs_kept_spectra_launch<P>(a, nb, st);
+  } else {
     {
       KTimer t(K_RS_HROW, st);
-      if (with_h && dm == 1)
-        hipLaunchKernelGGL((rs_hrow_kernel<P, 1>), ghr, bhr, 0, st, a);
-      else if (with_h && dm == 2)
-        hipLaunchKernelGGL((rs_hrow_kernel<P, 2>), ghr, bhr, 0, st, a);
-      else if (with_h)
-        hipLaunchKernelGGL((rs_hrow_kernel<P, 3>), ghr, bhr, 0, st, a);
-      else
-        hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), ghr, bhr, 0, st, a);
+      hipLaunchKernelGGL((rs_hrow_kernel<P, 0>), rs_grid<UHrow<P>>(rows, nb), dim3(UHrow<P>::NT), 0, st, a);
     }
     KTimer t(K_RS_HCOL, st);
-    hipLaunchKernelGGL(rs_hcol_kernel<P>, ghc, bhc, 0, st, a);
-    for (int i = 0; with_h && i < 2; ++i) {
-      if (!a.dg[i]) continue;
-      RsArgs d = a;   // the derivative row transforms, unconjugated
-      d.hr = a.dgr[i];
-      d.hh = a.dg[i];
-      d.adjoint = 0;
-      d.hstored = 1;
-      hipLaunchKernelGGL(rs_hcol_kernel<P>, ghc, bhc, 0, st, d);
-    }
+    hipLaunchKernelGGL(rs_hcol_kernel<P>, rs_grid<UHcol<P>>(P / 2 + 1, nb), dim3(UHcol<P>::NT), 0, st, a);
   }
   {
     KTimer t(K_RS_UROW, st);
-    // plain inputs (no masks, no Ez) over fewer row blocks than resident
-    // slots: one block per (row, component)
-    const bool one = P <= 2048 && a.ncomp > 1 && a.nin == a.ncomp && a.ez_mode == EZ_NONE && !a.mask.st[0].kind &&
-                     !a.mask.st[1].kind && rows * nb < 2048;
+    // plain inputs (no masks, no Ez): one block per (row, component), where
+    // the row blocks alone leave resident slots empty, and at P = 4096 (two
+    // rows per block: 69 us against 84 us at 2048^2, three components)
+    const bool one = a.ncomp > 1 && a.nin == a.ncomp && a.ez_mode == EZ_NONE && !a.mask.st[0].kind &&
+                     !a.mask.st[1].kind && (P >= 4096 || rows * nb < 2048);
     using U1 = UUrow<P, true>;
     using U3 = UUrow<P, false>;
     if (one) hipLaunchKernelGGL((rs_urow_kernel<P, true>), rs_grid<U1>(rows, nb, a.ncomp), dim3(U1::NT), 0, st, a);
@@ -754,29 +781,30 @@ inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
   }
   {
     KTimer t(K_RS_COL, st);
-    const dim3 grid = rs_grid<UCol<P>>(P, nb, a.ncomp);
-    if (a.spec_mode == 1)
-      hipLaunchKernelGGL((rs_col_kernel<P, 1>), grid, bcl, 0, st, a);
-    else if (a.spec_mode == 2 && dm == 1)
-      hipLaunchKernelGGL((rs_col_kernel<P, 3>), grid, bcl, 0, st, a);
-    else if (a.spec_mode == 2 && dm == 2)
-      hipLaunchKernelGGL((rs_col_kernel<P, 4>), grid, bcl, 0, st, a);
-    else if (a.spec_mode == 2 && dm == 3)
-      hipLaunchKernelGGL((rs_col_kernel<P, 5>), grid, bcl, 0, st, a);
-    else
-      hipLaunchKernelGGL((rs_col_kernel<P, 0>), grid, bcl, 0, st, a);
+    const dim3 grid = rs_grid<UCol<P>>(P, nb, a.ncomp), blk(UCol<P>::NT);
+    bool done = false;
+    if constexpr (KEEP) {
+      const int gb = a.spec_mode == 2 ? (a.dg[0] ? 1 : 0) | (a.dg[1] ? 2 : 0) : 0;
+      done = a.spec_mode == 1 || gb != 0;
+      if (a.spec_mode == 1) hipLaunchKernelGGL((rs_col_kernel<P, 1>), grid, blk, 0, st, a);
+      else if (gb == 1) hipLaunchKernelGGL((rs_col_kernel<P, 3>), grid, blk, 0, st, a);
+      else if (gb == 2) hipLaunchKernelGGL((rs_col_kernel<P, 4>), grid, blk, 0, st, a);
+      else if (gb == 3) hipLaunchKernelGGL((rs_col_kernel<P, 5>), grid, blk, 0, st, a);
+    }
+    if (!done) hipLaunchKernelGGL((rs_col_kernel<P, 0>), grid, blk, 0, st, a);
   }
-  if (a.spec_mode == 2 && !a.partials_only) {
+  if (KEEP && a.spec_mode == 2 && !a.partials_only) {
     KTimer t(K_LOSS, st);
     hipLaunchKernelGGL(rs_grad_reduce_kernel, dim3(2), dim3(1024), 0, st, a.gpart[0], a.gpart[1], P * a.ncomp,
                        a.grad_out);
   }
   {
     KTimer t(K_RS_FINAL, st);
+    const dim3 blk(UFinal<P>::NT);
     if (a.intensity)
-      hipLaunchKernelGGL((rs_final_kernel<P, false>), rs_grid<UFinal<P>>(a.n, nb), bfn, 0, st, a);
+      hipLaunchKernelGGL((rs_final_kernel<P, false>), rs_grid<UFinal<P>>(a.n, nb), blk, 0, st, a);
     else
-      hipLaunchKernelGGL((rs_final_kernel<P, true>), rs_grid<UFinal<P>>(a.n, nb, a.ncomp), bfn, 0, st, a);
+      hipLaunchKernelGGL((rs_final_kernel<P, true>), rs_grid<UFinal<P>>(a.n, nb, a.ncomp), blk, 0, st, a);
   }
   return hipGetLastError();
 }

@@ -122,7 +122,26 @@ int check_mask(const xl_mask_stage* m, int nin, int batch = 1) {
 }
 
 // ---------------------------------------------------------------- RS
+// The power-of-two length that holds a problem: it sizes every buffer, and is
+// the length of calls that keep or reuse spectra.
 int rs_fft_len(int n) { return std::max(64, next_pow2(2 * (int64_t)n - 1)); }
+
+// The length a plain call runs at: from n = 513 on, the shortest of 2^k,
+// 5 * 2^k and 3 * 2^k that holds 2n - 1 samples.  Work and traffic follow the
+// length in both axes (one box, kernels of a VRS call: 1200^2 at 4096 / 2560 217 /
+// 156 us, 1500^2 at 4096 / 3072 248 / 198, 600^2 at 2048 / 1280 82 / 68, 750^2 at
+// 2048 / 1536 92 / 81; error against float64 7e-7 -> 3.5e-7 .. 5e-7, two table
+// entries per twiddle set instead of one).  Below, a call is bound by its launches
+// and the radix-16 lengths stay.  Calls that keep spectra (hhat, spec)
+// stay at 2^k: their buffers hold that layout, and the float64 gradients formed
+// behind them are then the same to the last bit whatever n.
+int rs_plain_len(int n) {
+  const int P = rs_fft_len(n), need = 2 * n - 1;
+  if (P < 2048) return P;
+  if (need <= P / 8 * 5) return P / 8 * 5;
+  if (need <= P / 4 * 3) return P / 4 * 3;
+  return P;
+}
 
 // complex64 elements of one problem's workspace block: tiles + kernel spectrum
 int64_t rs_ws_elems(int n, int ncomp) {
@@ -327,8 +346,9 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
   if (!device_ready()) return fail(XL_EINVAL, "xl_init() has not run on this device");
   const int n = p->n;
   if (n < 2) return fail(XL_EINVAL, "grid side must be >= 2");
-  const int P = rs_fft_len(n);
-  if (P > xl::MAX_FFT) return fail(XL_EINVAL, "grid side " + std::to_string(n) + " needs FFT length > 4096");
+  if (n > xl::MAX_FFT / 2) return fail(XL_EINVAL, "grid side " + std::to_string(n) + " needs FFT length > 4096");
+  const bool keeps = p->hhat_mode || p->spec_mode;
+  const int P2 = rs_fft_len(n), P = keeps ? P2 : rs_plain_len(n);
   if (p->nin < 1 || p->nin > 3) return fail(XL_EINVAL, "nin must be 1..3");
   if (p->ez_mode != XL_EZ_NONE && p->ez_mode != XL_EZ_VRS) return fail(XL_EINVAL, "RS supports XL_EZ_NONE / XL_EZ_VRS");
   if (p->ez_mode == XL_EZ_VRS && p->nin < 2) return fail(XL_EINVAL, "Ez construction needs Ex and Ey");
@@ -377,7 +397,7 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
   a.intensity = p->intensity;
   a.t = (float2*)w;
   a.hr = a.t;   // the row-transformed kernel, until the field's rows take its place
-  a.hh = p->hhat_mode ? (float2*)p->hhat : a.t + ncomp * nr4 * P;
+  a.hh = p->hhat_mode ? (float2*)p->hhat : a.t + ncomp * nr4 * P2;
   a.hstored = p->hhat_mode ? 1 : 0;
   a.hreuse = p->hhat_mode == 2 ? 1 : 0;
   a.x = p->x;
@@ -400,7 +420,7 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
   a.inten_bs = batch > 1 ? p->intensity_batch_stride : 0;
   a.mask_bs = batch > 1 ? p->mask_batch_stride : 0;
   a.t_bs = rs_ws_elems(n, ncomp);
-  a.hh_bs = p->hhat_mode ? (int64_t)(P / 2) * P + P : a.t_bs;   // hhat holds one spectrum per member
+  a.hh_bs = p->hhat_mode ? (int64_t)(P2 / 2) * P2 + P2 : a.t_bs;   // hhat holds one spectrum per member
   a.spec_mode = p->spec_mode;
   a.spec = nullptr;
   a.dg[0] = a.dg[1] = nullptr;
@@ -429,8 +449,14 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
       }
   }
   hipStream_t st = (hipStream_t)stream;
-  int rc = dispatch_q(P, [&](auto c) { (void)xl::rs_launch<decltype(c)::value>(a, st); });
-  if (rc) return rc;
+  switch (P) {
+    case 1280: (void)xl::rs_launch<1280, false>(a, st); break;
+    case 1536: (void)xl::rs_launch<1536, false>(a, st); break;
+    case 2560: (void)xl::rs_launch<2560, false>(a, st); break;
+    case 3072: (void)xl::rs_launch<3072, false>(a, st); break;
+    default:
+      if (int rc = dispatch_q(P, [&](auto c) { (void)xl::rs_launch<decltype(c)::value, true>(a, st); })) return rc;
+  }
   return hip_check(hipGetLastError(), "RS launch");
 }
 

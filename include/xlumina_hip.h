@@ -293,6 +293,14 @@ int xl_czt_gemm(const xl_czt_params* p, void* workspace, size_t workspace_bytes,
  * (optical_elements.py:87-332), high_NA_objective_lens (:515-594). */
 int xl_pre_forward(const xl_pre_params* p, void* stream);
 int xl_pre_backward(const xl_pre_params* p, void* stream);
+/* xl_rs_propagate (an adjoint call) followed by xl_pre_backward on its output:
+ * q->gout is p->out, q's plane is p's n x n and q->ncomp its component count.
+ * Where the pre-op is an SLM of per-pixel phases on one component, or the VRS
+ * Ez construction of an unmasked field, the propagation's last pass forms the
+ * pre-op's cotangents itself and p->out is not written; otherwise p->out holds
+ * the propagation's output as after the two calls. */
+int xl_rs_adjoint_pre(const xl_rs_params* p, const xl_pre_params* q, void* workspace, size_t workspace_bytes,
+                      void* stream);
 /* doubles of the gradient buffer of a scalar-form mask parameter in
  * xl_pre_backward over rows x cols pixels: the sum at element 0, one partial
  * sum per launch block after it (see XL_PF_SCALAR). */

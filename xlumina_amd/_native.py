@@ -148,6 +148,7 @@ SIGNATURES = {
     "xl_rs_spec_partials": (C.c_int64, [C.c_int32, C.c_int32, C.c_int32, C.POINTER(C.c_int32)]),
     "xl_pre_scalar_grad_elems": (C.c_size_t, [C.c_int32, C.c_int32]),
     "xl_rs_propagate": (C.c_int, [C.POINTER(RsParams), C.c_void_p, C.c_size_t, C.c_void_p]),
+    "xl_rs_adjoint_pre": (C.c_int, [C.POINTER(RsParams), C.POINTER(PreParams), C.c_void_p, C.c_size_t, C.c_void_p]),
     "xl_rs_propagate_noalloc": (C.c_int, [C.POINTER(RsParams), C.c_void_p]),
     "xl_czt_workspace_bytes": (C.c_size_t, [C.POINTER(CztParams)]),
     "xl_czt": (C.c_int, [C.POINTER(CztParams), C.c_void_p, C.c_size_t, C.c_void_p]),

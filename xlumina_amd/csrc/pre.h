@@ -308,6 +308,162 @@ __global__ __launch_bounds__(256) void pre_backward_kernel(PreArgs a0) {
   }
 }
 
+// Last pass of an adjoint RS / VRS propagation and the pre-op adjoint in one:
+// a row's cotangent components are inverse-transformed one after the other as
+// in rs_final_kernel and go from registers through the Ez construction's or
+// the mask's adjoint, so the cotangent of the padded field is neither written
+// nor read again (24 B each way per pixel of a VRS adjoint, and a launch).
+// EZ: the VRS Ez construction of an unmasked field; Ez' cotangent comes first
+// and stays (16 registers), Ex' and Ey' are finished and stored as they appear
+// (1024^2: 23.3 us, rs_final 14.8 + pre_backward 17 before).  Otherwise one
+// component behind an SLM of float32 or float64 per-pixel phases.  Masks on
+// three components keep the separate kernels: with an sSLM's phases, input and
+// gradients on top the pass runs at four waves and waits for its loads (1024^2
+// 44 us, separate 40), and a retarder couples Ex and Ey.
+// b.ezdz receives one partial sum per block.
+template <int P, bool EZ>
+__global__ __launch_bounds__(UFinal<P>::NT, 4) void rs_final_pre_kernel(RsArgs a, PreArgs b) {
+  using U = UFinal<P>;
+  constexpr int TPF = U::TPF, NC = EZ ? 3 : 1;
+  constexpr bool SMALL = P < 1024;
+  using LP = LastPass<P, TPF, SMALL>;
+  constexpr int QH = LP::R / 2, NPX = LP::BPT * QH;   // pixels per thread
+  __shared__ float2 lds[U::G * U::LS];
+  const int g = U::row_g(threadIdx.x), t = U::row_t(threadIdx.x);
+  float2* s = lds + g * U::LS;
+  const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
+  const RowTiles rt(a.n, g, t);
+  const bool load_ok = row < rt.nrg * 4, rowok = row < a.n;
+  const double Y = EZ ? b.y[rowok ? row : 0] : 0.0, z = EZ ? (b.z_dev ? *b.z_dev : b.z) : 0.0;
+  const uint32_t row_at = (uint32_t)(rowok ? row : 0) * a.n;
+  const bool ezdz = EZ && b.ezdz;
+  MaskStage m = b.mask.st[0];
+  m.kind = MASK_SLM;
+  float2 g2[NPX];
+  double acc_ez = 0.0;
+  NoIO none;
+#pragma unroll
+  for (int ci = 0; ci < NC; ++ci) {
+    const int c = EZ ? (ci + 2) % 3 : 0;   // Ez first
+    const float2* tc = a.t + (int64_t)c * rt.nrg * 4 * P + RowTiles::base(row0);
+    auto load = [&](int k) -> float2 { return load_ok ? ld_at(tc + rt.step(k), rt.lane) : make_float2(0.f, 0.f); };
+    typename LP::Type o, unused;
+    chain_io<P, TPF, true, SMALL, 0, SRC_FN, DST_REG, false, !SMALL>(s, t, load, none, unused, o);
+    if constexpr (SMALL) {
+      // (roundings are those of the whole transform, as in rs_final)
+#pragma unroll
+      for (int i = 0; i < LP::BPT; ++i)
+#pragma unroll
+        for (int q = QH; q < LP::R; ++q) asm volatile("" ::"v"(o.v[i][q].x), "v"(o.v[i][q].y));
+    }
+#pragma unroll
+    for (int i = 0; i < LP::BPT; ++i)
+#pragma unroll
+      for (int q = 0; q < QH; ++q) asm volatile("" : "+v"(o.v[i][q].x), "+v"(o.v[i][q].y));
+    if (c == 2) {
+#pragma unroll
+      for (int p = 0; p < NPX; ++p) g2[p] = o.v[p / QH][p % QH];
+      if (b.out) {
+#pragma unroll
+        for (int p = 0; p < NPX; ++p) {
+          const int col = LP::index(t, p / QH, p % QH);
+          if (rowok && LP::valid(t, p / QH) && col < a.n && max(b.nin, b.out_planes) > 2)
+            st_at(b.out + 2 * b.in_cs, row_at + col, make_float2(0.f, 0.f));
+        }
+      }
+      continue;
+    }
+    // GP pixels at a time, their loads ahead of the arithmetic (pixels beyond
+    // the row read its last one and are not stored)
+    constexpr int GP = NPX < 4 ? NPX : 4;
+    const bool wantp = !EZ && b.gparam[0][0];
+    const int form = EZ ? 0 : param_form(m, 0);
+#pragma unroll
+    for (int p0 = 0; p0 < NPX; p0 += GP) {
+      uint32_t pix[GP];
+      bool ok[GP];
+      double X[GP];
+      float2 e[GP];
+      float v[GP];
+#pragma unroll
+      for (int u = 0; u < GP; ++u) {
+        const int i = (p0 + u) / QH, q = (p0 + u) % QH, col = LP::index(t, i, q), cc = min(col, a.n - 1);
+        ok[u] = rowok && LP::valid(t, i) && col < a.n;
+        pix[u] = row_at + cc;
+        X[u] = EZ ? at32(b.x, (uint32_t)cc) : 0.0;
+        e[u] = make_float2(0.f, 0.f);
+        v[u] = 0.f;
+      }
+      if (wantp || ezdz) {
+#pragma unroll
+        for (int u = 0; u < GP; ++u) e[u] = at32(b.in + c * b.in_cs, pix[u]);
+      }
+      if constexpr (!EZ) {
+#pragma unroll
+        for (int u = 0; u < GP; ++u) v[u] = mask_param(m, 0, pix[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < GP; ++u) {
+        const int p = p0 + u;
+        float2 gc = o.v[p / QH][p % QH];
+        if constexpr (EZ) {
+          // direction cosine X/r or Y/r, to float32 from float64
+          const double ir = rsqrt_f64(X[u] * X[u] + Y * Y + z * z), D = c ? Y : X[u];
+          if (ezdz && ok[u])   // d Ez_in / dz, as in pre_backward_kernel
+            acc_ez += (double)(re_conj_mul(g2[p], e[u]) * (float)(D * (-z * (ir * ir * ir))));
+          gc = c_add(gc, c_scale(g2[p], (float)(D * ir)));
+        }
+        if (!ok[u]) continue;
+        if constexpr (!EZ) {
+          const float2 w = c_expi(v[u]);
+          if (wantp) {
+            // d/dphi = i e'; the roundings are written out, since float64 gradients show them: those of the
+            // separate kernels (the lone float32 SLM's, and pre_backward_kernel's)
+            const float2 e1 = e[u];
+            const float fy = form == 0 ? fmaf(e1.x, w.y, __fmul_rn(e1.y, w.x)) : fmaf(e1.y, w.x, __fmul_rn(e1.x, w.y));
+            const float fx = fmaf(e1.x, w.x, -__fmul_rn(e1.y, w.y));
+            const float d = fmaf(gc.y, fx, -__fmul_rn(gc.x, fy));
+            if (!(form & PF_F64)) b.gparam[0][0][pix[u]] = d;
+            else reinterpret_cast<double*>(b.gparam[0][0])[pix[u]] = (form & PF_UNIT) ? 6.283185307179586 * d : d;
+          }
+          gc = c_mul(gc, make_float2(w.x, -w.y));
+        }
+        if (b.out) {
+          st_at(b.out + c * b.in_cs, pix[u], gc);
+          if constexpr (!EZ)
+            for (int k = 1; k < b.out_planes; ++k) st_at(b.out + k * b.in_cs, pix[u], make_float2(0.f, 0.f));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (EZ) {
+    if (ezdz) {
+      __shared__ double red[U::NT / 64];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) acc_ez += __shfl_xor(acc_ez, o, 64);
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc_ez;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < U::NT / 64; ++w) v += red[w];
+        b.ezdz[1 + blockIdx.x] = v;
+      }
+    }
+  }
+}
+
+// Blocks of the fused last pass (its per-block partial sums).
+template <int P> inline int rs_final_pre_blocks(int n) { return (n + UFinal<P>::G - 1) / UFinal<P>::G; }
+
+template <int P> inline void rs_final_pre_launch(const RsArgs& a, const PreArgs& b, hipStream_t st) {
+  KTimer t(K_RS_FINAL, st);
+  const dim3 g(rs_final_pre_blocks<P>(a.n)), blk(UFinal<P>::NT);
+  if (b.ez_mode == EZ_NONE) hipLaunchKernelGGL((rs_final_pre_kernel<P, false>), g, blk, 0, st, a, b);
+  else hipLaunchKernelGGL((rs_final_pre_kernel<P, true>), g, blk, 0, st, a, b);
+}
+
 // buf[i][0] = sum of buf[i][1 .. n] for the scalar-form parameter gradients
 // and the Ez_in distance term (block i; null pointers skip), fixed order;
 // base4[0 .. nbase), if set, is added to the Ez_in term's sum.

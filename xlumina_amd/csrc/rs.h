@@ -751,9 +751,10 @@ inline void rs_kept_spectra_launch(const RsArgs& a, int nb, hipStream_t st) {
   }
 }
 
-// KEEP: calls that keep or reuse spectra (hhat, spec) run at this length.
+// All passes up to the column pass.  KEEP: calls that keep or reuse spectra
+// (hhat, spec) run at this length.
 template <int P, bool KEEP>
-inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
+inline void rs_launch(const RsArgs& a, hipStream_t st) {
   const int rows = rs_rows4(a.n);
   const int nb = a.batch > 1 ? a.batch : 1;
   // Hr lives in the tiles that rs_urow fills later, so the spectra come first
@@ -798,15 +799,18 @@ inline hipError_t rs_launch(const RsArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(rs_grad_reduce_kernel, dim3(2), dim3(1024), 0, st, a.gpart[0], a.gpart[1], P * a.ncomp,
                        a.grad_out);
   }
-  {
-    KTimer t(K_RS_FINAL, st);
-    const dim3 blk(UFinal<P>::NT);
-    if (a.intensity)
-      hipLaunchKernelGGL((rs_final_kernel<P, false>), rs_grid<UFinal<P>>(a.n, nb), blk, 0, st, a);
-    else
-      hipLaunchKernelGGL((rs_final_kernel<P, true>), rs_grid<UFinal<P>>(a.n, nb, a.ncomp), blk, 0, st, a);
-  }
-  return hipGetLastError();
+}
+
+// The last pass of a call that returns the field.
+template <int P>
+inline void rs_final_launch(const RsArgs& a, hipStream_t st) {
+  const int nb = a.batch > 1 ? a.batch : 1;
+  KTimer t(K_RS_FINAL, st);
+  const dim3 blk(UFinal<P>::NT);
+  if (a.intensity)
+    hipLaunchKernelGGL((rs_final_kernel<P, false>), rs_grid<UFinal<P>>(a.n, nb), blk, 0, st, a);
+  else
+    hipLaunchKernelGGL((rs_final_kernel<P, true>), rs_grid<UFinal<P>>(a.n, nb, a.ncomp), blk, 0, st, a);
 }
 
 }  // namespace xl

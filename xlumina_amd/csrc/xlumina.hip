@@ -341,13 +341,14 @@ size_t xl_rs_batch_workspace_bytes(int32_t n, int32_t ncomp, int32_t batch) {
   return rs_ws(n, ncomp, batch);
 }
 
-int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stream) {
+// pre: the pre-op adjoint that takes the place of the field's output (fused last pass).
+static int rs_run(const xl_rs_params* p, const xl::PreArgs* pre, void* ws, size_t ws_bytes, void* stream) {
   if (!p) return fail(XL_EINVAL, "null params");
   if (!device_ready()) return fail(XL_EINVAL, "xl_init() has not run on this device");
   const int n = p->n;
   if (n < 2) return fail(XL_EINVAL, "grid side must be >= 2");
   if (n > xl::MAX_FFT / 2) return fail(XL_EINVAL, "grid side " + std::to_string(n) + " needs FFT length > 4096");
-  const bool keeps = p->hhat_mode || p->spec_mode;
+  const bool keeps = p->hhat_mode || p->spec_mode || pre;   // (the fused last pass exists at 2^k)
   const int P2 = rs_fft_len(n), P = keeps ? P2 : rs_plain_len(n);
   if (p->nin < 1 || p->nin > 3) return fail(XL_EINVAL, "nin must be 1..3");
   if (p->ez_mode != XL_EZ_NONE && p->ez_mode != XL_EZ_VRS) return fail(XL_EINVAL, "RS supports XL_EZ_NONE / XL_EZ_VRS");
@@ -449,15 +450,26 @@ int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stre
       }
   }
   hipStream_t st = (hipStream_t)stream;
+  auto run = [&](auto c, auto keep) {
+    constexpr int L = decltype(c)::value;
+    xl::rs_launch<L, decltype(keep)::value>(a, st);
+    if constexpr (decltype(keep)::value)
+      if (pre) return xl::rs_final_pre_launch<L>(a, *pre, st);
+    xl::rs_final_launch<L>(a, st);
+  };
   switch (P) {
-    case 1280: (void)xl::rs_launch<1280, false>(a, st); break;
-    case 1536: (void)xl::rs_launch<1536, false>(a, st); break;
-    case 2560: (void)xl::rs_launch<2560, false>(a, st); break;
-    case 3072: (void)xl::rs_launch<3072, false>(a, st); break;
+    case 1280: run(std::integral_constant<int, 1280>(), std::false_type()); break;
+    case 1536: run(std::integral_constant<int, 1536>(), std::false_type()); break;
+    case 2560: run(std::integral_constant<int, 2560>(), std::false_type()); break;
+    case 3072: run(std::integral_constant<int, 3072>(), std::false_type()); break;
     default:
-      if (int rc = dispatch_q(P, [&](auto c) { (void)xl::rs_launch<decltype(c)::value, true>(a, st); })) return rc;
+      if (int rc = dispatch_q(P, [&](auto c) { run(c, std::true_type()); })) return rc;
   }
   return hip_check(hipGetLastError(), "RS launch");
+}
+
+int xl_rs_propagate(const xl_rs_params* p, void* ws, size_t ws_bytes, void* stream) {
+  return rs_run(p, nullptr, ws, ws_bytes, stream);
 }
 
 int xl_rs_propagate_noalloc(const xl_rs_params* p, void* stream) {
@@ -965,6 +977,50 @@ int xl_pre_backward(const xl_pre_params* p, void* stream) {
                          std::max(1, (int)p->ez_dz_base_n));
   }
   return hip_check(hipGetLastError(), "pre_backward launch");
+}
+
+// The pre-ops whose adjoint the last pass of the adjoint propagation takes on
+// (rs_final_pre_kernel): one component behind an SLM of per-pixel phases, or
+// the VRS Ez construction of an unmasked field.
+static bool rs_pre_fuses(const xl_rs_params* p, const xl_pre_params* q) {
+  const xl_mask_stage& m = q->mask[0];
+  if (q->mask[1].kind != XL_MASK_NONE || q->hna || q->batch > 1 || p->batch > 1 || p->intensity) return false;
+  if (q->gparam[0][1] || q->gparam[1][0] || q->gparam[1][1]) return false;
+  if (q->ez_mode == XL_EZ_VRS) return m.kind == XL_MASK_NONE && q->ncomp == 3 && !q->gparam[0][0];
+  return q->ez_mode == XL_EZ_NONE && m.kind == XL_MASK_SLM && q->nin == 1 && q->ncomp == 1 &&
+         !((m.forms & XL_PF_SCALAR) && q->gparam[0][0]);
+}
+
+int xl_rs_adjoint_pre(const xl_rs_params* p, const xl_pre_params* q, void* ws, size_t ws_bytes, void* stream) {
+  if (!p || !q) return fail(XL_EINVAL, "null params");
+  if (!p->adjoint) return fail(XL_EINVAL, "xl_rs_adjoint_pre takes an adjoint propagation");
+  if (q->rows != p->n || q->cols != p->n || q->ncomp != p->nin || q->comp_stride != p->out_comp_stride ||
+      q->gout != p->out)
+    return fail(XL_EINVAL, "the pre-op's plane and cotangent must be the propagation's output");
+  if (!rs_pre_fuses(p, q)) {
+    if (int rc = rs_run(p, nullptr, ws, ws_bytes, stream)) return rc;
+    return xl_pre_backward(q, stream);
+  }
+  xl::PreArgs a;
+  if (int rc = pre_common(q, &a)) return rc;
+  int blocks = 0;
+  const int P = rs_fft_len(p->n);
+  if (p->n < 2 || P > xl::MAX_FFT) return fail(XL_EINVAL, "grid side needs FFT length > 4096 or is below 2");
+  if (int rc = dispatch_q(P, [&](auto c) { blocks = xl::rs_final_pre_blocks<decltype(c)::value>(p->n); })) return rc;
+  if (q->ez_dz) {
+    if (q->ez_mode != XL_EZ_VRS) return fail(XL_EINVAL, "ez_dz is the XL_EZ_VRS construction's distance term");
+    if ((size_t)blocks + 1 > xl_pre_scalar_grad_elems(p->n, p->n)) return fail(XL_EINVAL, "ez_dz buffer too small");
+    a.ezdz = q->ez_dz;
+  }
+  if (int rc = rs_run(p, &a, ws, ws_bytes, stream)) return rc;
+  if (q->ez_dz) {
+    xl::KTimer t(xl::K_PRE_BWD, (hipStream_t)stream);
+    // (block 4 of pgrad_reduce_kernel's five sums, the others null)
+    hipLaunchKernelGGL(xl::pgrad_reduce_kernel, dim3(5), dim3(1024), 0, (hipStream_t)stream, nullptr, nullptr, nullptr,
+                       nullptr, q->ez_dz, q->ez_dz_base, blocks, std::max(1, (int)q->ez_dz_base_n));
+    return hip_check(hipGetLastError(), "distance-gradient reduction launch");
+  }
+  return XL_OK;
 }
 
 int xl_slm_backward_adam(const xl_pre_params* p, const xl_adam_params* ad, void* stream) {

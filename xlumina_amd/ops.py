@@ -339,7 +339,7 @@ def rs_propagate(src: torch.Tensor, x, y, z: float, wavelength: float, masks: Se
                  hhat: Optional[torch.Tensor] = None, hhat_mode: int = 0, noalloc: bool = False,
                  spec: Optional[torch.Tensor] = None, spec_mode: int = 0, spec_grads: int = 0,
                  grad_out: Optional[torch.Tensor] = None, quality_factor: Optional[torch.Tensor] = None,
-                 spec_dg: Optional[torch.Tensor] = None):
+                 spec_dg: Optional[torch.Tensor] = None, pre: Optional[dict] = None):
     """RS_propagation_jit / VRS_propagation_jit (wave_optics.py:281-289,
     vectorized_optics.py:364-373) with fused masks and Ez construction.
 
@@ -367,6 +367,11 @@ def rs_propagate(src: torch.Tensor, x, y, z: float, wavelength: float, masks: Se
     (with XL_RS_SPEC_PREBUILT) reads them there.
     quality_factor: optional 0-d float64 device tensor that the launch fills
     with the quality factor of the distance propagated (wave_optics.py:187-191).
+    pre: on an adjoint call, the arguments of pre_backward (src, masks, ez_mode,
+    nin, need_src, need_params, out, ez_dz, ez_dz_base; grid and distance are the
+    call's) for the pre-op adjoint of the propagated cotangent, which the last
+    pass takes on where it can (xl_rs_adjoint_pre): pre_backward's results are
+    returned instead of the field.
     noalloc: run on the library's own per-device scratch
     (xl_rs_propagate_noalloc, n <= 1024) instead of a workspace; with `out`
     (and `inten`) given the call allocates nothing.  Such calls share one
@@ -441,6 +446,20 @@ def rs_propagate(src: torch.Tensor, x, y, z: float, wavelength: float, masks: Se
         p.quality_factor, p.qf_rmax, p.qf_dr_real, p.qf_wavelength = (quality_factor.data_ptr(), float(rmax),
                                                                       float(dr_real), float(wavelength))
     keep = fill_masks(p.mask, masks, (n, n), dev, nin)
+    if pre is not None:
+        if noalloc or intensity or not adjoint:
+            raise ValueError("pre belongs to an adjoint call on a workspace")
+        psrc = _prep_field(pre["src"])
+        if tuple(psrc.shape[-2:]) != (n, n) or psrc.device != dev:
+            raise ValueError(f"the pre-op's source must be an {n} x {n} field on the cotangent's device")
+        pnin = pre["nin"]
+        q, pkeep = _pre_params(psrc, x, y, z, pre["masks"], pre["ez_mode"], False, ncomp, pnin, 0.0, 0.0, z_dev)
+        q.gout = out.data_ptr()
+        res = _pre_outputs(q, psrc, pnin, pre["need_src"], pre["need_params"], None, pre["out"], pre["ez_dz"],
+                           pre["ez_dz_base"])
+        N.check(lib.xl_rs_adjoint_pre(C.byref(p), C.byref(q), workspace.data_ptr(), workspace.numel(), _stream(dev)))
+        del keep, pkeep
+        return res
     if noalloc:
         N.check(lib.xl_rs_propagate_noalloc(C.byref(p), _stream(dev)))
     else:
@@ -849,13 +868,20 @@ def pre_backward(src: torch.Tensor, gout: torch.Tensor, x, y, z: float = 0.0, ma
     sum of the float64 device values `ez_dz_base` (fixed order) when given --
     one value, or the partial sums an adjoint propagation left in its spec
     buffer (rs_spec_partials)."""
-    lib = N.load()
     src = _prep_field(src)
     gout = _prep_field(gout)
     nin = src.shape[0] if nin is None else nin
-    ncomp = gout.shape[0]
-    p, keep = _pre_params(src, x, y, z, masks, ez_mode, hna, ncomp, nin, hna_radius, hna_f, z_dev)
+    p, keep = _pre_params(src, x, y, z, masks, ez_mode, hna, gout.shape[0], nin, hna_radius, hna_f, z_dev)
     p.gout = gout.data_ptr()
+    gsrc, gp = _pre_outputs(p, src, nin, need_src, need_params, gparams, out, ez_dz, ez_dz_base)
+    N.check(N.load().xl_pre_backward(C.byref(p), _stream(src.device)))
+    del keep
+    return gsrc, gp
+
+
+def _pre_outputs(p, src, nin, need_src, need_params, gparams, out, ez_dz, ez_dz_base):
+    """Output buffers of a pre-op adjoint, allocated or checked and set in p:
+    (gradient of src or None, [[g00, g01], [g10, g11]])."""
     rows, cols = src.shape[-2:]
     if out is not None and need_src:
         if (out.dtype != torch.complex64 or out.device != src.device or out.dim() != 3 or out.shape[0] < nin
@@ -897,8 +923,6 @@ def pre_backward(src: torch.Tensor, gout: torch.Tensor, x, y, z: float = 0.0, ma
                     or not ez_dz_base.is_contiguous()):
                 raise ValueError("ez_dz_base must be a contiguous float64 device tensor")
             p.ez_dz_base, p.ez_dz_base_n = ez_dz_base.data_ptr(), ez_dz_base.numel()
-    N.check(lib.xl_pre_backward(C.byref(p), _stream(src.device)))
-    del keep
     return gsrc, gp
 
 

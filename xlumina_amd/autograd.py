@@ -102,8 +102,8 @@ _SHARED_SPECTRA: dict = {}
 
 def _spectra_key(cfg: RSConfig, z_t, n: int, ncomp: int, dev):
     xd, yd = ops.device_grid(cfg.x, dev), ops.device_grid(cfg.y, dev)
-    zk = ("t", z_t.data_ptr(), z_t._version, str(z_t.device)) if z_t is not None else ("f", float(cfg.z))
-    key = (zk, xd.data_ptr(), yd.data_ptr(), n, ncomp, float(cfg.wavelength), str(dev))
+    zk = ("t", z_t.data_ptr(), z_t._version, z_t.device) if z_t is not None else ("f", float(cfg.z))
+    key = (zk, xd.data_ptr(), yd.data_ptr(), n, ncomp, float(cfg.wavelength), dev)
     return key, (None if z_t is None else z_t.detach(), xd, yd)
 
 
@@ -146,10 +146,7 @@ class _RSFunction(torch.autograd.Function):
         cfg.qf_out = None   # the backward's launches report nothing
         ctx.cfg = cfg
         ctx.spec_dg = spec_dg
-        ctx.save_for_backward(src, *[p if p is not None else torch.empty(0) for p in params],
-                              hhat if hhat is not None else torch.empty(0),
-                              spec if spec is not None else torch.empty(0))
-        ctx.has = [p is not None for p in params]
+        ctx.save_for_backward(src, *params, hhat, spec)
         ctx.z_meta = None if z_t is None else (z_t.shape, z_t.dtype, z_t.device)
         ctx.wl_meta = None if wl_t is None else (wl_t.shape, wl_t.dtype, wl_t.device)
         return out
@@ -157,11 +154,7 @@ class _RSFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gout):
         cfg = ctx.cfg
-        saved = ctx.saved_tensors
-        src = saved[0]
-        params = [saved[1 + i] if ctx.has[i] else None for i in range(4)]
-        hhat = saved[5] if saved[5].numel() else None
-        spec = saved[6] if saved[6].numel() else None
+        src, *params, hhat, spec = ctx.saved_tensors
         gout = gout.contiguous()
         want_z, want_wl = ctx.needs_input_grad[6], ctx.needs_input_grad[7]
         # with the VRS Ez_in term the pre-op adjoint's reduction also sums the
@@ -285,26 +278,10 @@ def _staged_tables(cfg: CZTConfig):
 
 
 def _czt_staged(share, attr: str, src, cfg: CZTConfig, **kw):
-    """ops.czt on the workspace share.<attr>: the first call stages the axis
+    """ops.czt on the workspace share.<attr>: the first call leaves the axis
     tables there, later calls with the same arguments use them."""
-    if share is None:
-        return ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, **kw)
-    ws = getattr(share, attr)
-    adjoint, ez_mode = kw.get("adjoint", False), kw.get("ez_mode", N.XL_EZ_NONE)
-    nin = kw.get("nin") or src.shape[-3]
-    ncomp = 3 if (ez_mode == N.XL_EZ_VCZT or cfg.mode == N.XL_CZT_HNA) and not adjoint else nin
-    if cfg.mode != cfg.geom.mode:
-        return ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, **kw)
-    try:
-        need = ops.czt_workspace_bytes(cfg.geom, ncomp=ncomp, nin=nin, adjoint=adjoint, ez_mode=ez_mode)
-    except ValueError:
-        return ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, **kw)   # raises with the plan error
-    if ws is not None and ws.numel() >= need and ws.device == src.device:
-        return ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, workspace=ws, tables_mode=2, **kw)
-    ws = torch.empty(need, dtype=torch.uint8, device=src.device)
-    ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, workspace=ws, tables_mode=1, **kw)   # stage only
-    setattr(share, attr, ws)
-    return ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, workspace=ws, tables_mode=2, **kw)
+    staged = (share, attr) if share is not None and cfg.mode == cfg.geom.mode else None
+    return ops.czt(src, cfg.geom, mode=cfg.mode, form=cfg.form, staged=staged, **kw)
 
 
 class _CZTFunction(torch.autograd.Function):
@@ -318,9 +295,7 @@ class _CZTFunction(torch.autograd.Function):
         ctx.tables = share
         ctx.cfg = cfg
         keep_out = (z_t is not None and ctx.needs_input_grad[6]) or (wl_t is not None and ctx.needs_input_grad[7])
-        ctx.save_for_backward(src, *[p if p is not None else torch.empty(0) for p in params],
-                              out if keep_out else torch.empty(0))
-        ctx.has = [p is not None for p in params]
+        ctx.save_for_backward(src, *params, out if keep_out else None)
         ctx.z_meta = None if z_t is None else (z_t.shape, z_t.dtype, z_t.device)
         ctx.wl_meta = None if wl_t is None else (wl_t.shape, wl_t.dtype, wl_t.device)
         return out
@@ -329,21 +304,19 @@ class _CZTFunction(torch.autograd.Function):
     def backward(ctx, gout):
         cfg = ctx.cfg
         g = cfg.geom
-        saved = ctx.saved_tensors
-        src = saved[0]
-        params = [saved[1 + i] if ctx.has[i] else None for i in range(4)]
+        src, *params, kept_out = ctx.saved_tensors
         g_pre = _czt_staged(ctx.tables, "adj", gout.contiguous(), cfg, adjoint=True)
         masks = _rebuild(cfg.mask_struct, params)
         hna = cfg.mode == N.XL_CZT_HNA
         g_z = None
         if ctx.z_meta is not None and ctx.needs_input_grad[6]:
             shape, dtype, device = ctx.z_meta
-            g_z = _czt_z_grad(cfg, src, masks, gout.contiguous(), g_pre, saved[5]).to(device=device, dtype=dtype)
+            g_z = _czt_z_grad(cfg, src, masks, gout.contiguous(), g_pre, kept_out).to(device=device, dtype=dtype)
             g_z = g_z.reshape(shape)
         g_wl = None
         if ctx.wl_meta is not None and ctx.needs_input_grad[7]:
             shape, dtype, device = ctx.wl_meta
-            g_wl = _czt_z_grad(cfg, src, masks, gout.contiguous(), g_pre, saved[5], wrt="wavelength")
+            g_wl = _czt_z_grad(cfg, src, masks, gout.contiguous(), g_pre, kept_out, wrt="wavelength")
             g_wl = g_wl.to(device=device, dtype=dtype).reshape(shape)
         need_params = ((ctx.needs_input_grad[2] and params[0] is not None, ctx.needs_input_grad[3] and params[1] is not None),
                        (ctx.needs_input_grad[4] and params[2] is not None, ctx.needs_input_grad[5] and params[3] is not None))
@@ -501,16 +474,13 @@ class _PreFunction(torch.autograd.Function):
         out = ops.pre_forward(src, cfg.x, cfg.y, cfg.z, masks=masks, ez_mode=cfg.ez_mode, hna=cfg.hna,
                               ncomp=cfg.ncomp, nin=cfg.nin, hna_radius=cfg.hna_radius, hna_f=cfg.hna_f)
         ctx.cfg = cfg
-        ctx.save_for_backward(src, *[p if p is not None else torch.empty(0) for p in params])
-        ctx.has = [p is not None for p in params]
+        ctx.save_for_backward(src, *params)
         return out
 
     @staticmethod
     def backward(ctx, gout):
         cfg = ctx.cfg
-        saved = ctx.saved_tensors
-        src = saved[0]
-        params = [saved[1 + i] if ctx.has[i] else None for i in range(4)]
+        src, *params = ctx.saved_tensors
         masks = _rebuild(cfg.mask_struct, params)
         need_params = ((ctx.needs_input_grad[2] and params[0] is not None, ctx.needs_input_grad[3] and params[1] is not None),
                        (ctx.needs_input_grad[4] and params[2] is not None, ctx.needs_input_grad[5] and params[3] is not None))

@@ -70,26 +70,46 @@ def content_key(b: bytes):
 
 
 _grid_cache: dict = {}
-_grid_ids: dict = {}   # (id(array), device) -> (weak reference, its bytes, device copy)
+_grid_ids: dict = {}   # (id(array), device) -> (weak reference, its bytes, GridInfo)
+
+
+class GridInfo:
+    """What a call needs of a 1-D grid: its float64 device copy, its length and
+    its first step."""
+    __slots__ = ("t", "n", "step")
+
+    def __init__(self, t: torch.Tensor, host: np.ndarray):
+        self.t = t
+        self.n = int(host.size)
+        self.step = float(host[1] - host[0]) if host.size > 1 else 0.0
+
+
+def grid_info(arr, device) -> GridInfo:
+    """GridInfo of a 1-D grid, cached by content (a grid array seen before is
+    recognised by identity and a comparison of its bytes)."""
+    host = arr
+    if isinstance(arr, torch.Tensor):
+        host = arr.detach().cpu().numpy()
+        if arr.device == device and arr.dtype == torch.float64 and arr.is_contiguous():
+            return GridInfo(arr, np.asarray(host, dtype=np.float64).ravel())
+    ident = isinstance(host, np.ndarray)
+    if ident:
+        ent = _grid_ids.get((id(host), device))
+        if ent is not None and ent[0]() is host and ent[1] == host.tobytes():
+            return ent[2]
+    info = GridInfo(_device_grid_by_content(host, device), np.asarray(host, dtype=np.float64).ravel())
+    if ident:
+        if len(_grid_ids) > 256:
+            _grid_ids.clear()
+        _grid_ids[(id(host), device)] = (weakref.ref(host), host.tobytes(), info)
+    return info
 
 
 def device_grid(arr, device) -> torch.Tensor:
-    """float64 device copy of a 1-D grid, cached by content (a grid array
-    seen before is recognised by identity and a comparison of its bytes)."""
-    if isinstance(arr, torch.Tensor):
-        if arr.device == device and arr.dtype == torch.float64 and arr.is_contiguous():
-            return arr
-        arr = arr.detach().cpu().numpy()
-    if isinstance(arr, np.ndarray):
-        ent = _grid_ids.get((id(arr), device))
-        if ent is not None and ent[0]() is arr and ent[1] == arr.tobytes():
-            return ent[2]
-    t = _device_grid_by_content(arr, device)
-    if isinstance(arr, np.ndarray):
-        if len(_grid_ids) > 256:
-            _grid_ids.clear()
-        _grid_ids[(id(arr), device)] = (weakref.ref(arr), arr.tobytes(), t)
-    return t
+    """float64 device copy of a 1-D grid (see grid_info); a tensor that is one already is returned as it is."""
+    if isinstance(arr, torch.Tensor) and arr.device == device and arr.dtype == torch.float64 and arr.is_contiguous():
+        return arr
+    return grid_info(arr, device).t
 
 
 def _device_grid_by_content(arr, device) -> torch.Tensor:
@@ -158,15 +178,10 @@ def fill_masks(dst, masks: Sequence[MaskSpec], shape, device, nin: int, batch: O
     if batch is not None:
         return _fill_masks_batched(dst, masks, shape, device, batch)
     keep = []
-    for i in range(2):
+    for i, m in enumerate(masks):
+        if m is None:
+            continue   # (a new parameter struct's slots are zero: XL_MASK_NONE)
         st = dst[i]
-        if i >= len(masks) or masks[i] is None:
-            st.kind = N.XL_MASK_NONE
-            st.forms = 0
-            st.m0 = st.m1 = None
-            st.s0 = st.s1 = 0.0
-            continue
-        m = masks[i]
         p0, f0 = _param_with_form(m.p0, shape, device, bool(m.unit & 1), allow_f64)
         p1, f1 = _param_with_form(m.p1, shape, device, bool(m.unit & 2), allow_f64)
         keep += [p0, p1]
@@ -285,10 +300,6 @@ def check_rs_args(src_shape, nin: int, ncomp: int, nx: int, ny: int, out, inten,
         check_buffer(inten, (n, n), torch.float32, dev, "inten")
 
 
-def _grid_len(g) -> int:
-    return int(g.numel()) if isinstance(g, torch.Tensor) else len(np.asarray(g).ravel())
-
-
 def _z_ptr(z_dev: Optional[torch.Tensor], dev):
     if z_dev is None:
         return None
@@ -385,9 +396,9 @@ def rs_propagate(src: torch.Tensor, x, y, z: float, wavelength: float, masks: Se
         raise ValueError("RS propagation needs a square grid (the reference builds one lag vector for both axes)")
     nin = src.shape[0] if nin is None else nin
     ncomp = 3 if ez_mode == N.XL_EZ_VRS else nin
-    check_rs_args(tuple(src.shape), nin, ncomp, _grid_len(x), _grid_len(y), out, inten if intensity else None, dev)
+    gx, gy = grid_info(x, dev), grid_info(y, dev)
+    check_rs_args(src.shape, nin, ncomp, gx.n, gy.n, out, inten if intensity else None, dev)
     check_workspace(workspace, dev)
-    xd, yd = device_grid(x, dev), device_grid(y, dev)
     if out is None:
         out = torch.empty((ncomp, n, n), dtype=torch.complex64, device=dev)
     if intensity and inten is None:
@@ -413,14 +424,12 @@ def rs_propagate(src: torch.Tensor, x, y, z: float, wavelength: float, masks: Se
     p.intensity = _ptr(inten) or None
     p.n = n
     p.adjoint = 1 if adjoint else 0
-    p.x = xd.data_ptr()
-    p.y = yd.data_ptr()
+    p.x = gx.t.data_ptr()
+    p.y = gy.t.data_ptr()
     p.z = float(z)
     p.k = 2 * math.pi / wavelength
-    xa = np.asarray(x, dtype=np.float64) if not isinstance(x, torch.Tensor) else x.detach().cpu().double().numpy()
-    ya = np.asarray(y, dtype=np.float64) if not isinstance(y, torch.Tensor) else y.detach().cpu().double().numpy()
-    p.dx = float(xa[1] - xa[0])
-    p.dy = float(ya[1] - ya[0])
+    p.dx = gx.step
+    p.dy = gy.step
     p.z_dev = _z_ptr(z_dev, dev)
     p.kernel_dz = int(kernel_dz)
     if hhat_mode:
@@ -509,7 +518,8 @@ def rs_propagate_batched(src: torch.Tensor, x, y, wavelength: float, z_dev: torc
     ncin = src.shape[-3]
     nin = ncin if nin is None else nin
     ncomp = 3 if ez_mode == N.XL_EZ_VRS else nin
-    check_rs_args((ncin, n, n), nin, ncomp, _grid_len(x), _grid_len(y), None, None, dev)
+    gx, gy = grid_info(x, dev), grid_info(y, dev)
+    check_rs_args((ncin, n, n), nin, ncomp, gx.n, gy.n, None, None, dev)
     if (not isinstance(z_dev, torch.Tensor) or z_dev.dtype != torch.float64 or z_dev.device != dev
             or z_dev.numel() != batch or not z_dev.is_contiguous()):
         raise ValueError(f"z_dev must be a contiguous float64 tensor of {batch} distances on the field's device")
@@ -526,7 +536,6 @@ def rs_propagate_batched(src: torch.Tensor, x, y, wavelength: float, z_dev: torc
     need = rs_batch_workspace_bytes(n, ncomp, batch)
     if workspace is None or workspace.numel() < need:
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-    xd, yd = device_grid(x, dev), device_grid(y, dev)
     p = N.RsParams()
     p.inp = src.data_ptr()
     p.in_comp_stride = n * n
@@ -537,12 +546,9 @@ def rs_propagate_batched(src: torch.Tensor, x, y, wavelength: float, z_dev: torc
     p.intensity = _ptr(inten) or None
     p.n = n
     p.adjoint = 1 if adjoint else 0
-    p.x, p.y = xd.data_ptr(), yd.data_ptr()
+    p.x, p.y = gx.t.data_ptr(), gy.t.data_ptr()
     p.k = 2 * math.pi / wavelength
-    xa = np.asarray(x, dtype=np.float64) if not isinstance(x, torch.Tensor) else x.detach().cpu().double().numpy()
-    ya = np.asarray(y, dtype=np.float64) if not isinstance(y, torch.Tensor) else y.detach().cpu().double().numpy()
-    p.dx = float(xa[1] - xa[0])
-    p.dy = float(ya[1] - ya[0])
+    p.dx, p.dy = gx.step, gy.step
     p.z = 0.0
     p.z_dev = z_dev.data_ptr()
     if hhat_mode:
@@ -591,6 +597,8 @@ class CztGeometry:
 def _f64(a) -> np.ndarray:
     if isinstance(a, torch.Tensor):
         a = a.detach().cpu().numpy()
+    if type(a) is np.ndarray and a.dtype == np.float64 and a.ndim == 1 and a.flags.c_contiguous:
+        return a   # (itself: its device copy is found by identity)
     return np.ascontiguousarray(np.asarray(a, dtype=np.float64).ravel())
 
 
@@ -681,7 +689,7 @@ def resolve_czt_form(g: "CztGeometry", form: Optional[str] = None, ncomp: int = 
 def czt(src: torch.Tensor, g: CztGeometry, masks: Sequence[MaskSpec] = (), ez_mode: int = N.XL_EZ_NONE,
         nin: Optional[int] = None, ncomp: Optional[int] = None, adjoint: bool = False, mode: Optional[int] = None,
         out: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
-        form: Optional[str] = None, batch: Optional[int] = None, tables_mode: int = 0) -> torch.Tensor:
+        form: Optional[str] = None, batch: Optional[int] = None, tables_mode: int = 0, staged=None) -> torch.Tensor:
     """CZT_jit / VCZT_jit / CZT_for_high_NA_jit / VCZT_objective_lens core.
 
     Forward: src (C, ny, nx) -> (ncomp, my, mx).  Adjoint: src (ncomp, my, mx)
@@ -694,6 +702,10 @@ def czt(src: torch.Tensor, g: CztGeometry, masks: Sequence[MaskSpec] = (), ez_mo
     axis tables into the workspace (src and out are not touched), 2 uses the
     tables a mode-1 call with the same arguments staged there (a mode-0 call
     with a caller workspace leaves the same tables there too).
+    `staged` (Bluestein form): (object, attribute) that holds such a workspace
+    between calls of one geometry and direction: the tables in it are used where
+    it is there and large enough, otherwise this call makes it and leaves its
+    tables there.
     """
     if batch is not None:
         return _czt_batched(src, g, masks, ez_mode, nin, ncomp, adjoint, mode, out, workspace, batch)
@@ -727,9 +739,17 @@ def czt(src: torch.Tensor, g: CztGeometry, masks: Sequence[MaskSpec] = (), ez_mo
             raise ValueError("staged CZT tables need the Bluestein form and a caller workspace of "
                              "czt_workspace_bytes")
         p.tables_mode = int(tables_mode)
-    if workspace is None or workspace.numel() < need:
+    if staged is not None and not use_gemm:
+        workspace = getattr(*staged)
+        if workspace is not None and workspace.numel() >= need and workspace.device == dev:
+            p.tables_mode = 2
+        else:
+            workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+    elif workspace is None or workspace.numel() < need:
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     N.check(runfn(C.byref(p), workspace.data_ptr(), workspace.numel(), _stream(dev)))
+    if staged is not None and not use_gemm and not p.tables_mode:
+        setattr(*staged, workspace)
     del keep
     return out
 

@@ -32,18 +32,34 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // grid (kMseBlocks, batch): partial[b][blk] = sum over the block's pixels of
-// (|E|^2 - T)^2, accumulated in a fixed order.
+// (|E|^2 - T)^2, accumulated in a fixed order.  kMseUnroll pixels' loads are in
+// flight together (8 x 1024^2 with the gradient, 134 MB: one 30.2 us, four 24.5).
+constexpr int kMseUnroll = 4;
 __global__ __launch_bounds__(kMseThreads) void mse_kernel(MseArgs a) {
   const int b = blockIdx.y;
   const float2* e = a.field + (int64_t)b * a.fbs;
   float2* g = a.grad ? a.grad + (int64_t)b * a.gbs : nullptr;
   float acc = 0.f;
-  for (int64_t p = (int64_t)blockIdx.x * kMseThreads + threadIdx.x; p < a.npix;
-       p += (int64_t)gridDim.x * kMseThreads) {
-    const float2 v = e[p];
-    const float d = v.x * v.x + v.y * v.y - a.target[p];
-    acc += d * d;
-    if (g) g[p] = make_float2(a.gscale * d * v.x, a.gscale * d * v.y);
+  const int64_t stride = (int64_t)gridDim.x * kMseThreads;
+  for (int64_t p = (int64_t)blockIdx.x * kMseThreads + threadIdx.x; p < a.npix; p += kMseUnroll * stride) {
+    float2 v[kMseUnroll];
+    float t[kMseUnroll];
+#pragma unroll
+    for (int u = 0; u < kMseUnroll; ++u) {
+      const int64_t q = p + u * stride;
+      if (q < a.npix) {
+        v[u] = e[q];
+        t[u] = a.target[q];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kMseUnroll; ++u) {
+      const int64_t q = p + u * stride;
+      if (q >= a.npix) break;
+      const float d = v[u].x * v[u].x + v[u].y * v[u].y - t[u];
+      acc += d * d;
+      if (g) g[q] = make_float2(a.gscale * d * v[u].x, a.gscale * d * v[u].y);
+    }
   }
   __shared__ float red[kMseThreads / 64];
   acc = wave_sum(acc);

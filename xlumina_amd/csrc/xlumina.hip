@@ -1312,7 +1312,9 @@ int xl_beam_splitter(const xl_bs_params* p, void* stream) {
   a.adjoint = p->adjoint ? 1 : 0;
   hipStream_t st = (hipStream_t)stream;
   xl::KTimer t(xl::K_BS, st);
-  const int64_t blocks = std::min<int64_t>((p->npix + 255) / 256, 4096);
+  // one pixel a thread while that leaves CUs without a block, kBsUnroll from 512 blocks a plane on
+  const int64_t per = 256 * xl::kBsUnroll, one = (p->npix + 255) / 256;
+  const int64_t blocks = std::min<int64_t>(std::max<int64_t>((p->npix + per - 1) / per, std::min<int64_t>(one, 512)), 2048);
   hipLaunchKernelGGL(xl::bs_kernel, dim3((unsigned)blocks, a.zero_ez ? 3 : 2), dim3(256), 0, st, a);
   return hip_check(hipGetLastError(), "beam splitter launch");
 }

@@ -6,7 +6,8 @@ operator run by the same kernels:
     correlation is a convolution with the conjugated transform);
   * CZT / VCZT / high-NA: conj(F) (K_y^H (conj(F0 c) G) conj(K_x)) through the
     Bluestein kernels with adjoint tables;
-  * fused Jones masks / Ez construction / lens map: xl_pre_backward, which
+  * fused Jones masks / Ez construction / lens map: xl_pre_backward (for RS / VRS
+    with the propagation's adjoint in one call, xl_rs_adjoint_pre), which
     also returns the cotangents of the per-pixel mask parameters.
 Only the inputs (field, mask parameters) are saved; masked intermediates are
 recomputed in the backward pass, so a chain keeps one field per stage alive.

@@ -560,7 +560,9 @@ int xl_czt(const xl_czt_params* p, void* ws, size_t ws_bytes, void* stream) {
     ax.zl = (ap.q & (ap.q - 1)) == 0 && 2 * std::max(ap.m, ap.M) <= ap.q;
   }
   if (p->tables_mode < 0 || p->tables_mode > 2) return fail(XL_EINVAL, "tables_mode must be 0, 1 or 2");
-  if (p->tables_mode != 2) {
+  // a batch's factor tables are built beside the axis tables where those need one launch
+  const bool joint = cp.ftab && p->tables_mode == 0 && cp.x.q == cp.y.q;
+  if (p->tables_mode != 2 && !joint) {
     if (cp.x.q == cp.y.q) {
       if (int rc = dispatch_czt_q(cp.x.q, [&](auto c) { xl::czt_setup_launch<decltype(c)::value>(pair, 2, st); }))
         return rc;
@@ -610,8 +612,16 @@ int xl_czt(const xl_czt_params* p, void* ws, size_t ws_bytes, void* stream) {
   if (cp.ftab) {
     float2* ft = (float2*)align256((char*)(tiles + cp.tiles_bytes / sizeof(float2)));
     float2* f0 = ft + (size_t)cp.rin * cp.lin_x;
-    xl::KTimer t(xl::K_CZT_SETUP, st);
-    hipLaunchKernelGGL(xl::czt_ftab_kernel, grid_for(cp.ftab_bytes / sizeof(float2)), dim3(256), 0, st, a, ft, f0);
+    const int64_t elems = cp.ftab_bytes / sizeof(float2);
+    if (joint) {
+      if (int rc = dispatch_q(cp.x.q, [&](auto c) {
+            xl::czt_setup_ftab_launch<decltype(c)::value>(pair, a, ft, f0, elems, st);
+          }))
+        return rc;
+    } else {
+      xl::KTimer t(xl::K_CZT_SETUP, st);
+      hipLaunchKernelGGL(xl::czt_ftab_kernel, grid_for(elems), dim3(256), 0, st, a, ft, f0);
+    }
     a.ftab = ft;
     a.f0tab = f0;
   }

@@ -102,10 +102,17 @@ _SHARED_SPECTRA: dict = {}
 
 
 def _spectra_key(cfg: RSConfig, z_t, n: int, ncomp: int, dev):
+    """(key, the key's tensors).  The distance and a grid that the caller holds
+    on the device (it is used as it is) count as unchanged by address and
+    version; the key is None where a version is not tracked (inference tensors)."""
     xd, yd = ops.device_grid(cfg.x, dev), ops.device_grid(cfg.y, dev)
-    zk = ("t", z_t.data_ptr(), z_t._version, z_t.device) if z_t is not None else ("f", float(cfg.z))
-    key = (zk, xd.data_ptr(), yd.data_ptr(), n, ncomp, float(cfg.wavelength), dev)
-    return key, (None if z_t is None else z_t.detach(), xd, yd)
+    keep = (None if z_t is None else z_t.detach(), xd, yd)
+    held = [t for t in (z_t, cfg.x if cfg.x is xd else None, cfg.y if cfg.y is yd else None) if t is not None]
+    if any(t.is_inference() for t in held):
+        return None, keep
+    zk = ("t", z_t.data_ptr(), z_t.device) if z_t is not None else ("f", float(cfg.z))
+    key = (zk, xd.data_ptr(), yd.data_ptr(), *(t._version for t in held), n, ncomp, float(cfg.wavelength), dev)
+    return key, keep
 
 
 class _RSFunction(torch.autograd.Function):
@@ -124,7 +131,7 @@ class _RSFunction(torch.autograd.Function):
         key = None
         if any(ctx.needs_input_grad[1:]):
             key, keep = _spectra_key(cfg, z_t, n, ncomp, src.device)
-            hit = _SHARED_SPECTRA.get(key)
+            hit = _SHARED_SPECTRA.get(key) if key is not None else None
             if hit is not None and hit["hhat"]() is not None:
                 # an earlier propagation over this distance built the spectra
                 hhat, hhat_mode = hit["hhat"](), 2

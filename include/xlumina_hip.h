@@ -244,6 +244,9 @@ int xl_max_fft_length(void);
 /* Builds the float64-generated twiddle table on the current device (called
  * once per device before any other call; later calls are no-ops). */
 int xl_init(void);
+/* Id of the graph capture that `stream` records into, 0 when it records none:
+ * work recorded into one capture has not run before its graph is replayed. */
+int xl_capture_id(void* stream, uint64_t* id);
 
 /* RS_propagation_jit (wave_optics.py:281-289), VRS_propagation_jit
  * (vectorized_optics.py:364-373) with Jones masks / Ez construction fused. */

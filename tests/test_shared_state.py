@@ -1,6 +1,8 @@
 """State that differentiated propagations share: kernel spectra by grid and
 distance, CZT tables by geometry.  What may be shared, and what may not.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -9,6 +11,7 @@ from oracle import xlumina_ref as R
 from tests.conftest import rel_l2
 from xlumina_amd import _native as N
 from xlumina_amd import autograd as AG
+from xlumina_amd import ops
 
 CPU = torch.device("cpu")
 
@@ -33,6 +36,88 @@ def test_spectra_of_untracked_grids_are_not_shared():
     with torch.inference_mode():
         x = torch.linspace(-8.0, 8.0, 16, dtype=torch.float64)
     assert AG._spectra_key(_rs_config(x), None, 16, 1, CPU)[0] is None
+
+
+def test_spectra_key_follows_the_launch_scope(monkeypatch):
+    x = torch.linspace(-8.0, 8.0, 16, dtype=torch.float64)
+    keys = []
+    for scope in ((0, 0), (1, 0), (1, 7), (1, 8), (2, 0)):   # (stream, graph capture)
+        monkeypatch.setattr(ops, "launch_scope", lambda dev: scope, raising=False)
+        keys.append(AG._spectra_key(_rs_config(x), None, 16, 1, CPU)[0])
+    assert len(set(keys)) == len(keys)
+
+
+def test_capture_id_of_the_default_stream():
+    assert ops.launch_scope(CPU) == (0, 0)
+    cid = ctypes.c_uint64(5)
+    N.check(N.load().xl_capture_id(None, ctypes.byref(cid)))
+    assert cid.value == 0
+    with pytest.raises(ValueError):
+        N.check(N.load().xl_capture_id(None, None))
+
+
+def _c64(gen, *shape):
+    return torch.view_as_complex(torch.randn((*shape, 2), generator=gen, device=gen.device))
+
+
+@pytest.mark.gpu
+def test_propagations_on_two_streams_build_their_own_spectra(cuda_dev):
+    """Forward and adjoint on two streams at once: the bits of the same calls
+    one after the other."""
+    n = 160
+    x = np.linspace(-150.0, 150.0, n)
+    gen = torch.Generator(device=cuda_dev).manual_seed(5)
+    src, w = _c64(gen, 2, 1, n, n), torch.rand((2, n, n), generator=gen, device=cuda_dev)
+
+    def step(i):
+        s = src[i].clone().requires_grad_(True)
+        out = AG.rs(s, x, x, 700.0, 0.65)
+        return out, torch.autograd.grad((w[i] * out.abs() ** 2).sum(), s, retain_graph=True)[0]
+
+    AG._SHARED_SPECTRA.clear()
+    one = [step(i) for i in range(2)]
+    assert len(AG._SHARED_SPECTRA) == 1
+    torch.cuda.synchronize()
+    AG._SHARED_SPECTRA.clear()
+    streams = [torch.cuda.Stream(cuda_dev) for _ in range(2)]
+    two = []
+    for i, st in enumerate(streams):
+        with torch.cuda.stream(st):
+            two.append(step(i))
+    assert len(AG._SHARED_SPECTRA) == 2
+    torch.cuda.synchronize()
+    for (a, ga), (b, gb) in zip(one, two):
+        assert torch.equal(a.detach(), b.detach()) and torch.equal(ga, gb)
+
+
+@pytest.mark.gpu
+def test_captured_propagation_builds_its_own_spectra(cuda_dev):
+    """A step captured while an eager step's output over the same distance is
+    alive on the capture's stream, replayed after that output and its memory
+    are gone: the eager values, each time."""
+    n = 96
+    x = np.linspace(-150.0, 150.0, n)
+    gen = torch.Generator(device=cuda_dev).manual_seed(6)
+    src = _c64(gen, 1, n, n).requires_grad_(True)
+    st = torch.cuda.Stream(cuda_dev)
+    st.wait_stream(torch.cuda.current_stream(cuda_dev))
+    with torch.cuda.stream(st):
+        eager = AG.rs(src, x, x, 700.0, 0.65)
+        ref = eager.detach().clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        out = AG.rs(src, x, x, 700.0, 0.65)
+    del eager
+    for _ in range(3):
+        junk = torch.full((64 << 20,), float("nan"), device=cuda_dev)   # takes what the eager step held
+        with torch.cuda.stream(st):
+            side = torch.full((4 << 20,), float("nan"), device=cuda_dev)
+            out.detach().zero_()
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.detach(), ref)
+        del junk, side
 
 
 @pytest.mark.gpu

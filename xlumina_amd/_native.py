@@ -141,6 +141,7 @@ SIGNATURES = {
     "xl_abi_version": (C.c_int, []),
     "xl_max_fft_length": (C.c_int, []),
     "xl_init": (C.c_int, []),
+    "xl_capture_id": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64)]),
     "xl_rs_workspace_bytes": (C.c_size_t, [C.c_int32, C.c_int32]),
     "xl_rs_batch_workspace_bytes": (C.c_size_t, [C.c_int32, C.c_int32, C.c_int32]),
     "xl_rs_hhat_bytes": (C.c_size_t, [C.c_int32]),

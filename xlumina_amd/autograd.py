@@ -93,9 +93,9 @@ class RSConfig:
 
 
 # Kernel and derivative spectra of the differentiated forward propagations,
-# by geometry and distance: a later propagation over the same distance (one
-# distance tensor, unchanged, or one float) reuses them instead of building
-# its own.  An entry holds its key's tensors (so their addresses cannot be
+# by geometry, distance and launch scope: a later propagation over the same
+# distance (one distance tensor, unchanged, or one float) on the same stream
+# reuses them instead of building its own.  An entry holds its key's tensors (so their addresses cannot be
 # reused by others while it lives) and weak references to the spectra, which
 # live as long as the first propagation's saved state.
 _SHARED_SPECTRA: dict = {}
@@ -111,7 +111,8 @@ def _spectra_key(cfg: RSConfig, z_t, n: int, ncomp: int, dev):
     if any(t.is_inference() for t in held):
         return None, keep
     zk = ("t", z_t.data_ptr(), z_t.device) if z_t is not None else ("f", float(cfg.z))
-    key = (zk, xd.data_ptr(), yd.data_ptr(), *(t._version for t in held), n, ncomp, float(cfg.wavelength), dev)
+    key = (zk, xd.data_ptr(), yd.data_ptr(), *(t._version for t in held), n, ncomp, float(cfg.wavelength), dev,
+           ops.launch_scope(dev))
     return key, keep
 
 
@@ -132,9 +133,10 @@ class _RSFunction(torch.autograd.Function):
         if any(ctx.needs_input_grad[1:]):
             key, keep = _spectra_key(cfg, z_t, n, ncomp, src.device)
             hit = _SHARED_SPECTRA.get(key) if key is not None else None
-            if hit is not None and hit["hhat"]() is not None:
+            hhat = hit["hhat"]() if hit is not None else None
+            if hhat is not None:
                 # an earlier propagation over this distance built the spectra
-                hhat, hhat_mode = hit["hhat"](), 2
+                hhat_mode = 2
                 if spec_grads and (spec_grads & ~hit["bits"]) == 0 and hit["spec"] is not None:
                     spec_dg = hit["spec"]()
                 key = None

@@ -313,6 +313,17 @@ int xl_abi_version(void) { return 10; }
 int xl_max_fft_length(void) { return xl::MAX_FFT; }
 int xl_init(void) { return ensure_init(); }
 
+int xl_capture_id(void* stream, uint64_t* id) {
+  if (!id) return fail(XL_EINVAL, "null id");
+  *id = 0;
+  if (!stream) return XL_OK;   // the default stream records no capture
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  unsigned long long v = 0;
+  if (int rc = hip_check(hipStreamGetCaptureInfo((hipStream_t)stream, &cs, &v), "capture query")) return rc;
+  if (cs != hipStreamCaptureStatusNone) *id = v;
+  return XL_OK;
+}
+
 size_t xl_rs_hhat_bytes(int32_t n) {
   if (n < 2) return 0;
   const int64_t P = rs_fft_len(n);

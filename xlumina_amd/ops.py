@@ -56,6 +56,20 @@ def _stream(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def launch_scope(device):
+    """(stream, graph capture) that a launch on `device` goes to now.  What one
+    launch writes is there for a later one of the same scope: other streams do
+    not wait for it, and a capture's launches run when its graph is replayed."""
+    if device.type != "cuda":
+        return 0, 0
+    stream = _stream(device)
+    if not stream:
+        return 0, 0
+    cid = C.c_uint64()
+    N.check(N.load().xl_capture_id(stream, C.byref(cid)))
+    return stream, cid.value
+
+
 try:
     from xxhash import xxh3_64_intdigest as _digest
 except ImportError:

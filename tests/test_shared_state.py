@@ -2,6 +2,7 @@
 distance, CZT tables by geometry.  What may be shared, and what may not.
 """
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -118,6 +119,68 @@ def test_captured_propagation_builds_its_own_spectra(cuda_dev):
         torch.cuda.synchronize()
         assert torch.equal(out.detach(), ref)
         del junk, side
+
+
+def _czt_config(n=16):
+    x = np.linspace(-100.0, 100.0, n)
+    xo = np.linspace(-9.0, 9.0, 10)
+    return AG.CZTConfig(ops.czt_geometry(x, x, xo, xo, 3e4, 0.65), N.XL_EZ_NONE, 1, N.XL_CZT_RS)
+
+
+def test_staged_tables_follow_the_launch_scope_and_thread(monkeypatch):
+    shares = [AG._staged_tables(_czt_config(), CPU)]
+    assert AG._staged_tables(_czt_config(), CPU) is shares[0]
+    for scope in ((1, 0), (1, 7), (2, 0)):
+        monkeypatch.setattr(ops, "launch_scope", lambda dev: scope)
+        shares.append(AG._staged_tables(_czt_config(), CPU))
+    worker = threading.Thread(target=lambda: shares.append(AG._staged_tables(_czt_config(), CPU)))
+    worker.start()
+    worker.join()
+    assert len({id(s) for s in shares}) == 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["streams", "threads"])
+def test_zooms_of_one_geometry_at_once(cuda_dev, how):
+    """Differentiated zooms of one geometry on two streams, and from two
+    threads on one stream: the bits of the same calls one after the other."""
+    n, m = 300, 200
+    x = np.linspace(-900.0, 900.0, n)
+    xo = np.linspace(-90.0, 90.0, m)
+    gen = torch.Generator(device=cuda_dev).manual_seed(8)
+    src, w = _c64(gen, 2, 2, n, n), torch.rand((2, m, m), generator=gen, device=cuda_dev)
+
+    def forward(i):
+        s = src[i].clone().requires_grad_(True)
+        geom = ops.czt_geometry(x, x, xo, xo, 3e4, 0.65)
+        return s, [AG.czt(s, geom, nin=2, form="bluestein") for _ in range(4)]
+
+    def step(i):
+        s, outs = forward(i)
+        return [o.detach() for o in outs], torch.autograd.grad(sum((w[i] * o.abs() ** 2).sum() for o in outs), s)[0]
+
+    ref = [step(i) for i in range(2)]
+    torch.cuda.synchronize()
+    got = [None, None]
+
+    def on(i, st):
+        with torch.cuda.stream(st):
+            got[i] = step(i)
+
+    if how == "streams":
+        streams = [torch.cuda.Stream(cuda_dev) for _ in range(2)]
+        for i in range(2):
+            on(i, streams[i])
+    else:
+        st = torch.cuda.Stream(cuda_dev)
+        workers = [threading.Thread(target=on, args=(i, st)) for i in range(2)]
+        for t in workers:
+            t.start()
+        for t in workers:
+            t.join()
+    torch.cuda.synchronize()
+    for (outs, g), (outs2, g2) in zip(ref, got):
+        assert all(torch.equal(a, b) for a, b in zip(outs, outs2)) and torch.equal(g, g2)
 
 
 @pytest.mark.gpu

@@ -15,6 +15,7 @@ recomputed in the backward pass, so a chain keeps one field per stage alive.
 from __future__ import annotations
 
 import math
+import threading
 import weakref
 from dataclasses import dataclass, field
 from typing import Optional, Sequence, Tuple
@@ -257,7 +258,11 @@ class _StagedTables:
     spectra, functions of the geometry only) of one CZT geometry: one for the
     forward calls, one for the adjoints.  Every differentiated call of the
     geometry holds it, so it lives until the last of their backward passes;
-    the first call of each direction stages the tables, the others use them."""
+    the first call of each direction stages the tables, the others use them.
+    A workspace also holds the intermediate of each call that runs on it, so
+    only calls that run one after the other have it in common: one launch
+    scope, and for the forward calls one thread (the adjoints of a device run
+    on its one backward thread)."""
     __slots__ = ("fwd", "adj", "__weakref__")
 
     def __init__(self):
@@ -268,15 +273,16 @@ class _StagedTables:
 _STAGED_TABLES: dict = {}
 
 
-def _staged_tables(cfg: CZTConfig):
-    """The _StagedTables of cfg's geometry, found by content (each call
-    builds its own geometry object); None for the GEMM form."""
+def _staged_tables(cfg: CZTConfig, dev):
+    """The _StagedTables of cfg's geometry on `dev`, for calls of this thread and
+    launch scope, found by content (each call builds its own geometry object);
+    None for the GEMM form."""
     if cfg.form != "bluestein":
         return None
     g = cfg.geom
     grids = (g.x.tobytes(), g.y.tobytes(), g.xout.tobytes(), g.yout.tobytes())
     key = (cfg.mode, float(g.z), float(g.wavelength), float(g.dm), int(g.mode), float(g.hna_radius), float(g.hna_f),
-           *(ops.content_key(b) for b in grids))
+           *(ops.content_key(b) for b in grids), dev, ops.launch_scope(dev), threading.get_ident())
     hit = _STAGED_TABLES.get(key)
     share = hit[1]() if hit is not None and hit[0] == grids else None
     if share is None:
@@ -300,7 +306,7 @@ class _CZTFunction(torch.autograd.Function):
         params = (p00, p01, p10, p11)
         masks = _rebuild(cfg.mask_struct, params)
         # the calls of one geometry in a differentiated step stage its tables once
-        share = _staged_tables(cfg) if any(ctx.needs_input_grad[1:]) else None
+        share = _staged_tables(cfg, src.device) if any(ctx.needs_input_grad[1:]) else None
         out = _czt_staged(share, "fwd", src, cfg, masks=masks, ez_mode=cfg.ez_mode, nin=cfg.nin)
         ctx.tables = share
         ctx.cfg = cfg

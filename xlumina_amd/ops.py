@@ -90,12 +90,20 @@ _grid_ids: dict = {}   # (id(array), device) -> (weak reference, its bytes, Grid
 class GridInfo:
     """What a call needs of a 1-D grid: its float64 device copy, its length and
     its first step."""
-    __slots__ = ("t", "n", "step")
+    __slots__ = ("t", "n", "_step")
 
-    def __init__(self, t: torch.Tensor, host: np.ndarray):
+    def __init__(self, t: torch.Tensor, host):
+        host = np.asarray(host, dtype=np.float64)
         self.t = t
         self.n = int(host.size)
-        self.step = float(host[1] - host[0]) if host.size > 1 else 0.0
+        d = host[1] - host[0] if host.ndim and len(host) > 1 else None
+        self._step = float(d.item()) if d is not None and d.size == 1 else None
+
+    @property
+    def step(self) -> float:
+        if self._step is None:
+            raise ValueError("the sample spacing needs a 1-D grid of two or more samples")
+        return self._step
 
 
 def grid_info(arr, device) -> GridInfo:
@@ -105,13 +113,13 @@ def grid_info(arr, device) -> GridInfo:
     if isinstance(arr, torch.Tensor):
         host = arr.detach().cpu().numpy()
         if arr.device == device and arr.dtype == torch.float64 and arr.is_contiguous():
-            return GridInfo(arr, np.asarray(host, dtype=np.float64).ravel())
+            return GridInfo(arr, host)
     ident = isinstance(host, np.ndarray)
     if ident:
         ent = _grid_ids.get((id(host), device))
         if ent is not None and ent[0]() is host and ent[1] == host.tobytes():
             return ent[2]
-    info = GridInfo(_device_grid_by_content(host, device), np.asarray(host, dtype=np.float64).ravel())
+    info = GridInfo(_device_grid_by_content(host, device), host)
     if ident:
         if len(_grid_ids) > 256:
             _grid_ids.clear()

@@ -97,6 +97,14 @@ template <int L, int TPF> struct FftPlan {
 
 __device__ __forceinline__ int lpad(int i) { return i + (i >> 4); }
 template <int L> struct LdsLen { static constexpr int value = L + L / 16; };
+// lpad(i + k) - lpad(i) for a constant k, where no carry from the low four
+// bits depends on i: a pass adds it to one address per thread (left to the
+// compiler, some passes formed every second address by itself and wrote
+// unpaired: czt_rows<2048>, 400 rows, one in ten us).
+__host__ __device__ constexpr int lstep(int k) { return k + (k >> 4); }
+// Whether that holds for the outputs idxD + r NS of a radix-R pass of stride
+// NS (idxD = (j / NS) NS R + j % NS).
+constexpr bool lpad_flat(int NS, int R) { return NS % 16 == 0 || ((NS & (NS - 1)) == 0 && NS * R % 16 == 0); }
 // Threads per FFT: one radix-16 butterfly per thread and pass up to L = 2048;
 // two at L = 4096, so that four 4096-point FFTs per block run on 512 threads
 // with up to 256 VGPRs each instead of spilling at 1024 threads (128 VGPRs).
@@ -361,7 +369,7 @@ __device__ __forceinline__ void stockham_pass(float2* s, int t) {
     const int j = t + b * TPF;
     if (act && (NB % TPF == 0 || j < NB)) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[b][r] = s[lpad(j + r * NB)];
+      for (int r = 0; r < R; ++r) v[b][r] = NB % 16 ? s[lpad(j + r * NB)] : s[lpad(j) + lstep(r * NB)];
       if constexpr (NS > 1) apply_twiddles<R, INV, L>(v[b], (j % NS) * (Tw<L>::N / (NS * R)));
       DFT<R, INV>::run(v[b]);
     }
@@ -373,7 +381,7 @@ __device__ __forceinline__ void stockham_pass(float2* s, int t) {
     if (act && (NB % TPF == 0 || j < NB)) {
       const int idxD = (j / NS) * NS * R + (j % NS);
 #pragma unroll
-      for (int r = 0; r < R; ++r) s[lpad(idxD + r * NS)] = v[b][r];
+      for (int r = 0; r < R; ++r) s[lpad_flat(NS, R) ? lpad(idxD) + lstep(r * NS) : lpad(idxD + r * NS)] = v[b][r];
     }
   }
   __syncthreads();

@@ -50,7 +50,7 @@ __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& sto
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         if (ZHI && r >= R / 2) v[b][r] = make_float2(0.f, 0.f);
-        else if constexpr (SRC == SRC_LDS) v[b][r] = s[lpad(j + r * NB)];
+        else if constexpr (SRC == SRC_LDS) v[b][r] = NB % 16 ? s[lpad(j + r * NB)] : s[lpad(j) + lstep(r * NB)];
         else if constexpr (SRC == SRC_FN) v[b][r] = load(b * TPF + r * NB);
         else v[b][r] = reg.v[b][r];
       }
@@ -73,7 +73,7 @@ __device__ __forceinline__ void pass_io(float2* s, int t, Load& load, Store& sto
       const int idxD = (j / NS) * NS * R + (j % NS);
 #pragma unroll
       for (int r = 0; r < (LOW ? R / 2 : R); ++r) {
-        if constexpr (DST == DST_LDS) s[lpad(idxD + r * NS)] = v[b][r];
+        if constexpr (DST == DST_LDS) s[lpad_flat(NS, R) ? lpad(idxD) + lstep(r * NS) : lpad(idxD + r * NS)] = v[b][r];
         else if constexpr (DST == DST_FN) store(b * TPF + r * NS, v[b][r]);
         else reg.v[b][r] = v[b][r];
       }

@@ -333,7 +333,7 @@ __global__ __launch_bounds__(UFinal<P>::NT, 4) void rs_final_pre_kernel(RsArgs a
   float2* s = lds + g * U::LS;
   const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
   const RowTiles rt(a.n, g, t);
-  const bool load_ok = row < rt.nrg * 4, rowok = row < a.n;
+  const bool load_ok = U::WHOLE || row < rt.nrg * 4, rowok = row < a.n;
   const double Y = EZ ? b.y[rowok ? row : 0] : 0.0, z = EZ ? (b.z_dev ? *b.z_dev : b.z) : 0.0;
   const uint32_t row_at = (uint32_t)(rowok ? row : 0) * a.n;
   const bool ezdz = EZ && b.ezdz;

@@ -97,13 +97,6 @@ __device__ __forceinline__ RsArgs rs_member(const RsArgs& a0, int b) {
   return a;
 }
 
-// lag value of circular slot s on a P-point axis with N samples (0 => unused)
-__device__ __forceinline__ bool lag_of(const double* g, int s, int n, int P, double* d) {
-  if (s < n) { *d = g[s] - g[0]; return true; }
-  if (s > P - n) { *d = g[P - s] - g[0]; return true; }
-  return false;
-}
-
 // 1/sqrt(x) in float64 for x > 0: the hardware estimate (v_rsq_f64) refined by
 // two Newton steps y <- y (3/2 - x y^2 / 2), which take any estimate within
 // 2^-20 to the last bits of float64; the kernel values need r = x / sqrt(x) to
@@ -234,6 +227,9 @@ template <int P, int G_> struct Units {
   static constexpr int RAW = LdsLen<P>::value;
   static constexpr int WANT = G == 1 ? 0 : (G >= 8 ? 4 : 32 / G);
   static constexpr int LS = G == 1 ? RAW : RAW + (WANT - RAW % 32 + 32) % 32;
+  // Up to four rows per block divide a tile's four: the blocks' rows are all
+  // among the tiled ones, and the accesses carry no predicate for them.
+  static constexpr bool WHOLE = G <= 4;
   // column pass: neighbouring lanes on the G columns of a row
   __device__ static int col_g(int tid) { return G == 1 ? 0 : tid % G; }
   __device__ static int col_t(int tid) { return G == 1 ? tid : tid / G; }
@@ -287,18 +283,19 @@ __global__ __launch_bounds__(UHrow<P>::NT, 4) void rs_hrow_kernel(RsArgs a0) {
   float2* s = lds + g * U::LS;
   const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, r = row0 + g;
   const RowTiles rt(a.n, g, t);
-  const bool store_ok = r < rt.nrg * 4;
+  const bool store_ok = U::WHOLE || r < rt.nrg * 4;
   const double z = a.z_dev ? *a.z_dev : a.z;
-  double dy;
-  const bool rowok = lag_of(a.y, r, a.n, P, &dy) && r < a.n;
+  // columns c < N of a row r < N (N <= P/2: the lags above are mirrors)
+  const int ncol = r < a.n ? a.n : 0;
+  const double dy = a.y[r < a.n ? r : 0] - a.y[0];
   float2 dv[2][NCOL];
 #pragma unroll
   for (int i = 0; i < NCOL; ++i) {
     const int c = t + i * TPF;
     if (c > P / 2) break;
-    double dx;
     float2 v = make_float2(0.f, 0.f), vz = v, vk = v;
-    if (rowok && lag_of(a.x, c, a.n, P, &dx)) {
+    if (c < ncol) {
+      const double dx = a.x[c] - a.x[0];
       if constexpr (DM == 0)
         v = a.kernel_dz == 1   ? rs_kernel_dz_value(dx, dy, z, a.k)
             : a.kernel_dz == 2 ? rs_kernel_dk_value(dx, dy, z, a.k)
@@ -364,7 +361,7 @@ __global__ __launch_bounds__((UUrow<P, ONE>::NT), P == 1536 ? 3 : 1) void rs_uro
   float2* s = lds + g * U::LS;
   const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
   const RowTiles rt(a.n, g, t);
-  const bool store_ok = row < rt.nrg * 4, rowok = row < a.n;
+  const bool store_ok = U::WHOLE || row < rt.nrg * 4, rowok = row < a.n;
   NoIO none;
   typename LastPass<P, TPF, true>::Type unused;
   if constexpr (ONE) {
@@ -437,13 +434,16 @@ __global__ __launch_bounds__(UHcol<P>::NT, 4) void rs_hcol_kernel(RsArgs a0) {
   const int g = U::col_g(threadIdx.x), t = U::col_t(threadIdx.x);
   float2* s = lds + g * U::LS;
   const int col0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, col = col0 + g;
-  const bool act = col <= P / 2;
+  const bool act = U::G == 1 || col <= P / 2;
   const int nrg = (a.n + 3) >> 2;
   const float2* hc = a.hr + (int64_t)(col0 >> 2) * nrg * 16 + (col0 & 3);
   const uint32_t lane = (g >> 2) * nrg * 16 + (g & 3);
   auto load = [&](int k) -> float2 {
+    // (rows beyond N read row N - 1 and are zeroed: a select, where a predicate
+    // would put a branch around each load)
     const int r = t + k, rr = r <= P / 2 ? r : P - r;
-    return (act && rr < a.n) ? ld_at(hc, lane + 4 * rr) : make_float2(0.f, 0.f);
+    const float2 v = ld_at(hc, lane + 4 * min(rr, a.n - 1));
+    return act && rr < a.n ? v : make_float2(0.f, 0.f);
   };
   typename HO::Type u;
   fft_forward_to_regs<P, TPF, SRC_FN>(s, t, load, u);
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(UFinal<P>::NT) void rs_final_kernel(RsArgs a0) {
   float2* s = lds + g * U::LS;
   const int row0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, row = row0 + g;
   const RowTiles rt(a.n, g, t);
-  const bool load_ok = row < rt.nrg * 4;
+  const bool load_ok = U::WHOLE || row < rt.nrg * 4;
   // output columns < N <= P/2 are slots q < R/2 of the last pass
   constexpr int QH = LP::R / 2;
   float inten[LP::BPT][QH];

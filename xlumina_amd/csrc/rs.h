@@ -23,7 +23,8 @@
 //   rs_col    : per (column, component): FFT(T col) * Hhat -> IFFT, keep rows
 //               0..N-1 -> T
 //   rs_final  : row IFFT of T, keep columns 0..N-1 -> output (+ |E|^2)
-// Hr lives where rs_urow puts T afterwards.
+// Hr lies beside Hhat in the spectrum's part of the workspace, with its last
+// columns in T where both do not fit (RsArgs::hr, hr2).
 #pragma once
 #include "fft.h"
 #include "fftio.h"
@@ -39,7 +40,8 @@ struct RsArgs {
   int64_t out_cs;
   float* intensity;       // optional N x N, sum_c |out_c|^2
   float2* t;              // tiles, ncomp x NR4*4 x P
-  float2* hr;             // Hr: N rows x (P/2 + 1) columns in tiles (rs_hr_elems)
+  float2* hr;             // Hr: N rows x (P/2 + 1) columns in tiles (rs_hr_elems): columns < rs_hr_split(P),
+  float2* hr2;            // and the others, at the same offsets from hr2 (hr itself, or T)
   float2* hh;             // Hhat: columns kx <= P/2 of stride rs_hh_stride, ky <= P/2 (even in kx and ky)
   const double* x;
   const double* y;
@@ -87,6 +89,7 @@ __device__ __forceinline__ RsArgs rs_member(const RsArgs& a0, int b) {
   if (a.intensity) a.intensity += b * a0.inten_bs;
   a.t += b * a0.t_bs;
   a.hr += b * a0.t_bs;
+  a.hr2 += b * a0.t_bs;
   a.hh += b * a0.hh_bs;
   if (a.z_dev) a.z_dev += b;
 #pragma unroll
@@ -188,9 +191,19 @@ __device__ __forceinline__ float2 stream_load(const float2* p) {
   return make_float2(__builtin_nontemporal_load(&p->x), __builtin_nontemporal_load(&p->y));
 }
 
-// Elements of Hr (n rows, columns kx <= P/2): at most half the n x P tiles of
-// one component of T, where it lives until rs_urow writes T.
-__host__ __device__ constexpr int64_t rs_hr_elems(int n, int P) { return (int64_t)(P / 8 + 1) * ((n + 3) / 4) * 16; }
+// Elements of Hr (n rows, columns kx <= P/2 or below `cols`): at most half the
+// n x P tiles of one component of T.
+__host__ __device__ constexpr int64_t rs_hr_elems(int n, int P, int cols = 0) {
+  return (int64_t)(cols ? cols / 4 : P / 8 + 1) * ((n + 3) / 4) * 16;
+}
+// First column of Hr's second part, a multiple of every pass's last stride.
+// T's lines are still in the caches of the XCDs that ran the last passes of
+// the call before, and writes to them cost more.  With all of Hr in T, RS
+// 1000^2 takes 16.4 us for the kernel's rows, 16.9 for the field's rows after
+// them and 64.5 in all, with Hr beside Hhat 13.2, 15.3 and 59.3; 1024^2, where
+// seven eighths fit, 17.7, 17.2 and 66 against 13.4, 16.7 and 61.4.
+constexpr int RS_HR_SPLIT_MIN = 256;   // shorter lengths have Hr in one place
+__host__ __device__ constexpr int rs_hr_split(int P) { return P / 16 * 7; }
 // Column stride of Hhat: ky = 0..P/2 and a pad to whole 128 B lines.
 __host__ __device__ constexpr int rs_hh_stride(int P) { return P / 2 + 16; }
 
@@ -312,9 +325,10 @@ __global__ __launch_bounds__(UHrow<P>::NT, 4) void rs_hrow_kernel(RsArgs a0) {
   NoIO none;
   typename LastPass<P, TPF, true>::Type unused;
   {
-    float2* dst = a.hr + RowTiles::base(row0);
+    float2 *dst = a.hr + RowTiles::base(row0), *dst2 = a.hr2 + RowTiles::base(row0);
     auto store = [&](int k, float2 v) {
-      if (store_ok && (k < P / 2 || (k == P / 2 && t == 0))) st_at(dst + rt.step(k), rt.lane, v);
+      if (store_ok && (k < P / 2 || (k == P / 2 && t == 0)))
+        st_at((k < rs_hr_split(P) ? dst : dst2) + rt.step(k), rt.lane, v);
     };
     fft_io<P, TPF, false, SRC_LDS, DST_FN>(s, t, none, store, unused);
   }
@@ -429,6 +443,7 @@ __global__ __launch_bounds__(UHcol<P>::NT, 4) void rs_hcol_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
   using U = UHcol<P>;
   constexpr int TPF = U::TPF;
+  static_assert(P < RS_HR_SPLIT_MIN || rs_hr_split(P) % U::G == 0, "a block's columns lie in one part of Hr");
   using HO = HandOff<P, TPF>;
   __shared__ float2 lds[U::G * U::LS];
   const int g = U::col_g(threadIdx.x), t = U::col_t(threadIdx.x);
@@ -436,7 +451,7 @@ __global__ __launch_bounds__(UHcol<P>::NT, 4) void rs_hcol_kernel(RsArgs a0) {
   const int col0 = xcd_remap(blockIdx.x, gridDim.x) * U::G, col = col0 + g;
   const bool act = U::G == 1 || col <= P / 2;
   const int nrg = (a.n + 3) >> 2;
-  const float2* hc = a.hr + (int64_t)(col0 >> 2) * nrg * 16 + (col0 & 3);
+  const float2* hc = (col0 < rs_hr_split(P) ? a.hr : a.hr2) + (int64_t)(col0 >> 2) * nrg * 16 + (col0 & 3);
   const uint32_t lane = (g >> 2) * nrg * 16 + (g & 3);
   auto load = [&](int k) -> float2 {
     // (rows beyond N read row N - 1 and are zeroed: a select, where a predicate
@@ -743,7 +758,7 @@ inline void rs_kept_spectra_launch(const RsArgs& a, int nb, hipStream_t st) {
   for (int i = 0; with_h && i < 2; ++i) {
     if (!a.dg[i]) continue;
     RsArgs d = a;   // the derivative row transforms, unconjugated
-    d.hr = a.dgr[i];
+    d.hr = d.hr2 = a.dgr[i];
     d.hh = a.dg[i];
     d.adjoint = 0;
     d.hstored = 1;
@@ -757,7 +772,7 @@ template <int P, bool KEEP>
 inline void rs_launch(const RsArgs& a, hipStream_t st) {
   const int rows = rs_rows4(a.n);
   const int nb = a.batch > 1 ? a.batch : 1;
-  // Hr lives in the tiles that rs_urow fills later, so the spectra come first
+  // Hr may lie in the tiles that rs_urow fills later, so the spectra come first
   if (KEEP && (a.hstored || a.spec_mode)) {
     if constexpr (KEEP) rs_kept_spectra_launch<P>(a, nb, st);
   } else {

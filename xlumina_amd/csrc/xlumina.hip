@@ -408,8 +408,16 @@ static int rs_run(const xl_rs_params* p, const xl::PreArgs* pre, void* ws, size_
   a.out_cs = p->out_comp_stride;
   a.intensity = p->intensity;
   a.t = (float2*)w;
-  a.hr = a.t;   // the row-transformed kernel, until the field's rows take its place
-  a.hh = p->hhat_mode ? (float2*)p->hhat : a.t + ncomp * nr4 * P2;
+  float2* spectra = a.t + ncomp * nr4 * P2;
+  a.hh = p->hhat_mode ? (float2*)p->hhat : spectra;
+  // the row-transformed kernel: in the room that Hhat leaves; where that is too small (2n - 1 close to a power of
+  // two), the columns from rs_hr_split on in T
+  const int64_t hh_elems = p->hhat_mode ? 0 : (int64_t)(P / 2 + 1) * xl::rs_hh_stride(P);
+  const int64_t room = (int64_t)(P2 / 2) * P2 + P2 - hh_elems;
+  const bool whole = xl::rs_hr_elems(n, P) <= room;
+  const bool part = P >= xl::RS_HR_SPLIT_MIN && xl::rs_hr_elems(n, P, xl::rs_hr_split(P)) <= room;
+  a.hr = whole || part ? spectra + hh_elems : a.t;
+  a.hr2 = whole ? a.hr : a.t;
   a.hstored = p->hhat_mode ? 1 : 0;
   a.hreuse = p->hhat_mode == 2 ? 1 : 0;
   a.x = p->x;

@@ -57,3 +57,31 @@ def test_kernel_rows_in_either_place(cuda_dev, n):
         a = ops.rs_propagate(src, x, x, 30.0 * n, 0.65, **kw)
         b = ops.rs_propagate(src, x, x, 30.0 * n, 0.65, hhat=hh, hhat_mode=1, **kw)
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [2, 3, 29, 31, 63, 66, 127, 130, 255])
+def test_rows_of_two_components(cuda_dev, n):
+    rng = np.random.default_rng(n)
+    x, y = R.space(3.0 * n, n)
+    e = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
+    p = rng.uniform(-np.pi, np.pi, (2, n, n)).astype(np.float32)
+    masks = [MaskSpec(N.XL_MASK_SSLM, *(torch.tensor(v, device=cuda_dev) for v in p))]
+    out = ops.rs_propagate(torch.tensor(e.astype(np.complex64), device=cuda_dev), x, y, 40.0 * n, 0.65, masks=masks)
+    for i in range(2):
+        ref = R.rs_propagation(e[i] * np.exp(1j * p[i].astype(np.float64)), x, y, 0.65, 40.0 * n)[0]
+        assert rel_l2(out[i].cpu().numpy(), ref) < 1e-5
+
+
+# members whose rows together stay within or exceed 2048
+@pytest.mark.parametrize("n,batch", [(64, 40), (128, 17), (250, 8), (250, 9), (256, 8), (256, 9)])
+def test_rows_of_a_batch(cuda_dev, n, batch):
+    g = gen(n)
+    x = np.linspace(-1.5 * n, 1.5 * n, n)
+    src = cplx(g, batch, 2, n, n)
+    masks = lambda p: [MaskSpec(N.XL_MASK_LCD, p[0], p[1])]
+    p = uni(g, 2, n, n)
+    z = torch.linspace(20.0 * n, 30.0 * n, batch, dtype=torch.float64, device=cuda_dev)
+    kw = dict(ez_mode=N.XL_EZ_VRS, nin=2)
+    out = ops.rs_propagate_batched(src, x, x, 0.65, z, masks=masks(p), **kw)
+    for b in (0, batch // 2, batch - 1):
+        near(out[b], ops.rs_propagate(src[b], x, x, 0.0, 0.65, masks=masks(p), z_dev=z[b:b + 1], **kw), 2e-6)

@@ -85,3 +85,44 @@ def test_rows_of_a_batch(cuda_dev, n, batch):
     out = ops.rs_propagate_batched(src, x, x, 0.65, z, masks=masks(p), **kw)
     for b in (0, batch // 2, batch - 1):
         near(out[b], ops.rs_propagate(src[b], x, x, 0.0, 0.65, masks=masks(p), z_dev=z[b:b + 1], **kw), 2e-6)
+
+
+# up to 256 rows of 4096 points: three components side by side; more: one after the other
+@pytest.mark.parametrize("m", [2, 3, 255, 256, 257])
+@pytest.mark.parametrize("hna", [False, True])
+def test_few_long_rows(cuda_dev, m, hna):
+    n = 2048
+    x = np.linspace(-1800.0, 1800.0, n)
+    xo, yo = np.linspace(-9.0, 8.0, 200), np.linspace(-8.0, 9.0, m)
+    geom = (ops.hna_geometry(x, x, xo, yo, 0.635, 1800.0, 2000.0) if hna else ops.czt_geometry(x, x, xo, yo, 3e4, 0.635))
+    g = gen(m)
+    cot = cplx(g, 3, m, 200)
+    got = ops.czt(cot, geom, adjoint=True, form="bluestein")
+    for c in range(3):   # a component alone takes the one-buffer rows
+        if hna:
+            only = torch.zeros_like(cot)
+            only[c] = cot[c]
+            one = ops.czt(only, geom, adjoint=True, form="bluestein")
+            assert float(one[[i for i in range(3) if i != c]].abs().max()) == 0.0
+            near(got[c], one[c], 2e-6)
+        else:
+            near(got[c:c + 1], ops.czt(cot[c:c + 1], geom, adjoint=True, form="bluestein"), 2e-6)
+    f = cplx(g, 3, n, n)
+    af = ops.czt(f, geom, form="bluestein") if not hna else None
+    if af is not None:
+        adjoint_identity(f, af, cot, got)
+
+
+@pytest.mark.parametrize("n", [200, 256, 258])
+def test_long_rows_of_a_small_pupil(cuda_dev, n):
+    """Few input rows onto a wide window: 4096-point rows of three components."""
+    rng = np.random.default_rng(n)
+    x, y = R.space(1800.0, n)
+    xo = np.linspace(-60.0, 60.0, 1900)
+    e = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
+    src = torch.tensor(e.astype(np.complex64), device=cuda_dev)
+    out = ops.czt(src, ops.hna_geometry(x, y, xo, xo, 0.65, 1800.0, 2000.0), nin=2, form="bluestein")
+    ref = np.stack(R.vczt_objective_lens(e[0], e[1], x, y, 0.65, 1800.0, 2000.0, xo, xo))
+    assert rel_l2(out.cpu().numpy(), ref) < 1e-5
+    out = ops.czt(src, ops.czt_geometry(x, y, xo, xo, 3e4, 0.65), ez_mode=N.XL_EZ_VCZT, nin=2, form="bluestein")
+    assert rel_l2(out.cpu().numpy(), np.stack(R.vczt(e[0], e[1], x, y, 0.65, 3e4, xo, xo))) < 1e-5

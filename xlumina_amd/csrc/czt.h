@@ -574,8 +574,15 @@ __global__ __launch_bounds__(CztCols1<Q>::NT, 4) void czt_cols1_kernel(CztArgs a
 // Power-of-two lengths (the 3 * 2^k ones serve the column pass only).
 template <int Q> struct CztPow2 { static constexpr bool value = (Q & (Q - 1)) == 0; };
 
-// The one-buffer form for one component and for the 4096-point zero-half
-// rows, the three-buffer form otherwise (see czt_rows1_kernel).
+// Three-buffer blocks of a 4096-point row that run at once (104 KB of LDS: one
+// per CU).
+constexpr int CZT_ROWS_RESIDENT = 256;
+
+// The one-buffer form for one component and for the 4096-point zero-half rows
+// from the second round of three-buffer blocks on, the three-buffer form
+// otherwise (see czt_rows1_kernel).  The 4096-point rows of three components,
+// three buffers against one: 64 rows 16.7 / 26.6 us, 192 20.7 / 28.6, 256 23.3 /
+// 30.0, 320 34.1 / 31.7, 768 44.7 / 37.6.
 template <int Q, int K, bool ZL>
 inline void czt_rows_launch_k(const CztArgs& a, int batch, hipStream_t st) {
   using U1 = CztRows1<Q>;
@@ -585,13 +592,14 @@ inline void czt_rows_launch_k(const CztArgs& a, int batch, hipStream_t st) {
       hipLaunchKernelGGL((czt_rows1_kernel<Q, K, ZL, false>), g1, b1, 0, st, a);
       return;
     }
-  if constexpr (ZL && Q >= 4096) {
-    hipLaunchKernelGGL((czt_rows1_kernel<Q, K, ZL, true>), g1, b1, 0, st, a);
-  } else {
-    const dim3 g(a.rin, batch), b(a.ncomp * Q / 16);
-    const size_t lds = (size_t)a.ncomp * LdsLen<Q>::value * sizeof(float2);
-    hipLaunchKernelGGL((czt_rows_kernel<Q, K, ZL>), g, b, lds, st, a);
-  }
+  if constexpr (ZL && Q >= 4096)
+    if (a.ncomp > 1 && (int64_t)a.rin * batch > CZT_ROWS_RESIDENT) {
+      hipLaunchKernelGGL((czt_rows1_kernel<Q, K, ZL, true>), g1, b1, 0, st, a);
+      return;
+    }
+  const dim3 g(a.rin, batch), b(a.ncomp * Q / 16);
+  const size_t lds = (size_t)a.ncomp * LdsLen<Q>::value * sizeof(float2);
+  hipLaunchKernelGGL((czt_rows_kernel<Q, K, ZL>), g, b, lds, st, a);
 }
 template <int Q, bool ZL>
 inline void czt_rows_launch_zl(const CztArgs& a, int batch, hipStream_t st) {
@@ -609,13 +617,11 @@ inline void czt_rows_launch(const CztArgs& a, int batch, hipStream_t st) {
 // the library's initialisation for every length it runs at.
 template <int Q, bool ZL> inline hipError_t czt_set_attribute_zl() {
   hipError_t e = hipSuccess;
-  if constexpr (!(ZL && Q >= 4096)) {
-    const int mx = 3 * LdsLen<Q>::value * (int)sizeof(float2);
-    for (const void* f : {(const void*)czt_rows_kernel<Q, PREK_F, ZL>, (const void*)czt_rows_kernel<Q, PREK_HNA, ZL>,
-                          (const void*)czt_rows_kernel<Q, PREK_SIMPLE, ZL>}) {
-      const hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, mx);
-      if (r != hipSuccess) e = r;
-    }
+  const int mx = 3 * LdsLen<Q>::value * (int)sizeof(float2);
+  for (const void* f : {(const void*)czt_rows_kernel<Q, PREK_F, ZL>, (const void*)czt_rows_kernel<Q, PREK_HNA, ZL>,
+                        (const void*)czt_rows_kernel<Q, PREK_SIMPLE, ZL>}) {
+    const hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, mx);
+    if (r != hipSuccess) e = r;
   }
   return e;
 }

@@ -126,3 +126,19 @@ def test_long_rows_of_a_small_pupil(cuda_dev, n):
     assert rel_l2(out.cpu().numpy(), ref) < 1e-5
     out = ops.czt(src, ops.czt_geometry(x, y, xo, xo, 3e4, 0.65), ez_mode=N.XL_EZ_VCZT, nin=2, form="bluestein")
     assert rel_l2(out.cpu().numpy(), np.stack(R.vczt(e[0], e[1], x, y, 0.65, 3e4, xo, xo))) < 1e-5
+
+
+# 64 MB of tiles: columns of the batch staged, a member's alone direct; then rows of one component whose plane factors
+# come from a table, most of the row being input or not
+@pytest.mark.parametrize("n,m,batch", [(1024, 1024, 8), (1023, 1009, 9), (700, 300, 4), (640, 300, 4), (641, 300, 4),
+                                       (1500, 500, 4)])
+def test_forms_of_a_batch(cuda_dev, n, m, batch):
+    g = gen(n)
+    x, xo = np.linspace(-900.0, 900.0, n), np.linspace(-400.0, 390.0, m)
+    geom = ops.czt_geometry(x, x, xo, xo, 3e4, 0.635)
+    src, cot, ph = cplx(g, batch, 1, n, n), cplx(g, batch, 1, m, m), uni(g, batch, n, n)
+    out = ops.czt(src, geom, masks=[MaskSpec(N.XL_MASK_SLM, ph)], batch=batch)
+    adj = ops.czt(cot, geom, adjoint=True, batch=batch)
+    for b in (0, batch - 1):
+        near(out[b], ops.czt(src[b], geom, masks=[MaskSpec(N.XL_MASK_SLM, ph[b])], form="bluestein"), 2e-6)
+        near(adj[b], ops.czt(cot[b], geom, adjoint=True, form="bluestein"), 2e-6)

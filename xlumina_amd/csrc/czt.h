@@ -582,13 +582,18 @@ constexpr int CZT_ROWS_RESIDENT = 256;
 // from the second round of three-buffer blocks on, the three-buffer form
 // otherwise (see czt_rows1_kernel).  The 4096-point rows of three components,
 // three buffers against one: 64 rows 16.7 / 26.6 us, 192 20.7 / 28.6, 256 23.3 /
-// 30.0, 320 34.1 / 31.7, 768 44.7 / 37.6.
+// 30.0, 320 34.1 / 31.7, 768 44.7 / 37.6.  One component keeps three buffers'
+// staging where a batch takes its plane factors from a table (nothing but loads
+// to wait for) and most of a full-length row is input: 4 members of 1500 -> 500
+// 59.5 / 67.6 us, of 700 -> 300 19.7 / 23.4, 16 members of 1200 -> 800 187.6 /
+// 180.0; elsewhere the one buffer is 4 to 50 % faster.
 template <int Q, int K, bool ZL>
 inline void czt_rows_launch_k(const CztArgs& a, int batch, hipStream_t st) {
   using U1 = CztRows1<Q>;
   const dim3 g1((a.rin + U1::G - 1) / U1::G, batch), b1(U1::NT);
+  const bool tabled = !ZL && Q >= 1024 && a.ftab && 8 * a.ax.lin > 5 * Q;
   if constexpr (K != PREK_HNA)
-    if (a.ncomp == 1) {
+    if (a.ncomp == 1 && !tabled) {
       hipLaunchKernelGGL((czt_rows1_kernel<Q, K, ZL, false>), g1, b1, 0, st, a);
       return;
     }

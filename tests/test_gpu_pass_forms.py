@@ -142,3 +142,19 @@ def test_forms_of_a_batch(cuda_dev, n, m, batch):
     for b in (0, batch - 1):
         near(out[b], ops.czt(src[b], geom, masks=[MaskSpec(N.XL_MASK_SLM, ph[b])], form="bluestein"), 2e-6)
         near(adj[b], ops.czt(cot[b], geom, adjoint=True, form="bluestein"), 2e-6)
+
+
+# columns staged through LDS or not: outputs within, at and above the inputs (full and zero-half lengths 128..1024)
+@pytest.mark.parametrize("n,m", [(50, 30), (64, 66), (100, 28), (120, 130), (130, 120), (61, 400), (200, 300), (300, 200),
+                                 (99, 250), (100, 200), (100, 199), (100, 500), (300, 700), (512, 512)])
+def test_column_forms(cuda_dev, n, m):
+    rng = np.random.default_rng(n + m)
+    x, y = R.space(2.0 * n, n)
+    xo = np.linspace(-0.3 * n, 0.35 * n, m)
+    e = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
+    src = torch.tensor(e.astype(np.complex64), device=cuda_dev)
+    geom = ops.czt_geometry(x, y, xo, xo, 3e4, 0.635)
+    out = ops.czt(src, geom, ez_mode=N.XL_EZ_VCZT, nin=2, form="bluestein")
+    assert rel_l2(out.cpu().numpy(), np.stack(R.vczt(e[0], e[1], x, y, 0.635, 3e4, xo, xo))) < 1e-5
+    cot = cplx(gen(n), 2, m, m)
+    adjoint_identity(src, ops.czt(src, geom, form="bluestein"), cot, ops.czt(cot, geom, adjoint=True, form="bluestein"))

@@ -571,6 +571,71 @@ __global__ __launch_bounds__(CztCols1<Q>::NT, 4) void czt_cols1_kernel(CztArgs a
     }
 }
 
+// The same pass staged through LDS: the block's four columns, one tile group,
+// are loaded with lane-contiguous accesses and the outputs are transposed to
+// rows, so that a row segment of 32 B is stored at once.  The first pass reads
+// LDS, the last one leaves its outputs in registers.
+template <int Q, bool ZL>
+__global__ __launch_bounds__(4 * Q / 16) void czt_cols_staged_kernel(CztArgs a0) {
+  const CztArgs a = czt_member(a0, blockIdx.z);
+  constexpr int TPF = Q / 16, LS = LdsLen<Q>::value, CPB = 4, NT = CPB * TPF;
+  using HO = HandOff<Q, TPF>;
+  using LP = LastPass<Q, TPF, false>;
+  __shared__ float2 lds[CPB * LS];
+  const int f = threadIdx.x / TPF, t = threadIdx.x % TPF;
+  float2* s = lds + f * LS;
+  const int kx0 = xcd_remap(blockIdx.x, gridDim.x) * CPB, c = blockIdx.y;
+  const int lout_x = a.ax.lout, lin = a.ay.lin, lout = a.ay.lout;
+  const float2* src = a.t + (int64_t)c * a.t_cs;
+  typename HO::Type u;
+  NoIO none;
+  // IT elements per thread, loaded U at a time before their products
+  constexpr int IT = (ZL ? Q / 2 : Q) / TPF, U = IT < 8 ? IT : 8;
+#pragma unroll
+  for (int i0 = 0; i0 < IT; i0 += U) {
+    float2 tv[U], pv[U];
+#pragma unroll
+    for (int u1 = 0; u1 < U; ++u1) {
+      const int e = threadIdx.x + (i0 + u1) * NT, r = e / CPB, g = e % CPB;
+      const bool ok = r < lin && kx0 + g < lout_x;
+      tv[u1] = src[czt_tidx(a.rin4, ok ? r : 0, ok ? kx0 + g : kx0)];
+      pv[u1] = a.ay.pre[ok ? r : 0];
+    }
+#pragma unroll
+    for (int u1 = 0; u1 < U; ++u1) {
+      const int e = threadIdx.x + (i0 + u1) * NT, r = e / CPB, g = e % CPB;
+      const bool ok = r < lin && kx0 + g < lout_x;
+      lds[g * LS + lpad(r)] = ok ? cmul(tv[u1], pv[u1]) : make_float2(0.f, 0.f);
+    }
+  }
+  __syncthreads();
+  fft_forward_to_regs<Q, TPF, SRC_LDS, ZL>(s, t, none, u);
+#pragma unroll
+  for (int b = 0; b < HO::BPT; ++b)
+#pragma unroll
+    for (int q = 0; q < HO::R; ++q) u.v[b][q] = cmul(u.v[b][q], a.ay.gf[HO::index(t, b, q)]);
+  typename LP::Type o;
+  chain_io<Q, TPF, true, false, 0, SRC_REG, DST_REG, false, ZL>(s, t, none, none, u, o);
+  __syncthreads();   // the last pass of other waves may still read LDS
+#pragma unroll
+  for (int b = 0; b < LP::BPT; ++b)
+#pragma unroll
+    for (int q = 0; q < (ZL ? LP::R / 2 : LP::R); ++q) {
+      const int ky = LP::index(t, b, q);
+      if (ky < lout) lds[ky * CPB + f] = cmul(o.v[b][q], a.ay.post[ky]);
+    }
+  __syncthreads();
+  float2* oc = a.out + (int64_t)c * a.out_cs;
+  for (int e = threadIdx.x; e < lout * CPB; e += NT) {
+    const int ky = e / CPB, kx = kx0 + e % CPB;
+    if (kx >= lout_x) continue;
+    float2 v = lds[e];
+    if (a.f0tab) v = c_mul(v, a.f0tab[(int64_t)ky * lout_x + kx]);
+    else if (a.post_mode != POST_NONE) v = c_mul(v, czt_post_factor(a, ky, kx));
+    oc[(int64_t)ky * lout_x + kx] = v;
+  }
+}
+
 // Power-of-two lengths (the 3 * 2^k ones serve the column pass only).
 template <int Q> struct CztPow2 { static constexpr bool value = (Q & (Q - 1)) == 0; };
 
@@ -643,10 +708,37 @@ inline hipError_t czt_set_attributes() {
   return e;
 }
 
+// Whether the power-of-two column pass of a.ay stages its columns through LDS
+// (us, staged / direct, MI355X).  Up to 1024 points it does, unless the outputs
+// outnumber the inputs (twice where both fit half the length), when the staging
+// of the zero padding costs more than the stores gain: 250 -> 99 samples 8.3 /
+// 9.3, 400 -> 61 8.4 / 10.8, 61 -> 400 15.6 / 13.4, 512 -> 512 (three
+// components) 14.0 / 15.1, 700 -> 300 (4 members) 12.3 / 15.4, 300 -> 700 20.6 /
+// 19.8, 100 -> 500 12.6 / 11.0.  At 2048 its blocks of four columns are fewer
+// and wait longer (1024 -> 400, three components, 17.0 / 14.0), but read a tile
+// line once where the direct blocks of two columns read it twice, which shows
+// when the tiles no longer stay in the caches: 1024 -> 1024, 4 members 36.0 /
+// 36.5, 8 members 62.6 / 65, 16 members 130 / 152, 64 members 503 / 640, and
+// 900 -> 900, 32 members 255 / 287 (1200 -> 800, 16 members 115 / 110).  At 4096
+// direct blocks always win.
+constexpr int64_t CZT_STAGED_TILE_BYTES = 64 << 20;
+template <int Q> inline bool czt_cols_staged(const CztArgs& a, int batch) {
+  if (Q > 2048) return false;
+  if (Q == 2048) return a.ay.zl && batch * a.ncomp * a.t_cs * (int64_t)sizeof(float2) >= CZT_STAGED_TILE_BYTES;
+  return a.ay.zl ? a.ay.lout < 2 * a.ay.lin : a.ay.lout <= a.ay.lin;
+}
+
 template <int Q>
 inline void czt_cols_launch(const CztArgs& a, int batch, hipStream_t st) {
   KTimer t(K_CZT_COLS, st);
   if constexpr (CztPow2<Q>::value) {
+    if constexpr (Q <= 2048)
+      if (czt_cols_staged<Q>(a, batch)) {
+        const dim3 g((a.ax.lout + 3) / 4, a.ncomp, batch), b(Q / 4);
+        if (a.ay.zl) hipLaunchKernelGGL((czt_cols_staged_kernel<Q, true>), g, b, 0, st, a);
+        else hipLaunchKernelGGL((czt_cols_staged_kernel<Q, false>), g, b, 0, st, a);
+        return;
+      }
     using U = CztCols1<Q>;
     const dim3 g((a.ax.lout + U::G - 1) / U::G, a.ncomp, batch);
     if (a.ay.zl) hipLaunchKernelGGL((czt_cols1_kernel<Q, true>), g, dim3(U::NT), 0, st, a);

@@ -59,6 +59,19 @@ def test_kernel_rows_in_either_place(cuda_dev, n):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n", [1537, 2047])
+def test_longest_length(cuda_dev, n):
+    """The first side past the shorter lengths and the last odd one."""
+    g = gen(n)
+    x = np.linspace(-1.2 * n, 1.2 * n, n)
+    f, c = cplx(g, 1, n, n), cplx(g, 1, n, n)
+    af = ops.rs_propagate(f, x, x, 4e4, 0.65)
+    adjoint_identity(f, af, c, ops.rs_propagate(c, x, x, 4e4, 0.65, adjoint=True))
+    three = ops.rs_propagate(f.expand(3, n, n).contiguous(), x, x, 4e4, 0.65)
+    for i in range(3):
+        near(three[i:i + 1], af, 2e-6)
+
+
 @pytest.mark.parametrize("n", [2, 3, 29, 31, 63, 66, 127, 130, 255])
 def test_rows_of_two_components(cuda_dev, n):
     rng = np.random.default_rng(n)
@@ -85,6 +98,38 @@ def test_rows_of_a_batch(cuda_dev, n, batch):
     out = ops.rs_propagate_batched(src, x, x, 0.65, z, masks=masks(p), **kw)
     for b in (0, batch // 2, batch - 1):
         near(out[b], ops.rs_propagate(src[b], x, x, 0.0, 0.65, masks=masks(p), z_dev=z[b:b + 1], **kw), 2e-6)
+
+
+# columns staged through LDS or not: outputs within, at and above the inputs (full and zero-half lengths 128..1024)
+@pytest.mark.parametrize("n,m", [(50, 30), (64, 66), (100, 28), (120, 130), (130, 120), (61, 400), (200, 300), (300, 200),
+                                 (99, 250), (100, 200), (100, 199), (100, 500), (300, 700), (512, 512)])
+def test_column_forms(cuda_dev, n, m):
+    rng = np.random.default_rng(n + m)
+    x, y = R.space(2.0 * n, n)
+    xo = np.linspace(-0.3 * n, 0.35 * n, m)
+    e = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
+    src = torch.tensor(e.astype(np.complex64), device=cuda_dev)
+    geom = ops.czt_geometry(x, y, xo, xo, 3e4, 0.635)
+    out = ops.czt(src, geom, ez_mode=N.XL_EZ_VCZT, nin=2, form="bluestein")
+    assert rel_l2(out.cpu().numpy(), np.stack(R.vczt(e[0], e[1], x, y, 0.635, 3e4, xo, xo))) < 1e-5
+    cot = cplx(gen(n), 2, m, m)
+    adjoint_identity(src, ops.czt(src, geom, form="bluestein"), cot, ops.czt(cot, geom, adjoint=True, form="bluestein"))
+
+
+# 64 MB of tiles: columns of the batch staged, a member's alone direct; then rows of one component whose plane factors
+# come from a table, most of the row being input or not
+@pytest.mark.parametrize("n,m,batch", [(1024, 1024, 8), (1023, 1009, 9), (700, 300, 4), (640, 300, 4), (641, 300, 4),
+                                       (1500, 500, 4)])
+def test_forms_of_a_batch(cuda_dev, n, m, batch):
+    g = gen(n)
+    x, xo = np.linspace(-900.0, 900.0, n), np.linspace(-400.0, 390.0, m)
+    geom = ops.czt_geometry(x, x, xo, xo, 3e4, 0.635)
+    src, cot, ph = cplx(g, batch, 1, n, n), cplx(g, batch, 1, m, m), uni(g, batch, n, n)
+    out = ops.czt(src, geom, masks=[MaskSpec(N.XL_MASK_SLM, ph)], batch=batch)
+    adj = ops.czt(cot, geom, adjoint=True, batch=batch)
+    for b in (0, batch - 1):
+        near(out[b], ops.czt(src[b], geom, masks=[MaskSpec(N.XL_MASK_SLM, ph[b])], form="bluestein"), 2e-6)
+        near(adj[b], ops.czt(cot[b], geom, adjoint=True, form="bluestein"), 2e-6)
 
 
 # up to 256 rows of 4096 points: three components side by side; more: one after the other
@@ -128,33 +173,31 @@ def test_long_rows_of_a_small_pupil(cuda_dev, n):
     assert rel_l2(out.cpu().numpy(), np.stack(R.vczt(e[0], e[1], x, y, 0.65, 3e4, xo, xo))) < 1e-5
 
 
-# 64 MB of tiles: columns of the batch staged, a member's alone direct; then rows of one component whose plane factors
-# come from a table, most of the row being input or not
-@pytest.mark.parametrize("n,m,batch", [(1024, 1024, 8), (1023, 1009, 9), (700, 300, 4), (640, 300, 4), (641, 300, 4),
-                                       (1500, 500, 4)])
-def test_forms_of_a_batch(cuda_dev, n, m, batch):
+@pytest.mark.parametrize("n", [31, 130, 514])
+def test_distance_term_of_the_joined_adjoint(cuda_dev, n):
+    """The joined adjoint call on a device distance, its distance term started
+    from the column pass's partial sums, against the separate calls started
+    from their sum: float32 products summed in float64, 2^-21 of the terms."""
     g = gen(n)
-    x, xo = np.linspace(-900.0, 900.0, n), np.linspace(-400.0, 390.0, m)
-    geom = ops.czt_geometry(x, x, xo, xo, 3e4, 0.635)
-    src, cot, ph = cplx(g, batch, 1, n, n), cplx(g, batch, 1, m, m), uni(g, batch, n, n)
-    out = ops.czt(src, geom, masks=[MaskSpec(N.XL_MASK_SLM, ph)], batch=batch)
-    adj = ops.czt(cot, geom, adjoint=True, batch=batch)
-    for b in (0, batch - 1):
-        near(out[b], ops.czt(src[b], geom, masks=[MaskSpec(N.XL_MASK_SLM, ph[b])], form="bluestein"), 2e-6)
-        near(adj[b], ops.czt(cot[b], geom, adjoint=True, form="bluestein"), 2e-6)
-
-
-# columns staged through LDS or not: outputs within, at and above the inputs (full and zero-half lengths 128..1024)
-@pytest.mark.parametrize("n,m", [(50, 30), (64, 66), (100, 28), (120, 130), (130, 120), (61, 400), (200, 300), (300, 200),
-                                 (99, 250), (100, 200), (100, 199), (100, 500), (300, 700), (512, 512)])
-def test_column_forms(cuda_dev, n, m):
-    rng = np.random.default_rng(n + m)
-    x, y = R.space(2.0 * n, n)
-    xo = np.linspace(-0.3 * n, 0.35 * n, m)
-    e = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
-    src = torch.tensor(e.astype(np.complex64), device=cuda_dev)
-    geom = ops.czt_geometry(x, y, xo, xo, 3e4, 0.635)
-    out = ops.czt(src, geom, ez_mode=N.XL_EZ_VCZT, nin=2, form="bluestein")
-    assert rel_l2(out.cpu().numpy(), np.stack(R.vczt(e[0], e[1], x, y, 0.635, 3e4, xo, xo))) < 1e-5
-    cot = cplx(gen(n), 2, m, m)
-    adjoint_identity(src, ops.czt(src, geom, form="bluestein"), cot, ops.czt(cot, geom, adjoint=True, form="bluestein"))
+    x, y = np.linspace(-1.2 * n, 1.2 * n, n), np.linspace(-1.1 * n, 1.3 * n, n)
+    z = torch.tensor([2.1e4], dtype=torch.float64, device=cuda_dev)
+    src, gout = cplx(g, 2, n, n), cplx(g, 3, n, n)
+    hh = torch.empty(ops.rs_hhat_bytes(n), dtype=torch.uint8, device=cuda_dev)
+    sp = torch.empty(ops.rs_spec_bytes(n, 3), dtype=torch.uint8, device=cuda_dev)
+    ops.rs_propagate(src, x, y, 0.0, 0.65, ez_mode=N.XL_EZ_VRS, nin=2, z_dev=z, hhat=hh, hhat_mode=1, spec=sp, spec_mode=1,
+                     spec_grads=1)
+    adj = dict(adjoint=True, z_dev=z, hhat=hh, hhat_mode=2, spec=sp, spec_mode=2)
+    dz, dz2 = (torch.full((ops.pre_scalar_grad_elems(n, n),), float("nan"), dtype=torch.float64, device=cuda_dev)
+               for _ in range(2))
+    pre = dict(ez_mode=N.XL_EZ_VRS, nin=2, masks=[], need_src=True, need_params=((False,) * 2,) * 2, out=None)
+    got, _ = ops.rs_propagate(gout, x, y, 0.0, 0.65, spec_grads=1 | N.XL_RS_SPEC_PREBUILT | N.XL_RS_SPEC_PARTIALS,
+                              pre=dict(pre, src=src, ez_dz=dz, ez_dz_base=ops.rs_spec_partials(sp, n, 3, 0)), **adj)
+    sums = torch.empty(2, dtype=torch.float64, device=cuda_dev)
+    g_pre = ops.rs_propagate(gout, x, y, 0.0, 0.65, spec_grads=1 | N.XL_RS_SPEC_PREBUILT, grad_out=sums, **adj)
+    ref, _ = ops.pre_backward(src, g_pre, x, y, 0.0, z_dev=z, ez_dz=dz2, ez_dz_base=sums[:1], **pre)
+    near(got, ref, 1e-6)
+    X, Y = torch.from_numpy(x).cuda()[None, :], torch.from_numpy(y).cuda()[:, None]
+    w = float(z) / torch.sqrt(X * X + Y * Y + z * z) ** 3
+    e = src.to(torch.complex128)
+    terms = g_pre[2].abs().double() * (e[0].abs() * X.abs() + e[1].abs() * Y.abs()) * w
+    assert abs(float(dz[0]) - float(dz2[0])) <= 2.0 ** -21 * float(terms.sum()) + 1e-12 * abs(float(sums[0]))

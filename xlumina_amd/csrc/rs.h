@@ -212,20 +212,24 @@ __host__ __device__ constexpr int rs_hh_stride(int P) { return P / 2 + 16; }
 // 4x4 tile group, lanes spread over the G transforms, so that an access of a
 // wave covers G/4 of each 128 B line it touches instead of a quarter; more
 // than one 35 KB buffer behind common barriers hides less of the transforms'
-// latency, and small grids need all their blocks.  Chosen per kernel (us, one
-// component set of P/2 squared samples, MI355X):
-//                      P = 4096          2048             1024          512
-//                      G = 1     2       1     2     4    1     2       2     4
-//   hrow               26.6  28.2    10.1  10.2  10.2   7.7   7.7     7.2   7.4
-//   hcol               19.2  23.9     7.8   8.0  10.3   4.8   5.3     4.7   5.2
-//   urow (3 comp.)     90.8  97.9    23.7  22.6  25.0  13.6  13.4    10.6  11.6
-//   urow, plain input  78.2  69.5    17.6  17.1  18.8   7.8   6.8     4.4   4.6
-//   col (3 comp.)       133   151    39.2  38.8  51.0  12.6  13.1     6.9   8.2
-//   col (1 comp.)                    15.6  14.8         7.9   7.5
-//   final (3 comp.)    74.5  66.7    17.1  15.0  17.4   6.5   5.8     4.4   4.4
-// The lengths between take the column of the next power of two (VRS 1200^2 at
-// P = 2560, G = 1 / 2 everywhere: 156 / 188 us).  Below P = 1024 a block holds
-// at least one wave.
+// latency, and small grids need all their blocks.  Chosen per kernel (us within
+// repeated calls of P/2 squared samples, MI355X):
+//                      P = 4096          2048                1024
+//                      G = 1     2       1     2     4       1     2     4
+//   hrow               25.3  25.7    13.1  12.9  13.5     8.7   8.8   9.3
+//   hcol               17.3  20.1     7.3   7.6  10.4     5.3   5.8   6.6
+//   urow, SLM          36.8  42.5    17.5  16.4  16.8    10.0  10.1  10.4
+//   urow, LCD and Ez   86.4   105    28.0  25.6  29.2    19.6  20.0  21.8
+//   urow, 3 plain      80.3  66.5    16.4  16.0  18.4    12.2  11.5  12.0
+//   col (1 comp.)      48.5  53.5    15.8  16.3  19.6     9.2   8.9  10.6
+//   col (3 comp.)       142   158    35.1  37.5  53.0    16.6  17.4  19.9
+//   col, dots (3)                    65.8  61.6
+//   final (1 comp.)    19.5  20.4     7.8   7.5   8.0     4.3   4.5   4.8
+//   final (3 comp.)    56.3  53.6    16.2  15.0  16.7     6.6   6.4   6.9
+// The column pass of kept spectra (their layout follows its blocks) has a line
+// of its own.  1280 and 1536 take the 1024 column, 2560 and 3072 that of 4096
+// (VRS 1200^2 at 2560, G = 1 / 2: col 67 / 82, urow 35 / 41, hrow 13.4 / 15.5).
+// Below P = 1024 a block holds at least one wave.
 constexpr int rs_g(int P, int g4096, int g2048, int g1024) {
   return P > 2048 ? g4096 : P == 2048 ? g2048 : P >= 1024 ? g1024 : 1024 / P;
 }
@@ -253,7 +257,7 @@ template <int P, int G_> struct Units {
 template <int P> using UHrow = Units<P, rs_g(P, 1, 1, 1)>;
 template <int P> using UHcol = Units<P, rs_g(P, 1, 1, 1)>;
 template <int P, bool ONE> using UUrow = Units<P, rs_g(P, ONE ? 2 : 1, 2, 2)>;
-template <int P> using UCol = Units<P, rs_g(P, 1, 2, 1)>;
+template <int P, bool KEPT> using UCol = Units<P, rs_g(P, 1, KEPT ? 2 : 1, 1)>;
 template <int P> using UFinal = Units<P, rs_g(P, 2, 2, 2)>;
 
 // Element `off` (a per-lane 32-bit offset) from a block-uniform base: one
@@ -525,7 +529,7 @@ __global__ __launch_bounds__(UHcol<P>::NT, 4) void rs_hcol_kernel(RsArgs a0) {
 // lanes tid % G), fixed order; every thread of the block calls it and thread
 // t = 0 of the column holds the sum.  `red` holds G * (waves per block) values.
 template <int P> __device__ __forceinline__ double column_sum_f64(double v, double* red) {
-  using U = UCol<P>;
+  using U = UCol<P, true>;
   constexpr int NW = U::NT / 64;
 #pragma unroll
   for (int o = 32; o >= U::G; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -555,11 +559,11 @@ template <int P> __device__ __forceinline__ double column_sum_f64(double v, doub
 // of RsArgs): acc[i] = sum over the column's ky of Re(conj(G) dg[i] U), G the
 // spectrum in registers (the cotangent's), U the kept input spectrum.
 template <int P, int SPEC>
-__global__ __launch_bounds__(UCol<P>::NT, 4) void rs_col_kernel(RsArgs a0) {
+__global__ __launch_bounds__((UCol<P, SPEC != 0>::NT), 4) void rs_col_kernel(RsArgs a0) {
   const RsArgs a = rs_member(a0, blockIdx.y);
   if (a.qf_out && blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x == 0)
     a.qf_out[blockIdx.y] = rs_quality_factor(a.z_dev ? *a.z_dev : a.z, a.qf_rmax, a.qf_dr, a.qf_wl);
-  using U = UCol<P>;
+  using U = UCol<P, SPEC != 0>;
   constexpr int TPF = U::TPF, NT = U::NT, HS = rs_hh_stride(P);
   using HO = HandOff<P, TPF>;
   constexpr int SLOTS = HO::BPT * HO::R;
@@ -845,9 +849,10 @@ inline void rs_launch(const RsArgs& a, hipStream_t st) {
   }
   {
     KTimer t(K_RS_COL, st);
-    const dim3 grid = rs_grid<UCol<P>>(P, nb, a.ncomp), blk(UCol<P>::NT);
     bool done = false;
     if constexpr (KEEP) {
+      using UK = UCol<P, true>;
+      const dim3 grid = rs_grid<UK>(P, nb, a.ncomp), blk(UK::NT);
       const int gb = a.spec_mode == 2 ? (a.dg[0] ? 1 : 0) | (a.dg[1] ? 2 : 0) : 0;
       done = a.spec_mode == 1 || gb != 0;
       if (a.spec_mode == 1) hipLaunchKernelGGL((rs_col_kernel<P, 1>), grid, blk, 0, st, a);
@@ -855,7 +860,8 @@ inline void rs_launch(const RsArgs& a, hipStream_t st) {
       else if (gb == 2) hipLaunchKernelGGL((rs_col_kernel<P, 4>), grid, blk, 0, st, a);
       else if (gb == 3) hipLaunchKernelGGL((rs_col_kernel<P, 5>), grid, blk, 0, st, a);
     }
-    if (!done) hipLaunchKernelGGL((rs_col_kernel<P, 0>), grid, blk, 0, st, a);
+    using U0 = UCol<P, false>;
+    if (!done) hipLaunchKernelGGL((rs_col_kernel<P, 0>), rs_grid<U0>(P, nb, a.ncomp), dim3(U0::NT), 0, st, a);
   }
   if (KEEP && a.spec_mode == 2 && !a.partials_only) {
     KTimer t(K_LOSS, st);

@@ -472,10 +472,10 @@ template <int Q> struct CztColsShape {
 };
 
 template <int Q>
-__global__ __launch_bounds__(CztColsShape<Q>::CPB * FftThreads<Q>::value)
+__global__ __launch_bounds__(CztColsShape<Q>::CPB * Q / 16)
 __attribute__((amdgpu_waves_per_eu(CztColsShape<Q>::WAVES))) void czt_cols_kernel(CztArgs a0) {
   const CztArgs a = czt_member(a0, blockIdx.z);
-  constexpr int TPF = FftThreads<Q>::value, LS = LdsLen<Q>::value;
+  constexpr int TPF = Q / 16, LS = LdsLen<Q>::value;
   constexpr int CPB = CztColsShape<Q>::CPB;
   using HO = HandOff<Q, TPF>;
   __shared__ float2 lds[CPB * LS];
@@ -517,9 +517,10 @@ __attribute__((amdgpu_waves_per_eu(CztColsShape<Q>::WAVES))) void czt_cols_kerne
 // G/4 of each tile line it touches and stores G-column row segments, straight
 // from and to its registers.  (Staged through LDS by blocks of half the
 // threads per transform, 232 VGPRs at 4096: the adjoint 256^2 -> 2048^2, three
-// components, 109 us, now 78 us of which the accesses alone take 59; zoom
-// 2048 -> 512 columns 31 -> 23 us.  G = 1, 2, 4 at 4096: 83, 78, 88 us; at
-// 2048, 1024^2 -> 400^2: 13.5, 13.3, 16.8 us.)
+// components, 109 us, now 76 us of which the accesses alone take 59; zoom
+// 2048 -> 512 columns 31 -> 24 us; against the staged form at the other lengths
+// see czt_cols_staged.  G = 1, 2, 4 at 4096: 83, 78, 88 us; at 2048, 1024^2 ->
+// 400^2: 13.5, 13.3, 16.8 us.)
 template <int Q> using CztCols1 = Units<Q, rs_g(Q, 2, 2, 2)>;
 
 template <int Q, bool ZL>
@@ -745,7 +746,7 @@ inline void czt_cols_launch(const CztArgs& a, int batch, hipStream_t st) {
     else hipLaunchKernelGGL((czt_cols1_kernel<Q, false>), g, dim3(U::NT), 0, st, a);
   } else {
     constexpr int CPB = CztColsShape<Q>::CPB;
-    const dim3 g((a.ax.lout + CPB - 1) / CPB, a.ncomp, batch), b(CPB * FftThreads<Q>::value);
+    const dim3 g((a.ax.lout + CPB - 1) / CPB, a.ncomp, batch), b(CPB * Q / 16);
     hipLaunchKernelGGL(czt_cols_kernel<Q>, g, b, 0, st, a);
   }
 }

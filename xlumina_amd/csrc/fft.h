@@ -1,16 +1,18 @@
 // LDS-staged Stockham FFT building blocks for gfx950 (64-wide waves).
 //
-// A workgroup runs FPW independent complex64 FFTs of a power-of-two length L
-// (64 <= L <= 4096), each on TPF = FftThreads<L> threads.  Every pass is radix 16
-// except a final radix 2/4/8 when log2(L) is not a multiple of 4.  Data lives
-// in LDS between passes (natural order in, natural order out); each thread
-// keeps its R points of a butterfly in registers.  LDS indices are padded by
-// one slot per 16 complex values so the stride-16 writes of the first pass
-// spread over the banks.
+// A workgroup runs one or more independent complex64 FFTs of length L = 2^k
+// (64..4096), 3 * 2^k or 5 * 2^k, each on TPF threads, one butterfly per thread
+// and pass: radix 16 at the powers of two with a final radix 2/4/8 when log2(L)
+// is not a multiple of 4, the mixed radices of FftPlan at the others.  Data
+// lives in LDS between passes (natural order in, natural order out); each
+// thread keeps its R points of a butterfly in registers.  LDS indices are
+// padded by one slot per 16 complex values so the stride-16 writes of the
+// first pass spread over the banks.
 //
-// Inter-pass twiddles come from a 4096-entry table e^{-2 pi i k/4096}
+// Inter-pass twiddles come from tables e^{-2 pi i k/N} (N = 4096, 3072, 2560)
 // generated once per device in float64 (xl_fft_init_kernel).  A butterfly
-// loads w and forms the other powers by complex products.
+// loads w (mixed radices: w and w^4) and forms the other powers by complex
+// products.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -105,10 +107,6 @@ __host__ __device__ constexpr int lstep(int k) { return k + (k >> 4); }
 // Whether that holds for the outputs idxD + r NS of a radix-R pass of stride
 // NS (idxD = (j / NS) NS R + j % NS).
 constexpr bool lpad_flat(int NS, int R) { return NS % 16 == 0 || ((NS & (NS - 1)) == 0 && NS * R % 16 == 0); }
-// Threads per FFT: one radix-16 butterfly per thread and pass up to L = 2048;
-// two at L = 4096, so that four 4096-point FFTs per block run on 512 threads
-// with up to 256 VGPRs each instead of spilling at 1024 threads (128 VGPRs).
-template <int L> struct FftThreads { static constexpr int value = L >= 4096 ? L / 32 : L / 16; };
 
 __device__ __forceinline__ float2 operator+(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 operator-(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }

@@ -3,8 +3,8 @@
 // Each pass is the radix-R Stockham step of fft.h, but its source can be LDS,
 // a caller functor (global loads, masks, on-the-fly generation) or registers,
 // and its sink LDS, a caller functor (global stores of only the samples that
-// are needed) or registers.  The forward chain uses radices [3,] 16,...,16,REM
-// and the inverse chain the same in reverse order, so the last forward pass leaves element
+// are needed) or registers.  The inverse chain runs the forward plan's radices
+// in reverse order, so the last forward pass leaves element
 // j + q*(L/R) in register v[b][q] (j = t + b*TPF) and the first inverse pass
 // reads exactly that layout: a frequency-domain product (transfer function,
 // chirp spectrum) is applied in registers between the two chains, with no
@@ -124,8 +124,8 @@ template <int L, int TPF, bool FWD> struct TwSet {
 // threads (so a chain may follow any earlier LDS use); a chain ending in
 // DST_FN / DST_REG leaves LDS free without a final barrier.
 // ZHI / LOW (see pass_io) apply to the first / last pass of the chain; both
-// need a plan that starts (ZHI) or ends (LOW) with an unstrided radix-16 pass
-// over the L/2 split, i.e. a power-of-two L.
+// need a plan that starts (ZHI) or ends (LOW) with an unstrided pass whose even
+// radix splits at L/2 (FftPlan::EVEN: 16, 12 or 10).
 template <int L, int TPF, bool INV, bool FWD, int I, int SRC, int DST, bool ZHI, bool LOW, bool TWPRE, class Load,
           class Store, class RegIn, class RegOut, class Hook>
 __device__ __forceinline__ void chain_pass(float2* s, int t, Load& load, Store& store, RegIn& rin, RegOut& rout,

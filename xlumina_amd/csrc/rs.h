@@ -1,5 +1,6 @@
 // Rayleigh-Sommerfeld convolution (scalar RS / vectorial VRS) on a P x P grid,
-// P >= 2N-1 (the next power of two, or 3 * 2^k / 5 * 2^k below it, rs_fft_len),
+// P >= 2N-1 (the next power of two; a plain call from N = 513 on the shortest of
+// 2^k, 3 * 2^k and 5 * 2^k),
 // with the pre-propagation Jones masks and the Ez construction fused into the
 // first row pass.
 //
@@ -10,7 +11,7 @@
 //     out[q,p] = sum_ij U[j,i] h(x_p - x_i, y_q - y_j) dx dy.
 // Here lag +t sits at index t and lag -t at index P-t (slots N..P-N are zero),
 // which gives the same linear convolution on any P >= 2N-1.  The kernel array
-// is even in both axes, so only rows 0..P/2-1 of its row transform are built
+// is even in both axes, so only rows 0..N-1 of its row transform are built
 // and the column pass mirrors them.
 //
 // Passes (intermediates of N x P samples in 4x4 tiles of 128 B, ordered [column
@@ -670,8 +671,9 @@ __global__ __launch_bounds__((UCol<P, SPEC != 0>::NT), 4) void rs_col_kernel(RsA
 // in registers, where the first N samples are stored and |E|^2 is accumulated
 // over the components.
 // ONE: one component (blockIdx.z) per block (no |E|^2 to accumulate across
-// components): ncomp N rows divide into the resident slots evenly where N row
-// blocks (2.67 rounds at P = 4096) leave a partly idle last round.
+// components): ncomp N / G blocks instead of N / G, and the last round of them
+// over the chip is fuller (at P = 4096 1024 blocks of two rows make 1.33
+// rounds, 3072 make 4).
 // Below P = 1024 the passes run in the forward order and form every output
 // (roundings are those of the whole transform).
 template <int P, bool ONE = false>

@@ -193,7 +193,7 @@ int plan_axis(int m, int M, double f1, double f2, double Dm, bool allow3, AxisPl
   // covering mp; any length >= mp gives the same linear convolution
   int q = std::max(64, next_pow2(mp));
   // a power of two that holds both m and M in its halves runs the zero-half
-  // passes and the staged column I/O, and then beats the shorter 3 * 2^k
+  // passes, and then beats the shorter 3 * 2^k
   const bool half = 2 * std::max(m, M) <= q;
   for (int q3 = 768; allow3 && !half && q3 <= 3072; q3 *= 2)
     if (q3 >= mp && q3 < q) {

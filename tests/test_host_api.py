@@ -172,13 +172,15 @@ def test_distances_mapped_together_match_one_by_one():
 
 @pytest.mark.parametrize("kind", ["numpy", "list", "tensor"])
 def test_sample_spacing_needs_a_1d_grid(kind):
-    """A grid laid out as a row has no spacing along its first axis (and its
-    propagation is refused); its samples alone are still found."""
+    """A grid laid out as a row has no spacing along its first axis and is
+    refused as a propagation's grid; its samples alone are still found."""
     make = {"numpy": lambda a: a, "list": lambda a: a.tolist(), "tensor": torch.from_numpy}[kind]
     x = np.linspace(-4.0, 4.0, 9)
     info = ops.grid_info(make(x), torch.device("cpu"))
     assert (info.n, info.step) == (9, 1.0)
-    row = ops.grid_info(make(x[None, :]), torch.device("cpu"))
-    assert row.n == 9
+    cpu = torch.device("cpu")
+    ops.check_rs_args((1, 9, 9), 1, 1, info.n, info.n, None, None, cpu)
+    row = ops.grid_info(make(x[None, :]), cpu)
+    assert row.t.shape[-1] == 9
     with pytest.raises(ValueError):
-        row.step
+        ops.check_rs_args((1, 9, 9), 1, 1, row.n, info.n, None, None, cpu)

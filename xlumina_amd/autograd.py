@@ -108,12 +108,12 @@ def _spectra_key(cfg: RSConfig, z_t, n: int, ncomp: int, dev):
     version; the key is None where a version is not tracked (inference tensors)."""
     xd, yd = ops.device_grid(cfg.x, dev), ops.device_grid(cfg.y, dev)
     keep = (None if z_t is None else z_t.detach(), xd, yd)
-    held = [t for t in (z_t, cfg.x if cfg.x is xd else None, cfg.y if cfg.y is yd else None) if t is not None]
-    if any(t.is_inference() for t in held):
+    try:
+        zk = ("f", float(cfg.z)) if z_t is None else ("t", z_t.data_ptr(), z_t._version, z_t.device)
+        xv, yv = xd._version if xd is cfg.x else -1, yd._version if yd is cfg.y else -1
+    except RuntimeError:   # an inference tensor has no version
         return None, keep
-    zk = ("t", z_t.data_ptr(), z_t.device) if z_t is not None else ("f", float(cfg.z))
-    key = (zk, xd.data_ptr(), yd.data_ptr(), *(t._version for t in held), n, ncomp, float(cfg.wavelength), dev,
-           ops.launch_scope(dev))
+    key = (zk, xd.data_ptr(), xv, yd.data_ptr(), yv, n, ncomp, float(cfg.wavelength), dev, ops.launch_scope(dev))
     return key, keep
 
 

@@ -89,21 +89,16 @@ _grid_ids: dict = {}   # (id(array), device) -> (weak reference, its bytes, Grid
 
 class GridInfo:
     """What a call needs of a 1-D grid: its float64 device copy, its length and
-    its first step."""
-    __slots__ = ("t", "n", "_step")
+    its first step.  A grid of another shape, which has no step along its first
+    axis, has length -1: a propagation's length check refuses it."""
+    __slots__ = ("t", "n", "step")
 
     def __init__(self, t: torch.Tensor, host):
         host = np.asarray(host, dtype=np.float64)
         self.t = t
-        self.n = int(host.size)
         d = host[1] - host[0] if host.ndim and len(host) > 1 else None
-        self._step = float(d.item()) if d is not None and d.size == 1 else None
-
-    @property
-    def step(self) -> float:
-        if self._step is None:
-            raise ValueError("the sample spacing needs a 1-D grid of two or more samples")
-        return self._step
+        ok = d is not None and d.size == 1
+        self.n, self.step = (int(host.size), float(d.item())) if ok else (-1, 0.0)
 
 
 def grid_info(arr, device) -> GridInfo:

@@ -664,14 +664,17 @@ def _czt_params(g: CztGeometry, dev, ncomp, nin, adjoint, ez_mode, mode=None):
 CZT_FORMS = ("auto", "bluestein", "gemm")
 _czt_form = "auto"
 # Where "auto" picks the split-BF16 MFMA zoom-DFT over the FP32 Bluestein FFT
-# form.  RS-mode transforms of several components, measured on MI355X (us,
-# forward + adjoint of three components, Bluestein / GEMM): 2048^2 -> 96^2 240 /
-# 214, 128^2 241 / 231, 160^2 243 / 270; 1500^2 -> 64^2 142 / 150, 128^2 143 /
-# 180; 1024^2 -> 96^2 94 / 116; 256^2 -> 96^2 52 / 85.  One component: 2048^2 ->
-# 96^2 forward 56 / 86.  So the GEMM form is left where an input side exceeds
-# GEMM_MIN_SIDE and the window fits GEMM_RS_WINDOW.  High-NA transforms keep
-# their own line, GEMM_CROSSOVER: the gradients of float64 masks behind them
-# stay what they were to the last bit (1024^2 -> 96^2 88 / 109 us).
+# form: RS-mode transforms of several components where an input side exceeds
+# GEMM_MIN_SIDE and the window fits GEMM_RS_WINDOW, high-NA transforms to
+# windows of GEMM_CROSSOVER.  Measured on MI355X (us, forward + adjoint of three
+# components, Bluestein / GEMM), RS mode: 2048^2 -> 48^2 207 / 186, 64^2 203 /
+# 189, 96^2 206 / 203, 128^2 206 / 218, 160^2 212 / 251; 1792^2 -> 96^2 144 / 190;
+# 1600^2 -> 64^2 132 / 146; 1500^2 -> 64^2 123 / 141; 1024^2 -> 96^2 83 / 109; 256^2
+# -> 96^2 48 / 86; one component, 2048^2 -> 96^2 forward 51 / 79.  High-NA: 2048^2
+# -> 64^2 190 / 167, 96^2 192 / 181, 128^2 194 / 197, 160^2 197 / 229; 1500^2 ->
+# 64^2 114 / 126; 1024^2 -> 96^2 81 / 102.  The lines were drawn when the Bluestein
+# passes were slower (2048^2 -> 128^2 241 us): today it would win all but windows
+# below about 100 samples of 2048^2.
 GEMM_CROSSOVER = 160
 GEMM_RS_WINDOW = 128
 GEMM_MIN_SIDE = 1536
